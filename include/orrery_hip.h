@@ -193,10 +193,10 @@ ORR_API int orr_tree_eval(orr_ctx* ctx, const orr_tree_args* args, orr_tree_stat
 
 /* Walk configuration (no reference counterpart; cuda_tree_solver.cpp fixes its
  * traversal): targets_per_lane 1 or 2 -- how many targets each lane of a
- * wave walks together -- or -1 to choose by size (2 for one system of 2^20 or
- * more particles, else 1; the default); lanes 64 or 32 -- how many lanes of a
- * wave hold targets -- or -1 to choose by size (32 for a launch of at most
- * 2048 full waves, two per SIMD, else 64; the default). Results are
+ * wave walks together -- or -1 for the engine's choice (1; the default); lanes
+ * 64 or 32 -- how many lanes of a wave hold targets -- or -1 to choose by size
+ * (16 for a launch of at most 256 full waves, 32 up to 2048, two per SIMD, else
+ * 64; the default). Results are
  * bit-identical either way; only the speed differs. sort_mode chooses the
  * Morton sort of every path (the tree's, the batch's, the direct ordering of
  * more than 4096 particles): 1 (the default) one launch per radix pass after

@@ -136,7 +136,7 @@ struct orr_ctx {
     int sort_mode = 1;  // Morton sort: 1 one-sweep passes, 2 histogram + scan + scatter per pass
     // Barnes-Hut walk configuration (orr_ctx_set_tree_config); 0 chooses by size.
     int walk_targets_per_lane = 0;
-    int walk_lanes = 0;  // active lanes per walk wave: 32, 64, or 0 = by size
+    int walk_lanes = 0;  // active lanes per walk wave: 32, 64, or 0 = by size (16, 32 or 64)
 
     // Host mirror of the last tree summary and the shape of its device layout.
     orr_tree_stats last_tree{};

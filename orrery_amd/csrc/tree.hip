@@ -60,6 +60,8 @@ constexpr std::uint32_t kNoChild = 0xffffffffu;
 // Spare float4 entries past the last particle of leaf_rel: a leaf's sources are
 // read in rounds of four.
 constexpr std::size_t kLeafPad = 3;
+// The fewest targets a walk wave holds.
+constexpr std::uint64_t kMinLanes = 16;
 
 struct WalkNode {
     float4 a;  // centre of mass relative to the root centre (FP32), mass
@@ -515,40 +517,22 @@ __global__ __launch_bounds__(kBlock) void internal_moments(
     }
 }
 
-// Minimum over the 64 lanes of a wave (all lanes active). Within each row of
-// 16 lanes, four DPP row shifts make lane 15 of the row hold the row minimum
-// (shifted-in lanes outside the row read the identity ~0); the four row minima
-// are then combined in scalar registers.
-template<int kCtrl> __device__ __forceinline__ std::uint32_t dpp_min(std::uint32_t v) {
-    const std::uint32_t moved = static_cast<std::uint32_t>(
-        __builtin_amdgcn_update_dpp(-1, static_cast<int>(v), kCtrl, 0xf, 0xf, false));
-    return min(v, moved);
-}
-
-__device__ inline std::uint32_t wave_min_u32(std::uint32_t v) {
-    v = dpp_min<0x111>(v);  // row_shr:1
-    v = dpp_min<0x112>(v);  // row_shr:2
-    v = dpp_min<0x114>(v);  // row_shr:4
-    v = dpp_min<0x118>(v);  // row_shr:8
-    const std::uint32_t r0 = __builtin_amdgcn_readlane(static_cast<int>(v), 15);
-    const std::uint32_t r1 = __builtin_amdgcn_readlane(static_cast<int>(v), 31);
-    const std::uint32_t r2 = __builtin_amdgcn_readlane(static_cast<int>(v), 47);
-    const std::uint32_t r3 = __builtin_amdgcn_readlane(static_cast<int>(v), 63);
-    return min(min(r0, r1), min(r2, r3));
-}
-
-__device__ inline unsigned long long wave_sum_u64(unsigned long long v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
 __device__ __forceinline__ void kahan(float p, float& s, float& c) {
     const float y = p - c;
     const float t = s + y;
     c = (t - s) - y;
     s = t;
 }
+
+// Up to this many full (64-lane) walk waves -- two per SIMD of the 256 CUs --
+// half-lane waves are faster (quadrupole walk, two-disc collision: 1.088 ->
+// 0.981 ms at N = 65,536, 1.328 -> 1.265 ms at 131,072); above it they are
+// slower (1.35 -> 1.83 ms at 262,144): the walk is bound by issue, not by
+// latency, once each SIMD has a few waves. Up to a quarter of a wave per SIMD,
+// waves of 16 targets (monopole walk of a 16,384-particle Plummer sphere: 64
+// targets a wave 0.566, 32 0.521, 16 0.470 ms).
+constexpr std::uint64_t kHalfLaneWaves = 2 * 4 * 256;
+constexpr std::uint64_t kQuarterLaneWaves = 256;
 
 // Workgroups are dispatched to the 8 XCDs in turn (block b to XCD b mod 8),
 // and each XCD has its own L2. Neighbouring targets in Morton order visit the
@@ -559,13 +543,6 @@ __device__ __forceinline__ void kahan(float p, float& s, float& c) {
 // system (one contiguous eighth each would leave the XCD with the densest part
 // finishing last). A bijection of [0, blocks): blocks past the last whole
 // round of runs keep their own index.
-// Up to this many full (64-lane) walk waves -- two per SIMD of the 256 CUs --
-// half-lane waves are faster (quadrupole walk, two-disc collision: 1.088 ->
-// 0.981 ms at N = 65,536, 1.328 -> 1.265 ms at 131,072); above it they are
-// slower (1.813 -> 2.194 ms at 262,144): the walk is bound by issue, not by
-// latency, once each SIMD has a few waves.
-constexpr std::uint64_t kHalfLaneWaves = 2 * 4 * 256;
-
 constexpr std::uint32_t kXcds = 8;
 constexpr std::uint32_t kXcdRun = 16;
 __device__ __forceinline__ std::uint32_t xcd_block(std::uint32_t b, std::uint32_t blocks) {
@@ -576,64 +553,70 @@ __device__ __forceinline__ std::uint32_t xcd_block(std::uint32_t b, std::uint32_
 }
 
 // One target's walk state: FP32 position relative to the root centre and
-// offset from its leaf centre, its leaf, the next node it needs, Kahan sums.
+// offset from its leaf centre, its leaf, Kahan sums and the running partial.
 struct WalkTarget {
     float4 xi, oi;
-    std::uint32_t own, mine;
+    std::uint32_t own;
     float sx, sy, sz, kx, ky, kz, px, py, pz;
-    // Per target, pp < N, pc <= M and visits <= M: 32 bits suffice.
-    std::uint32_t pp, pc, visits;
+    std::uint32_t pc;  // accepted nodes, at most M
 };
 
-// The target's step at node `cur` if it is the node it needs (tree_walk.cpp:20-83):
-// accept (monopole, optionally quadrupole, then skip the subtree), mark a leaf
-// for particle-particle terms (returns true), or open (descend to cur + 1).
+// Separation of the target from a node's centre of mass, and its square.
+__device__ __forceinline__ float separation(const WalkTarget& t, const float4& com, float& dx,
+                                            float& dy, float& dz) {
+    dx = com.x - t.xi.x;
+    dy = com.y - t.xi.y;
+    dz = com.z - t.xi.z;
+    return __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
+}
+
+// An accepted node's term (tree_walk.cpp:20-83): monopole, optionally quadrupole.
 template<bool kSafe, bool kQuad>
-__device__ __forceinline__ bool visit(WalkTarget& t, std::uint32_t cur, const WalkNode& nd,
-                                      const QuadF& Q, std::uint32_t next, float eps2) {
-    if (t.mine != cur) return false;
-    ++t.visits;
-    const float dx = nd.a.x - t.xi.x, dy = nd.a.y - t.xi.y, dz = nd.a.z - t.xi.z;
-    const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-    float acc;
-    std::memcpy(&acc, &nd.b.x, sizeof(acc));
-    if (r2 >= acc) {
-        // tree_walk.hpp:129-139 monopole.
-        float r2e = r2 + eps2;
-        if constexpr (kSafe) r2e = r2e > 0.f ? r2e : 1.f;
-        const float inv = __builtin_amdgcn_rsqf(r2e);
-        if constexpr (!kQuad) {
-            const float f = (nd.a.w * inv) * (inv * inv);
-            t.px = __builtin_fmaf(f, dx, t.px);
-            t.py = __builtin_fmaf(f, dy, t.py);
-            t.pz = __builtin_fmaf(f, dz, t.pz);
-        } else {
-            // Monopole plus tree_walk.hpp:156-181 in one update:
-            // d (m inv^3 + 2.5 (d.Q d) inv^7) - (Q d) inv^5.
-            const float i2 = inv * inv;
-            const float i3 = i2 * inv;
-            const float i5 = i3 * i2;
-            const float i7 = i5 * i2;
-            const float qx = __builtin_fmaf(Q.a.z, dz, __builtin_fmaf(Q.a.y, dy, Q.a.x * dx));
-            const float qy = __builtin_fmaf(Q.b.x, dz, __builtin_fmaf(Q.a.w, dy, Q.a.y * dx));
-            const float qz = __builtin_fmaf(Q.b.y, dz, __builtin_fmaf(Q.b.x, dy, Q.a.z * dx));
-            const float quadratic = __builtin_fmaf(dz, qz, __builtin_fmaf(dy, qy, dx * qx));
-            const float g = __builtin_fmaf(2.5f * quadratic, i7, nd.a.w * i3);
-            t.px = __builtin_fmaf(dx, g, __builtin_fmaf(qx, -i5, t.px));
-            t.py = __builtin_fmaf(dy, g, __builtin_fmaf(qy, -i5, t.py));
-            t.pz = __builtin_fmaf(dz, g, __builtin_fmaf(qz, -i5, t.pz));
-        }
-        ++t.pc;
-        t.mine = next;
-        return false;
+__device__ __forceinline__ void accept(WalkTarget& t, float mass, const float4& Qa, const float4& Qb,
+                                       float dx, float dy, float dz, float r2, float eps2) {
+    // tree_walk.hpp:129-139 monopole.
+    float r2e = r2 + eps2;
+    if constexpr (kSafe) r2e = r2e > 0.f ? r2e : 1.f;
+    const float inv = __builtin_amdgcn_rsqf(r2e);
+    if constexpr (!kQuad) {
+        const float f = (mass * inv) * (inv * inv);
+        t.px = __builtin_fmaf(f, dx, t.px);
+        t.py = __builtin_fmaf(f, dy, t.py);
+        t.pz = __builtin_fmaf(f, dz, t.pz);
+    } else {
+        // Monopole plus tree_walk.hpp:156-181 in one update:
+        // d (m inv^3 + 2.5 (d.Q d) inv^7) - (Q d) inv^5.
+        const float i2 = inv * inv;
+        const float i3 = i2 * inv;
+        const float i5 = i3 * i2;
+        const float i7 = i5 * i2;
+        const float qx = __builtin_fmaf(Qa.z, dz, __builtin_fmaf(Qa.y, dy, Qa.x * dx));
+        const float qy = __builtin_fmaf(Qb.x, dz, __builtin_fmaf(Qa.w, dy, Qa.y * dx));
+        const float qz = __builtin_fmaf(Qb.y, dz, __builtin_fmaf(Qb.x, dy, Qa.z * dx));
+        const float quadratic = __builtin_fmaf(dz, qz, __builtin_fmaf(dy, qy, dx * qx));
+        const float g = __builtin_fmaf(2.5f * quadratic, i7, mass * i3);
+        t.px = __builtin_fmaf(dx, g, __builtin_fmaf(qx, -i5, t.px));
+        t.py = __builtin_fmaf(dy, g, __builtin_fmaf(qy, -i5, t.py));
+        t.pz = __builtin_fmaf(dz, g, __builtin_fmaf(qz, -i5, t.pz));
     }
-    if (nd.b.w > 0) {
-        t.pp += nd.b.w - (t.own == cur ? 1u : 0u);
-        t.mine = next;
-        return true;
-    }
-    t.mine = cur + 1;
-    return false;
+}
+
+// Four consecutive leaf particles in scalar registers.
+struct LeafRound {
+    float4 q[4];
+};
+__device__ __forceinline__ LeafRound load_round(const float4* __restrict__ leaf_rel, std::uint32_t j) {
+    // Four sources from one base, so that their scalar loads are one load. A
+    // last round of fewer than four still loads four (leaf_rel holds kLeafPad
+    // spare entries past the last particle).
+    const float4* const q = leaf_rel + j;
+    LeafRound v{{q[0], q[1], q[2], q[3]}};
+    return v;
+}
+__device__ __forceinline__ void pin(const LeafRound& v) {
+    asm volatile("" ::"s"(v.q[0].x), "s"(v.q[0].y), "s"(v.q[0].z), "s"(v.q[0].w), "s"(v.q[1].x), "s"(v.q[1].y),
+                 "s"(v.q[1].z), "s"(v.q[1].w), "s"(v.q[2].x), "s"(v.q[2].y), "s"(v.q[2].z), "s"(v.q[2].w),
+                 "s"(v.q[3].x), "s"(v.q[3].y), "s"(v.q[3].z), "s"(v.q[3].w));
 }
 
 // Particle-particle terms of leaf [b, e) for one target, then the partial is
@@ -646,7 +629,7 @@ __device__ __forceinline__ void leaf_pairs(WalkTarget& t, const double4& cb, dou
     const float tx = t.oi.x - static_cast<float>(cb.x - cax);
     const float ty = t.oi.y - static_cast<float>(cb.y - cay);
     const float tz = t.oi.z - static_cast<float>(cb.z - caz);
-    auto pair = [&](const float4 q) {
+    auto pair = [&](const float4& q) {
         const float dx = q.x - tx, dy = q.y - ty, dz = q.z - tz;
         float r2 = __builtin_fmaf(dx, dx, eps2);
         r2 = __builtin_fmaf(dy, dy, r2);
@@ -658,20 +641,23 @@ __device__ __forceinline__ void leaf_pairs(WalkTarget& t, const double4& cb, dou
         t.py = __builtin_fmaf(f, dy, t.py);
         t.pz = __builtin_fmaf(f, dz, t.pz);
     };
-    // Four sources per round, addressed from one base so that their scalar
-    // loads are issued together and share one wait. A last round of fewer than
-    // four still loads four (leaf_rel holds kLeafPad spare entries past the
-    // last particle) and uses those in the leaf: most leaves hold under four.
-    for (std::uint32_t j = b; j < e; j += 4) {
-        const float4* q = leaf_rel + j;
-        const float4 q0 = q[0], q1 = q[1], q2 = q[2], q3 = q[3];
-        asm volatile("" ::"s"(q0.x), "s"(q0.y), "s"(q0.z), "s"(q0.w), "s"(q1.x), "s"(q1.y),
-                     "s"(q1.z), "s"(q1.w), "s"(q2.x), "s"(q2.y), "s"(q2.z), "s"(q2.w),
-                     "s"(q3.x), "s"(q3.y), "s"(q3.z), "s"(q3.w));
-        pair(q0);
-        if (j + 1 < e) pair(q1);
-        if (j + 2 < e) pair(q2);
-        if (j + 3 < e) pair(q3);
+    // Whole rounds without a branch between the four terms, whose chains then
+    // overlap; the sums still take them in index order.
+    std::uint32_t j = b;
+    for (; j + 4 <= e; j += 4) {
+        const LeafRound v = load_round(leaf_rel, j);
+        pin(v);
+        pair(v.q[0]);
+        pair(v.q[1]);
+        pair(v.q[2]);
+        pair(v.q[3]);
+    }
+    if (j < e) {
+        const LeafRound v = load_round(leaf_rel, j);
+        pin(v);
+        pair(v.q[0]);
+        if (j + 1 < e) pair(v.q[1]);
+        if (j + 2 < e) pair(v.q[2]);
     }
     kahan(t.px, t.sx, t.kx);
     kahan(t.py, t.sy, t.ky);
@@ -679,14 +665,56 @@ __device__ __forceinline__ void leaf_pairs(WalkTarget& t, const double4& cb, dou
     t.px = t.py = t.pz = 0.f;
 }
 
+// A wave's stack of pending sibling lists, level d in lane d of a few vector
+// registers. Writing is one v_writelane a word (no lane-compare, whatever the
+// execution mask); the lane select goes through m0, since the instruction can
+// read only one scalar register.
+__device__ __forceinline__ void lane_write(std::uint32_t& reg, std::uint32_t value, std::uint32_t lane) {
+    asm("s_mov_b32 m0, %2\n\ts_nop 0\n\tv_writelane_b32 %0, %1, m0" : "+v"(reg) : "s"(value), "s"(lane) : "m0");
+}
+__device__ __forceinline__ std::uint32_t lane_read(std::uint32_t reg, std::uint32_t lane) {
+    return static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(reg), static_cast<int>(lane)));
+}
+
+// The wave's accepted nodes (idle lanes count none).
+template<int kR> __device__ unsigned long long accepted(const WalkTarget (&t)[kR]) {
+    unsigned long long v = 0;
+#pragma unroll
+    for (int r = 0; r < kR; ++r) v += t[r].pc;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// One system's counts from a wave that walked several.
+__device__ void add_counts(unsigned long long* __restrict__ stats, std::uint32_t seg,
+                           unsigned long long pp, unsigned long long pc, unsigned long long visits,
+                           unsigned long long slots) {
+    unsigned long long* st = stats + 4 * static_cast<std::size_t>(seg);
+    atomicAdd(&st[0], pp);
+    atomicAdd(&st[1], pc);
+    atomicAdd(&st[2], visits);
+    atomicAdd(&st[3], slots);
+}
+
 // Wave-coherent walk. Each of the first kLanes lanes owns kR targets (wave w
 // owns the kLanes kR sorted particles from kLanes kR w, target r of lane l
 // being kLanes r + l; with kLanes = 32 the other half of the wave holds none,
-// which doubles the waves a small system gets); the wave visits
-// the smallest node any of its targets needs, loads it once, and every target
-// that needs it takes its step. A target therefore sees exactly the node
-// sequence and arithmetic of a walk of its own, whatever the other targets are.
-template<int kR, bool kSafe, bool kQuad, int kLanes>
+// which doubles the waves a small system gets). The wave goes through the nodes
+// that any of its targets visits, in depth-first order, each loaded once; every
+// target takes part in exactly the nodes of a walk of its own.
+//
+// The targets that reach a node are one lane mask per set r in scalar
+// registers, not a next-node index per lane: all targets that opened a cell
+// reach each of its children, and all that reached the cell go on after it. So
+// opening a cell pushes the mask of its sibling list with the escape index that
+// ends it, and reaching that index pops it. Which lanes accept is one compare
+// and scalar logic, the counts are scalar population counts, and the next node
+// needs no reduction over the lanes.
+//
+// kMany: the targets may belong to several systems (a batch); the systems of
+// a wave's targets are then walked one after another.
+template<int kR, bool kSafe, bool kQuad, int kLanes, bool kMany>
 __global__ __launch_bounds__(kBlock) void tree_walk(
     const WalkNode* __restrict__ nodes, const QuadF* __restrict__ quads,
     const double4* __restrict__ node_geo,
@@ -697,13 +725,12 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
     std::uint32_t n, float eps2, double G,
     double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
     unsigned long long* __restrict__ stats, unsigned long long* __restrict__ wave_stats) {
-    constexpr std::uint32_t kDone = 0xffffffffu;
     const std::uint32_t wave = xcd_block(blockIdx.x, gridDim.x) * (kBlock / 64) + threadIdx.x / 64;
     const std::uint32_t lane = threadIdx.x & 63;
     const std::uint32_t M = counters[0];
     WalkTarget t[kR];
     std::uint32_t seg[kR];
-    bool valid[kR];
+    std::uint64_t todo[kR];  // targets whose system the wave has not walked yet
     // Each lane's targets' own leaf centres, read at every leaf visit: held in
     // LDS rather than registers (12 KB a block at two targets a lane) or
     // re-read from memory at each visit. A lane reads only its own slots.
@@ -711,8 +738,8 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
 #pragma unroll
     for (int r = 0; r < kR; ++r) {
         const std::uint32_t i = wave * (kLanes * kR) + kLanes * r + lane;
-        valid[r] = lane < kLanes && i < n;
-        const std::uint32_t ic = valid[r] ? i : n - 1;
+        const bool valid = lane < kLanes && i < n;
+        const std::uint32_t ic = valid ? i : n - 1;
         t[r].xi = root_rel[ic];
         t[r].oi = leaf_rel[ic];
         t[r].own = leaf_of[ic];
@@ -720,129 +747,173 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
         s_own[r][0][threadIdx.x] = ca.x;
         s_own[r][1][threadIdx.x] = ca.y;
         s_own[r][2][threadIdx.x] = ca.z;
-        // The target's system starts at its root; the walk records' escape
-        // indices end the walk at the system's last subtree.
-        seg[r] = seg_of != nullptr ? seg_of[ic] : 0u;
-        const std::uint32_t root = seg_start != nullptr ? first_node[seg_start[seg[r]]] : 0u;
-        t[r].mine = valid[r] ? root : kDone;
+        seg[r] = kMany ? seg_of[ic] : 0u;
+        todo[r] = __ballot(valid);
         t[r].sx = t[r].sy = t[r].sz = t[r].kx = t[r].ky = t[r].kz = 0.f;
         t[r].px = t[r].py = t[r].pz = 0.f;
-        t[r].pp = t[r].pc = t[r].visits = 0;
+        t[r].pc = 0;
     }
+    // An FP32 instruction with a scalar operand issues at half the rate of one
+    // that reads only vector registers: eps^2 enters every term.
+    asm volatile("" : "+v"(eps2));
     std::uint32_t steps = 0;
-    // Each iteration advances at least one target, so a walk takes at most
-    // 64 kR M iterations; the cap only turns a corrupted tree into a wrong result.
-    // 32-bit counts (a 32-bit compare in the loop condition), the cap clamped.
-    const std::uint32_t cap = static_cast<std::uint32_t>(min(64ull * kR * M + 64, 0xffffffffull));
-    std::uint32_t least = t[0].mine;
+    std::uint32_t systems = 0;   // systems walked by this wave
+    std::uint32_t seg0 = 0;      // the first of them
+    // Particle-particle terms, and the visits that accepted nothing (leaves
+    // and opened cells); accepted nodes are counted per target.
+    unsigned long long pp = 0, stopped = 0;
+    while (true) {
+        std::uint32_t own_seg = 0;
+        std::uint64_t mask[kR];
+        bool left = false;
 #pragma unroll
-    for (int r = 1; r < kR; ++r) least = min(least, t[r].mine);
-    std::uint32_t cur = __builtin_amdgcn_readfirstlane(wave_min_u32(least));
-    while (cur != kDone && steps < cap) {
-        ++steps;
-        const WalkNode nd = nodes[cur];
-        QuadF Q{};
-        if constexpr (kQuad) Q = quads[cur];
-        // Every scalar load of the iteration is issued here and waited for once;
-        // left to itself the compiler sinks them into the branches below, one
-        // dependent wait each.
-        asm volatile("" ::"s"(nd.a.x), "s"(nd.a.y), "s"(nd.a.z), "s"(nd.a.w), "s"(nd.b.x),
-                     "s"(nd.b.y), "s"(nd.b.z), "s"(nd.b.w));
-        if constexpr (kQuad) {
-            asm volatile("" ::"s"(Q.a.x), "s"(Q.a.y), "s"(Q.a.z), "s"(Q.a.w), "s"(Q.b.x),
-                         "s"(Q.b.y));
-        }
-        // An escape index always lies past its node (or is kDone); the guard only
-        // makes a corrupted tree end the walk instead of looping.
-        const std::uint32_t next = nd.b.y > cur ? nd.b.y : kDone;
-        bool leaf[kR];
-        bool any_leaf = false;
-#pragma unroll
-        for (int r = 0; r < kR; ++r) {
-            leaf[r] = visit<kSafe, kQuad>(t[r], cur, nd, Q, next, eps2);
-            any_leaf = any_leaf || leaf[r];
-        }
-        if (__ballot(any_leaf) != 0) {
-            const double4 cb = node_geo[cur];
-            const std::uint32_t b = nd.b.z, e = nd.b.z + nd.b.w;
-#pragma unroll
-            for (int r = 0; r < kR; ++r) {
-                if (leaf[r]) {
-                    leaf_pairs<kSafe>(t[r], cb, s_own[r][0][threadIdx.x], s_own[r][1][threadIdx.x],
-                                      s_own[r][2][threadIdx.x], leaf_rel, b, e, eps2);
+        for (int r = kR - 1; r >= 0; --r) {
+            if (todo[r] != 0) {
+                left = true;
+                if constexpr (kMany) {
+                    own_seg = lane_read(seg[r], static_cast<std::uint32_t>(__builtin_ctzll(todo[r])));
                 }
             }
         }
-        // The wave's next node: cur + 1 when any target descends; else, most
-        // often, this node's escape `next` (some target is there and none
-        // before it), without the wave-wide minimum; else that minimum.
-        const std::uint32_t step = cur + 1;
-        bool descends = false, at_next = false, before_next = false;
-        least = t[0].mine;
+        if (!left) break;
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            descends = descends || t[r].mine == step;
-            at_next = at_next || t[r].mine == next;
-            before_next = before_next || t[r].mine < next;
-            least = min(least, t[r].mine);
+            mask[r] = kMany ? __ballot(seg[r] == own_seg) & todo[r] : todo[r];
+            todo[r] &= ~mask[r];
         }
-        if (__ballot(descends) != 0) {
-            cur = step;
-        } else if (__ballot(before_next) == 0 && __ballot(at_next) != 0) {
-            cur = next;
-        } else {
-            cur = __builtin_amdgcn_readfirstlane(wave_min_u32(least));
+        if (kMany && systems > 0) {
+            // A second system: the counts so far belong to the one before it.
+            const unsigned long long pc = accepted(t);
+            if (lane == 0) {
+                add_counts(stats, seg0, pp, pc, pc + stopped,
+                           static_cast<unsigned long long>(steps) * (kR * kLanes) / 64);
+            }
+#pragma unroll
+            for (int r = 0; r < kR; ++r) t[r].pc = 0;
+            pp = stopped = 0;
+            steps = 0;
+        }
+        seg0 = own_seg;
+        ++systems;
+        // The stack: the escape index that ends a sibling list and its masks.
+        std::uint32_t st_end = 0, st_lo[kR], st_hi[kR];
+#pragma unroll
+        for (int r = 0; r < kR; ++r) st_lo[r] = st_hi[r] = 0;
+        std::uint32_t depth = 0, end = 0;  // the outermost list ends nowhere
+        std::uint32_t cur = kMany ? __builtin_amdgcn_readfirstlane(first_node[seg_start[own_seg]]) : 0u;
+        // cur only ever grows, so the loop ends whatever the records hold.
+        while (cur < M) {
+            ++steps;
+            const float4 na = nodes[cur].a;
+            const uint4 nb = nodes[cur].b;
+            float4 qa{}, qb{};
+            if constexpr (kQuad) {
+                qa = quads[cur].a;
+                qb = quads[cur].b;
+            }
+            // Every scalar load of the iteration is issued here and waited for once;
+            // left to itself the compiler sinks them into the branches below, one
+            // dependent wait each.
+            asm volatile("" ::"s"(na.x), "s"(na.y), "s"(na.z), "s"(na.w), "s"(nb.x), "s"(nb.y), "s"(nb.z),
+                         "s"(nb.w));
+            if constexpr (kQuad) {
+                asm volatile("" ::"s"(qa.x), "s"(qa.y), "s"(qa.z), "s"(qa.w), "s"(qb.x), "s"(qb.y),
+                             "s"(qb.z), "s"(qb.w));
+            }
+            const float acc = __builtin_bit_cast(float, nb.x);
+            std::uint64_t rest[kR], any = 0;
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                rest[r] = 0;
+                if (kR > 1 && mask[r] == 0) continue;
+                float dx, dy, dz;
+                const float r2 = separation(t[r], na, dx, dy, dz);
+                const std::uint64_t far = __ballot(r2 >= acc) & mask[r];
+                rest[r] = mask[r] & ~far;
+                any |= rest[r];
+                if (__builtin_amdgcn_inverse_ballot_w64(far)) {
+                    accept<kSafe, kQuad>(t[r], na.w, qa, qb, dx, dy, dz, r2, eps2);
+                    ++t[r].pc;
+                }
+            }
+            // The successor when nothing opens: an escape index always lies past its
+            // node; the maximum only keeps a corrupted record from looping.
+            const std::uint32_t step = cur + 1;
+            const std::uint32_t next = max(nb.y, step);
+            std::uint32_t go = next;
+            if (any != 0) {
+                if (nb.w != 0) {
+                    const double4 cb = node_geo[cur];
+                    const std::uint32_t b = nb.z, e = nb.z + nb.w;
+#pragma unroll
+                    for (int r = 0; r < kR; ++r) {
+                        if (rest[r] == 0) continue;
+                        const std::uint32_t here = __popcll(rest[r]);
+                        stopped += here;
+                        pp += static_cast<unsigned long long>(here) * nb.w -
+                              __popcll(__ballot(t[r].own == cur) & rest[r]);
+                        if (__builtin_amdgcn_inverse_ballot_w64(rest[r])) {
+                            leaf_pairs<kSafe>(t[r], cb, s_own[r][0][threadIdx.x], s_own[r][1][threadIdx.x],
+                                              s_own[r][2][threadIdx.x], leaf_rel, b, e, eps2);
+                        }
+                    }
+                } else {
+                    // Open: the children for those that did, then everyone here
+                    // goes on at `next`.
+                    lane_write(st_end, end, depth);
+#pragma unroll
+                    for (int r = 0; r < kR; ++r) {
+                        stopped += __popcll(rest[r]);
+                        lane_write(st_lo[r], static_cast<std::uint32_t>(mask[r]), depth);
+                        lane_write(st_hi[r], static_cast<std::uint32_t>(mask[r] >> 32), depth);
+                        mask[r] = rest[r];
+                    }
+                    ++depth;  // at most 21 levels
+                    end = next;
+                    go = step;
+                }
+            }
+            cur = go;
+            // The end of one or more sibling lists: back to the masks of the
+            // lists they lie in (cur > 0, so never past the outermost).
+            while (cur == end) {
+                --depth;
+                end = lane_read(st_end, depth);
+#pragma unroll
+                for (int r = 0; r < kR; ++r) {
+                    mask[r] = static_cast<std::uint64_t>(lane_read(st_lo[r], depth)) |
+                              static_cast<std::uint64_t>(lane_read(st_hi[r], depth)) << 32;
+                }
+            }
         }
     }
-    std::uint32_t pp = 0, pc = 0, visits = 0;
-    bool mixed = false;
-    const std::uint32_t seg0 = __builtin_amdgcn_readfirstlane(seg[0]);
 #pragma unroll
     for (int r = 0; r < kR; ++r) {
         kahan(t[r].px, t[r].sx, t[r].kx);
         kahan(t[r].py, t[r].sy, t[r].ky);
         kahan(t[r].pz, t[r].sz, t[r].kz);
-        if (valid[r]) {
-            const std::uint32_t dst = index[wave * (kLanes * kR) + kLanes * r + lane];
+        const std::uint32_t i = wave * (kLanes * kR) + kLanes * r + lane;
+        if (lane < kLanes && i < n) {
+            const std::uint32_t dst = index[i];
             ax[dst] = G * (static_cast<double>(t[r].sx) - static_cast<double>(t[r].kx));
             ay[dst] = G * (static_cast<double>(t[r].sy) - static_cast<double>(t[r].ky));
             az[dst] = G * (static_cast<double>(t[r].sz) - static_cast<double>(t[r].kz));
-            pp += t[r].pp;
-            pc += t[r].pc;
-            visits += t[r].visits;
         }
-        mixed = mixed || (valid[r] && seg[r] != seg0);
     }
     // Counts: a wave inside one system writes its sums to its own slot, summed
     // per system by walk_counts (atomics on one address would serialise every
-    // wave); a wave spanning two systems adds per target.
+    // wave); a wave spanning systems adds them per system.
     unsigned long long* mine_slot = wave_stats + 4 * static_cast<std::size_t>(wave);
-    if (__ballot(mixed) == 0) {
-        const unsigned long long wpp = wave_sum_u64(pp);
-        const unsigned long long wpc = wave_sum_u64(pc);
-        const unsigned long long wvisits = wave_sum_u64(visits);
-        if (lane == 0) {
-            mine_slot[0] = wpp;
-            mine_slot[1] = wpc;
-            mine_slot[2] = wvisits;
-            // Lane-target slots, 64 per count.
-            mine_slot[3] = static_cast<unsigned long long>(steps) * kR * kLanes / 64;
-        }
-    } else {
-#pragma unroll
-        for (int r = 0; r < kR; ++r) {
-            if (valid[r]) {
-                unsigned long long* st = stats + 4 * static_cast<std::size_t>(seg[r]);
-                atomicAdd(&st[0], static_cast<unsigned long long>(t[r].pp));
-                atomicAdd(&st[1], static_cast<unsigned long long>(t[r].pc));
-                atomicAdd(&st[2], static_cast<unsigned long long>(t[r].visits));
-            }
-        }
-        if (lane == 0) {
-            atomicAdd(&stats[4 * static_cast<std::size_t>(seg0) + 3],
-                      static_cast<unsigned long long>(steps) * kR * kLanes / 64);
-            mine_slot[0] = mine_slot[1] = mine_slot[2] = mine_slot[3] = 0;
-        }
+    const unsigned long long pc = accepted(t), visits = pc + stopped;
+    if (lane == 0) {
+        // Lane-target slots, 64 per count.
+        const unsigned long long slots = static_cast<unsigned long long>(steps) * (kR * kLanes) / 64;
+        const bool mixed = kMany && systems > 1;
+        if (mixed) add_counts(stats, seg0, pp, pc, visits, slots);
+        mine_slot[0] = mixed ? 0 : pp;
+        mine_slot[1] = mixed ? 0 : pc;
+        mine_slot[2] = mixed ? 0 : visits;
+        mine_slot[3] = mixed ? 0 : slots;
     }
 }
 
@@ -926,7 +997,7 @@ std::size_t layout_bytes(std::uint64_t n, std::size_t nodes, bool quadrupole, st
     const std::size_t per_node = nodes * (4 * 3 + 1 + 4 * kMaxChildren + 32 + 32 + sizeof(WalkNode) + per_quad);
     const std::size_t counters = 16 + 8 * 4 * static_cast<std::size_t>(segments) +
                                  8 * ((n + kBlock - 1) / kBlock) +
-                                 32 * (kBlock / 64) * ((2 * n + kBlock - 1) / kBlock) + 512;
+                                 32 * (kBlock / 64) * (((64 / kMinLanes) * n + kBlock - 1) / kBlock) + 512;
     return per_particle + per_node + counters + 22 * 256 + 64;
 }
 
@@ -960,8 +1031,8 @@ Layout layout(orr_ctx* ctx, std::uint64_t n, std::size_t nodes, bool quadrupole,
     L.c32 = carve<std::uint32_t>(p, 4);
     L.c64 = carve<unsigned long long>(p, 4 * static_cast<std::size_t>(segments));
     L.block_counts = carve<uint2>(p, (n + kBlock - 1) / kBlock);
-    // Half-lane walks (kLanes = 32) launch twice the waves of full ones.
-    L.wave_stats = carve<unsigned long long>(p, 4 * (kBlock / 64) * ((2 * n + kBlock - 1) / kBlock));
+    // Walks with fewer lanes a wave launch more waves.
+    L.wave_stats = carve<unsigned long long>(p, 4 * (kBlock / 64) * (((64 / kMinLanes) * n + kBlock - 1) / kBlock));
     return L;
 }
 
@@ -1060,30 +1131,37 @@ void tree_enqueue(orr_ctx* ctx, const orr_tree_args& a, const SegmentView& segs,
         const float eps2 = static_cast<float>(a.softening_squared);
         const bool safe = !(a.softening_squared > 0);
         const bool quad = a.quadrupole != 0;
-        // Two targets per lane pay off for one large system (measured: 4.5 % at
-        // N = 2^21); zero in the context means choose by that rule.
-        const int R = ctx->walk_targets_per_lane != 0 ? ctx->walk_targets_per_lane
-                      : (segs.count == 1 && n >= (std::uint64_t{1} << 20) ? 2 : 1);
-        // Half the lanes of each wave for a launch of at most kHalfLaneWaves
-        // full waves (twice the waves, each over a tighter group of targets);
-        // zero in the context means choose by that rule. A target's walk and
-        // sums do not depend on which targets share its wave, so the results
-        // are the same bits either way.
+        // One target a lane at every size (2^21 particles, quadrupoles: 8.3 ms
+        // with one or two; below, one is faster); two only when configured.
+        const int R = ctx->walk_targets_per_lane != 0 ? ctx->walk_targets_per_lane : 1;
+        // Fewer targets a wave for a small launch (more waves, each over a
+        // tighter group of targets); zero in the context means choose by that
+        // rule. A target's walk and sums do not depend on which targets share
+        // its wave, so the results are the same bits either way.
         const std::uint64_t full_waves = (n + 64u * R - 1) / (64u * R);
         const int lanes = ctx->walk_lanes != 0 ? ctx->walk_lanes
-                          : (full_waves <= kHalfLaneWaves ? 32 : 64);
-        using Walk = decltype(&tree_walk<1, true, true, 64>);
-        auto pick = [&](auto r, auto l) -> Walk {
+                          : full_waves <= kQuarterLaneWaves && R == 1 ? 16
+                          : full_waves <= kHalfLaneWaves ? 32 : 64;
+        using Walk = decltype(&tree_walk<1, true, true, 64, false>);
+        auto many = [&](auto r, auto l, auto sv, auto q) -> Walk {
             constexpr int kRr = decltype(r)::value, kLl = decltype(l)::value;
-            return safe ? (quad ? tree_walk<kRr, true, true, kLl> : tree_walk<kRr, true, false, kLl>)
-                        : (quad ? tree_walk<kRr, false, true, kLl> : tree_walk<kRr, false, false, kLl>);
+            constexpr bool kS = decltype(sv)::value, kQ = decltype(q)::value;
+            return seg_of != nullptr ? tree_walk<kRr, kS, kQ, kLl, true> : tree_walk<kRr, kS, kQ, kLl, false>;
+        };
+        using Yes = std::true_type;
+        using No = std::false_type;
+        auto pick = [&](auto r, auto l) -> Walk {
+            return safe ? (quad ? many(r, l, Yes{}, Yes{}) : many(r, l, Yes{}, No{}))
+                        : (quad ? many(r, l, No{}, Yes{}) : many(r, l, No{}, No{}));
         };
         using One = std::integral_constant<int, 1>;
         using Two = std::integral_constant<int, 2>;
+        using Quarter = std::integral_constant<int, 16>;
         using Half = std::integral_constant<int, 32>;
         using Full = std::integral_constant<int, 64>;
         const Walk walk = R == 2 ? (lanes == 32 ? pick(Two{}, Half{}) : pick(Two{}, Full{}))
-                                 : (lanes == 32 ? pick(One{}, Half{}) : pick(One{}, Full{}));
+                                 : (lanes == 16 ? pick(One{}, Quarter{})
+                                                : lanes == 32 ? pick(One{}, Half{}) : pick(One{}, Full{}));
         const std::uint32_t per_wave = static_cast<std::uint32_t>(lanes * R);
         const std::uint32_t per_block = (kBlock / 64) * per_wave;
         const std::uint32_t walk_blocks = (n32 + per_block - 1) / per_block;

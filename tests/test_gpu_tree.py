@@ -357,3 +357,25 @@ def test_replayed_evaluations_are_bitwise(ctx):
     ref = (np.zeros(q.n), np.zeros(q.n), np.zeros(q.n))
     fresh.evaluate((q.x, q.y, q.z), q.m, ref)
     assert all(np.array_equal(acc[k], ref[k]) for k in range(3))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quadrupole", [False, True])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 65, 1000, 16384, 16385, 131072, 131073])
+def test_waves_chosen_by_size_walk_as_full_waves(ctx, n, quadrupole):
+    """The wave width taken by size (16, 32 or 64 targets) against 64: the same
+    accelerations and counts bit for bit, at the rule's edges and in ragged last waves."""
+    p = oracle.plummer(n, 11)
+    out = []
+    try:
+        for lanes in (-1, 64):
+            ctx.set_tree_config(lanes=lanes)
+            s = E.HipTreeSolver(E.TreeParameters(0.6, 8, quadrupole=quadrupole), E.Softening(0.01), context=ctx)
+            a = [np.zeros(n) for _ in range(3)]
+            s.evaluate((p.x, p.y, p.z), p.m, a)
+            c = s.interaction_count()
+            out.append((np.stack(a), c.particle_particle, c.particle_cell, s.node_visits()))
+    finally:
+        ctx.set_tree_config(lanes=-1)
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:]
