@@ -104,90 +104,105 @@ struct Compensated {
 
 constexpr int kTerms = 8;  // ke, px, py, pz, lx, ly, lz, pe
 
-// Columns of the potential's rows are summed in at most kColumnChunks chunks
-// of at least kColumnMin columns (whole tiles of kPotTile), so a system of a
-// few thousand particles still spreads over many waves.
-constexpr int kPotTile = 256;  // columns staged in LDS per step = threads per block
-constexpr std::uint64_t kColumnMin = 2048;
+// The potential's rows are summed in column chunks of whole kPotTile columns:
+// at most kColumnChunks of them for a system whose row blocks fill the device,
+// up to kMaxChunks below that (a few thousand particles otherwise give a few
+// dozen workgroups: a diagnostic of 4096 took 182 us with chunks of 2048
+// columns, 58 us with chunks of 256).
+constexpr int kPotTile = 256;  // rows of a block, one a thread
 constexpr std::uint64_t kColumnChunks = 16;
+constexpr std::uint64_t kMaxChunks = 64;
+// Row blocks times chunks wanted: a few dozen rounds of waves even out the
+// blocks on the diagonal (65,536 particles: 1.43 ms at 4096, 1.38 at 16,384).
+constexpr std::uint64_t kPotBlocks = 16384;
 
 __host__ __device__ inline std::uint64_t column_width(std::uint64_t n) {
-    const std::uint64_t even = (n + kColumnChunks - 1) / kColumnChunks;
-    const std::uint64_t w = even > kColumnMin ? even : kColumnMin;
+    const std::uint64_t row_blocks = (n + kPotTile - 1) / kPotTile;
+    std::uint64_t chunks = row_blocks == 0 ? 1 : kPotBlocks / row_blocks;
+    chunks = chunks < kColumnChunks ? kColumnChunks : (chunks > kMaxChunks ? kMaxChunks : chunks);
+    const std::uint64_t w = (n + chunks - 1) / chunks;
     return (w + kPotTile - 1) / kPotTile * kPotTile;
 }
 
-// 1 / sqrt(v) in FP64: the hardware reciprocal square root refined by two
-// Newton steps, y <- y (3/2 - (v/2) y^2) with the residual by FMA (each step
-// squares the relative error, so the result is within an ulp or two).
-// Branch-free: v = 0 gives +inf and NaN stays NaN, as 1 / sqrt(v) would.
-__device__ inline double inverse_sqrt(double v) {
-    const double h = 0.5 * v;
-    double y = __builtin_amdgcn_rsq(v);
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-        const double e = fma(-h, y * y, 0.5);
-        y = fma(y, e, y);
+// Accumulates m / sqrt(v), v = |d|^2 + e2 for the separation d = (dx, dy, dz),
+// into (sum, fix): the hardware reciprocal square root y (relative error below
+// 2^-22) and one third-order step, y (1 + e / 2 + 3 e^2 / 8) with
+// e = 1 - v y^2, whose own error is below 2.5 e^3 -- under the rounding of the
+// result. The leading terms and the corrections are summed apart, so that
+// neither waits on the other: thirteen FP64 instructions and the root a pair.
+// v = 0 (two coincident particles without softening) gives +inf and a NaN
+// stays one, as m / sqrt(v) would; with softening v is never zero.
+template<bool kSoft>
+__device__ __forceinline__ void add_potential(double m, double dx, double dy, double dz, double e2,
+                                              double& sum, double& fix) {
+    const double v = fma(dz, dz, fma(dy, dy, fma(dx, dx, e2)));
+    const double y = __builtin_amdgcn_rsq(v);
+    const double e = fma(-(v * y), y, 1.0);
+    const double lead = m * y;
+    const double half = lead * e;
+    sum += lead;
+    if constexpr (kSoft) {
+        fix = fma(half, fma(0.375, e, 0.5), fix);
+    } else {
+        fix = v == 0.0 ? fix : fma(half, fma(0.375, e, 0.5), fix);
     }
-    return v > 0.0 ? y : (v == 0.0 ? __builtin_huge_val() : __builtin_nan(""));
 }
 
-// m / sqrt(|d|^2 + e2) for the separation d = (dx, dy, dz).
-__device__ inline double pair_potential(double m, double dx, double dy, double dz, double e2) {
-    return m * inverse_sqrt(fma(dz, dz, fma(dy, dy, fma(dx, dx, e2))));
-}
-
-// Row i of the potential over column chunk blockIdx.y: a plain FP64 sum over
-// j > i of m_j / sqrt(r^2 + e^2) in index order (r^2 + e^2 by FMA) (diagnostics.cpp:129-158 sums
-// the whole row plainly; here the chunks' sums are folded in chunk order).
-// A block holds kPotTile rows; the chunk's columns pass through LDS a tile at
-// a time and every lane reads each staged column (a broadcast). Blocks wholly
-// below the diagonal write zeros and leave.
+// Row i of the potential over column chunk blockIdx.y: an FP64 sum over j > i
+// of m_j / sqrt(r^2 + e^2) in index order (diagnostics.cpp:129-158 sums the
+// whole row plainly; here the chunks' sums are folded in chunk order). A block
+// holds kPotTile rows, one a thread; the columns are wave-uniform and read four
+// at a time through the scalar unit, so no lane waits on LDS or a barrier
+// (staged through LDS, the four broadcast reads a pair took nearly as many
+// cycles a CU as the arithmetic). Blocks wholly below the diagonal write zeros
+// and leave. Bound by FP64 issue (4.5 cycles an instruction, 16 the root):
+// a diagnostic of 65,536 particles 1.82 -> 1.38 ms, of 131,072 6.23 -> 4.70 ms,
+// 1.8e12 pairs a second.
+template<bool kSoft>
 __global__ __launch_bounds__(kPotTile) void potential_rows(std::uint64_t n, std::uint64_t width,
                                                            const double* __restrict__ x,
                                                            const double* __restrict__ y,
                                                            const double* __restrict__ z,
                                                            const double* __restrict__ m, double e2,
                                                            double* __restrict__ rows) {
-    __shared__ double sx[kPotTile], sy[kPotTile], sz[kPotTile], sm[kPotTile];
     const std::uint64_t row0 = static_cast<std::uint64_t>(blockIdx.x) * kPotTile;
     const std::uint64_t i = row0 + threadIdx.x;
     const std::uint64_t c0 = static_cast<std::uint64_t>(blockIdx.y) * width;
     const std::uint64_t c1 = c0 + width < n ? c0 + width : n;
-    // First column any row of the block needs: row0 + 1.
-    const std::uint64_t j_begin = c0 > row0 + 1 ? c0 : row0 + 1;
-    double inter = 0.0;
-    if (j_begin < c1) {
+    // From here on the columns lie above every row of the block.
+    const std::uint64_t beyond = row0 + kPotTile;
+    std::uint64_t j = c0 > row0 + 1 ? c0 : row0 + 1;
+    double sum = 0.0, fix = 0.0;
+    if (j < c1) {
         const bool valid_row = i < n;
         const double xi = valid_row ? x[i] : 0.0, yi = valid_row ? y[i] : 0.0;
         const double zi = valid_row ? z[i] : 0.0;
-        // Tiles aligned to kPotTile from the first one holding j_begin.
-        for (std::uint64_t t0 = j_begin / kPotTile * kPotTile; t0 < c1; t0 += kPotTile) {
-            __syncthreads();
-            const std::uint64_t j = t0 + threadIdx.x;
-            const bool in = j < c1;
-            sx[threadIdx.x] = in ? x[j] : 0.0;
-            sy[threadIdx.x] = in ? y[j] : 0.0;
-            sz[threadIdx.x] = in ? z[j] : 0.0;
-            sm[threadIdx.x] = in ? m[j] : 0.0;
-            __syncthreads();
-            const std::uint64_t t1 = t0 + kPotTile < c1 ? t0 + kPotTile : c1;
-            const int count = static_cast<int>(t1 - t0);
-            if (t0 > row0 + kPotTile - 1 && count == kPotTile) {
-                // Every column of the tile lies above every row of the block.
-#pragma unroll 4
-                for (int k = 0; k < kPotTile; ++k) {
-                    inter += pair_potential(sm[k], sx[k] - xi, sy[k] - yi, sz[k] - zi, e2);
+        for (; j + 4 <= c1; j += 4) {
+            double mj[4], xj[4], yj[4], zj[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                mj[k] = m[j + k];
+                xj[k] = x[j + k];
+                yj[k] = y[j + k];
+                zj[k] = z[j + k];
+            }
+            if (j >= beyond) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    add_potential<kSoft>(mj[k], xj[k] - xi, yj[k] - yi, zj[k] - zi, e2, sum, fix);
                 }
             } else {
-                for (int k = 0; k < count; ++k) {
-                    if (t0 + k <= i) continue;
-                    inter += pair_potential(sm[k], sx[k] - xi, sy[k] - yi, sz[k] - zi, e2);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if (j + k > i) add_potential<kSoft>(mj[k], xj[k] - xi, yj[k] - yi, zj[k] - zi, e2, sum, fix);
                 }
             }
         }
+        for (; j < c1; ++j) {
+            if (j > i) add_potential<kSoft>(m[j], x[j] - xi, y[j] - yi, z[j] - zi, e2, sum, fix);
+        }
     }
-    if (i < n) rows[static_cast<std::uint64_t>(blockIdx.y) * n + i] = inter;
+    if (i < n) rows[static_cast<std::uint64_t>(blockIdx.y) * n + i] = sum + fix;
 }
 
 // Per-particle terms, term-major [kTerms][n].
@@ -230,6 +245,7 @@ __global__ __launch_bounds__(64) void chunk_sums(std::uint64_t n, const double* 
     const std::uint64_t b = chunk * per;
     const std::uint64_t e = b + per < n ? b + per : n;
     Compensated s;
+#pragma unroll 8
     for (std::uint64_t i = b; i < e; ++i) s.add(terms[term * n + i]);
     out[2 * id] = s.total;
     out[2 * id + 1] = s.correction;
@@ -245,9 +261,22 @@ __global__ __launch_bounds__(256) void final_sums(std::uint32_t chunks,
     __shared__ double s_total[256], s_corr[256];
     const int term = threadIdx.x / 32, lane = threadIdx.x % 32;
     Compensated acc;
-    for (std::uint32_t c = lane; c < chunks; c += 32) {
-        acc.add(parts[2 * (term * chunks + c)]);
-        acc.add(parts[2 * (term * chunks + c) + 1]);
+    // Loads first, eight chunks at a time, so that they are in flight together.
+    for (std::uint32_t c0 = lane; c0 < chunks; c0 += 8 * 32) {
+        double total[8], correction[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const std::uint32_t c = c0 + 32 * u < chunks ? c0 + 32 * u : c0;
+            total[u] = parts[2 * (term * chunks + c)];
+            correction[u] = parts[2 * (term * chunks + c) + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (c0 + 32 * u < chunks) {
+                acc.add(total[u]);
+                acc.add(correction[u]);
+            }
+        }
     }
     s_total[threadIdx.x] = acc.total;
     s_corr[threadIdx.x] = acc.correction;
@@ -334,7 +363,8 @@ void diagnostics_enqueue(orr_ctx* ctx, std::uint64_t n, const double* x, const d
     double* result = parts + 2 * kTerms * chunks;
     PhaseTimer t(ctx, kEnergy);
     const std::uint32_t row_blocks = static_cast<std::uint32_t>((n + 255) / 256);
-    hipLaunchKernelGGL(potential_rows, dim3(static_cast<std::uint32_t>((n + kPotTile - 1) / kPotTile), columns),
+    auto rows_kernel = e2 > 0.0 ? potential_rows<true> : potential_rows<false>;
+    hipLaunchKernelGGL(rows_kernel, dim3(static_cast<std::uint32_t>((n + kPotTile - 1) / kPotTile), columns),
                        dim3(kPotTile), 0, ctx->stream, n, width, x, y, z, m, e2, rows);
     ORR_LAUNCHED("potential_rows");
     hipLaunchKernelGGL(diagnostic_terms, dim3(row_blocks), dim3(256), 0, ctx->stream, n, x, y, z,

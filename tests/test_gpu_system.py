@@ -440,3 +440,19 @@ def test_fused_step_equals_host_kicks_around_device_evaluations(ctx, integrator,
         assert np.array_equal(got[name], x[c]), name
         assert np.array_equal(got["v" + name], v[c]), "v" + name
         assert np.array_equal(got["a" + name], a[c]), "a" + name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("eps", [0.0, 0.01])
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 255, 256, 257, 259, 511, 513, 1025, 4097])
+def test_potential_at_tile_edges(ctx, n, eps):
+    """The potential's rows at the edges of a block's rows, a chunk's columns and a
+    round of four: all terms have one sign, so a plain FP64 sum of n of them is within
+    n 2^-53 of the compensated one, and each term within a few units in the last place."""
+    p = oracle.plummer(n, 7 + n)
+    s = E.DeviceSystem(ctx, n)
+    s.upload(*p.arrays())
+    got = s.diagnostics(eps)["potential"]
+    want = oracle.diagnostics(p, eps * eps)["potential"]
+    s.close()
+    assert abs(got - want) <= (n + 16) * 2.0**-53 * abs(want)
