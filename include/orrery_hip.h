@@ -115,11 +115,11 @@ ORR_API int orr_direct_eval(orr_ctx* ctx, const orr_direct_args* args);
  * of 16 MiB per GPU, held from the first call on that GPU until the process
  * ends; nothing is allocated, no graph is built, phases are not timed. Same
  * arguments and result as orr_direct_eval, with these limits: count at most
- * 32,768 (ORR_ERR_LENGTH beyond); always the one-sided kernel; where the
- * one-sided kernel's split partials would not fit, fewer splits (the same
- * terms in fewer Kahan-summed groups, so not the same bits as orr_direct_eval;
- * the same bits whenever they fit and orr_direct_eval takes the one-sided
- * kernel). Calls that overlap on one GPU share the array and race. */
+ * 32,768 (ORR_ERR_LENGTH beyond); always the one-sided kernel; where a sum
+ * and compensation per target and group of source tiles would not fit, fewer
+ * groups (the same terms in fewer Kahan-summed groups, so not the same bits as
+ * orr_direct_eval; the same bits whenever they fit and orr_direct_eval takes
+ * the one-sided kernel). Calls that overlap on one GPU share the array and race. */
 ORR_API int orr_direct_eval_static(orr_ctx* ctx, const orr_direct_args* args);
 /* The limits above: the largest count and the scratch bytes per GPU. */
 ORR_API int orr_direct_static_limits(uint64_t* max_count, uint64_t* scratch_bytes);
@@ -129,8 +129,11 @@ ORR_API int orr_direct_static_limits(uint64_t* max_count, uint64_t* scratch_byte
  * targets_per_lane in {1, 2, 4}; refine = 1 applies a Newton step to the
  * hardware reciprocal square root of the cubed argument (off by default: the
  * pair terms' FP32 rounding, the close pairs' double-float terms and the
- * compensated sums keep the force within 1e-6 relative without it); block_target is the number of thread blocks the
- * source range is split to reach (default 32768). pair_mode 1 (default)
+ * compensated sums keep the force within 1e-6 relative without it);
+ * block_target (default 32768) sets how many source tiles the one-sided kernel
+ * sums together in FP32: as many groups as make that many blocks of four
+ * target tiles times groups, each of at least one tile (the groups' sums are
+ * added in FP64). pair_mode 1 (default)
  * evaluates each far pair of 64-particle tiles once and applies it to both
  * tiles where that is faster and fits: from 704 tiles (44,993 particles) up to
  * 856,064 particles (3 doubles per particle and later block of 8 tiles within

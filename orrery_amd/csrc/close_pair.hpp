@@ -42,26 +42,33 @@ ORR_HD inline double seed_rsq64(double x) {
 #endif
 }
 
-// G = (|D|^2 + eps2)^(-3/2) D for the separation D = b - a of two positions
-// given as (hi, lo) float pairs in one frame. R > 0 is the caller's condition
-// (a close pair is never a coincident, unsoftened one).
-ORR_HD inline void close_pair(const float ah[3], const float al[3], const float bh[3],
-                              const float bl[3], float eps2, double G[3]) {
+// G = (|D|^2 + eps2)^(-3/2) D for the separation D = b - a of two positions in
+// one frame, a in FP64 and b as a (hi, lo) float pair (both sums exact in
+// FP64). R > 0 is the caller's condition (a close pair is never a coincident,
+// unsoftened one). The root's seed y (relative error below 2^-22) takes one
+// third-order step, y (1 + e / 2 + 3 e^2 / 8) with e = 1 - r2 y^2, whose own
+// error is below 2.5 e^3.
+ORR_HD inline void close_pair(const double a[3], const float bh[3], const float bl[3], float eps2,
+                              double G[3]) {
 #pragma clang fp contract(off)
     double d[3];
     for (int c = 0; c < 3; ++c) {
-        d[c] = (static_cast<double>(bh[c]) + static_cast<double>(bl[c])) -
-               (static_cast<double>(ah[c]) + static_cast<double>(al[c]));
+        d[c] = (static_cast<double>(bh[c]) + static_cast<double>(bl[c])) - a[c];
     }
     const double r2 = __builtin_fma(d[2], d[2], __builtin_fma(d[1], d[1], __builtin_fma(d[0], d[0], static_cast<double>(eps2))));
-    const double h = 0.5 * r2;
     double y = seed_rsq64(r2);
-    for (int k = 0; k < 2; ++k) {
-        const double e = __builtin_fma(-h, y * y, 0.5);
-        y = __builtin_fma(y, e, y);
-    }
+    const double e = __builtin_fma(-(r2 * y), y, 1.0);
+    y = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
     const double g = (y * y) * y;
     for (int c = 0; c < 3; ++c) G[c] = g * d[c];
+}
+
+// The same with a as a (hi, lo) float pair.
+ORR_HD inline void close_pair(const float ah[3], const float al[3], const float bh[3],
+                              const float bl[3], float eps2, double G[3]) {
+    double a[3];
+    for (int c = 0; c < 3; ++c) a[c] = static_cast<double>(ah[c]) + static_cast<double>(al[c]);
+    close_pair(a, bh, bl, eps2, G);
 }
 
 // v split into floats hi + lo (hi the rounding of v, lo that of the rest).

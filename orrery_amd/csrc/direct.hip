@@ -300,15 +300,24 @@ __device__ __forceinline__ void source_tile(
     }
     const float4* __restrict__ src_lo = packed_lo + static_cast<std::size_t>(J) * kTile;
     float px[R], py[R], pz[R], pkx[R], pky[R], pkz[R], lim[R];
-    std::uint64_t close[R];  // per lane: bit j set when source j is a close pair
+    // Per lane, the sources that are close pairs: the flags of 32 sources in a
+    // word, shifted in from the right (one add with carry a source).
+    std::uint32_t close[R][2];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         px[r] = py[r] = pz[r] = pkx[r] = pky[r] = pkz[r] = 0.f;
         lim[r] = close_limit(ce[r].w, E.w, eps2);
-        close[r] = 0;
+        close[r][0] = close[r][1] = 0;
     }
 #pragma unroll 1
     for (int j0 = 0; j0 < kTile; j0 += kNearRun) {
+        if (j0 == kTile / 2) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                close[r][0] = close[r][1];
+                close[r][1] = 0;
+            }
+        }
         float qx[R], qy[R], qz[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) qx[r] = qy[r] = qz[r] = 0.f;
@@ -325,9 +334,10 @@ __device__ __forceinline__ void source_tile(
                 r2 = __builtin_fmaf(dy, dy, r2);
                 r2 = __builtin_fmaf(dz, dz, r2);
                 // A close pair's FP32 term is left out here and added in
-                // FP64 below.
-                const bool near_pair = r2 < lim[r] && r2 > 0.f;
-                close[r] |= near_pair ? std::uint64_t{1} << j : std::uint64_t{0};
+                // FP64 below (r^2 holds eps^2, so it is zero only without
+                // softening).
+                const bool near_pair = r2 < lim[r] && (!kSafe || r2 > 0.f);
+                close[r][1] = close[r][1] + close[r][1] + (near_pair ? 1u : 0u);
                 const float f = near_pair ? 0.f : q.w * inv_cubed<kSafe, kRefine>(r2);
                 qx[r] = __builtin_fmaf(f, dx, qx[r]);
                 qy[r] = __builtin_fmaf(f, dy, qy[r]);
@@ -344,15 +354,18 @@ __device__ __forceinline__ void source_tile(
     // The close pairs, each lane over its own (few): sources read by index.
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        std::uint64_t bits = close[r];
+        const double t[3] = {static_cast<double>(th[r][0]) + static_cast<double>(tl[r][0]),
+                             static_cast<double>(th[r][1]) + static_cast<double>(tl[r][1]),
+                             static_cast<double>(th[r][2]) + static_cast<double>(tl[r][2])};
+        std::uint64_t bits = static_cast<std::uint64_t>(close[r][0]) << 32 | close[r][1];
         while (bits != 0) {
-            const int j = __builtin_ctzll(bits);
-            bits &= bits - 1;
+            const int j = __builtin_clzll(bits);  // the first source is the highest bit
+            bits &= ~(std::uint64_t{1} << (63 - j));
             const float4 q = src[j];
             const float4 ql = src_lo[j];
             const float bh[3] = {q.x, q.y, q.z}, bl[3] = {ql.x, ql.y, ql.z};
             double G[3];
-            close_pair(th[r], tl[r], bh, bl, eps2, G);
+            close_pair(t, bh, bl, eps2, G);
             const double mq = q.w;
             float h, l;
             split(mq * G[0], h, l);
@@ -408,86 +421,17 @@ __global__ __launch_bounds__(256) void near_mask(const double4* __restrict__ cen
     }
 }
 
-template<int R, bool kSafe, bool kRefine, bool kMask>
-__global__ __launch_bounds__(kBlock) void direct_tiles(const float4* __restrict__ packed,
-                                                       const float4* __restrict__ packed_lo,
-                                                       const double4* __restrict__ centres,
-                                                       const float4* __restrict__ extents,
-                                                       const std::uint32_t* __restrict__ mask,
-                                                       std::uint32_t npad, std::uint32_t tiles,
-                                                       std::uint32_t tiles_per_split, float eps2,
-                                                       float* __restrict__ partial) {
-    const std::uint32_t split = blockIdx.y;
-    const std::uint32_t j0 = split * tiles_per_split;
-    const std::uint32_t j1 = min(tiles, j0 + tiles_per_split);
-    const std::uint32_t base = blockIdx.x * (kBlock * R) + threadIdx.x;
+// Where a one-sided evaluation's sums go: the fold's arguments.
+struct FieldOut {
+    std::uint64_t n = 0;
+    const std::uint32_t* order = nullptr;
+    double G = 1.0;
+    double* ax = nullptr;
+    double* ay = nullptr;
+    double* az = nullptr;
+    FusedKick kick;
+};
 
-    float ox[R], oy[R], oz[R], lx[R], ly[R], lz[R];
-    double cx[R], cy[R], cz[R];
-    float4 ce[R];
-    float sx[R], sy[R], sz[R], kx[R], ky[R], kz[R];
-    std::uint32_t row[R];  // first mask word of each target tile's row
-    const std::uint32_t words = (tiles + 31) / 32;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const std::uint32_t k = min(base + r * kBlock, npad - 1);
-        const float4 o = packed[k];
-        const float4 l = packed_lo[k];
-        // A wave's 64 targets are one whole tile (npad is a multiple of kTile,
-        // and a wave past the end clamps every lane to the last tile), so the
-        // tile's centre and extents are wave-uniform: scalar loads, SGPRs.
-        const std::uint32_t tile = __builtin_amdgcn_readfirstlane(k / kTile);
-        const double4 c = centres[tile];
-        ox[r] = o.x;
-        oy[r] = o.y;
-        oz[r] = o.z;
-        lx[r] = l.x;
-        ly[r] = l.y;
-        lz[r] = l.z;
-        cx[r] = c.x;
-        cy[r] = c.y;
-        cz[r] = c.z;
-        ce[r] = extents[tile];
-        row[r] = tile * words;
-        sx[r] = sy[r] = sz[r] = 0.f;
-        kx[r] = ky[r] = kz[r] = 0.f;
-    }
-
-    std::uint32_t bits = 0;
-    for (std::uint32_t J = j0; J < j1; ++J) {
-        bool near = false;
-        if constexpr (kMask) {
-            if (J == j0 || (J & 31u) == 0) {
-                bits = 0;
-#pragma unroll
-                for (int r = 0; r < R; ++r) bits |= mask[row[r] + J / 32];
-            }
-            near = ((bits >> (J & 31u)) & 1u) != 0;
-        }
-        source_tile<R, kSafe, kRefine, kMask>(packed, packed_lo, centres, extents, J, near, eps2,
-                                              ox, oy, oz, lx, ly, lz, cx, cy, cz, ce, sx, sy, sz, kx,
-                                              ky, kz);
-    }
-
-    // Component c of target k at partial[(6 split + c) npad + k], in 64-bit
-    // offsets (6 npad exceeds 32 bits from npad = 2^30 / 1.5).
-    const std::size_t np = npad;
-    float* out = partial + static_cast<std::size_t>(split) * 6 * np;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const std::uint32_t k = base + r * kBlock;
-        if (k < npad) {
-            out[k] = sx[r];
-            out[np + k] = sy[r];
-            out[2 * np + k] = sz[r];
-            out[3 * np + k] = kx[r];
-            out[4 * np + k] = ky[r];
-            out[5 * np + k] = kz[r];
-        }
-    }
-}
-
-// Fixed-order FP64 fold of the splits; sum - compensation per split.
 // The fold's output: a, and the fused kick's v += s a when there is one.
 __device__ __forceinline__ void store_field(std::uint64_t dst, double gx, double gy, double gz,
                                             double* __restrict__ ax, double* __restrict__ ay,
@@ -502,25 +446,127 @@ __device__ __forceinline__ void store_field(std::uint64_t dst, double gx, double
     }
 }
 
-__global__ __launch_bounds__(256) void direct_reduce(const float* __restrict__ partial,
-                                                     std::uint32_t splits, std::uint32_t npad,
-                                                     std::uint64_t n,
-                                                     const std::uint32_t* __restrict__ order,
-                                                     double G, double* __restrict__ ax,
-                                                     double* __restrict__ ay,
-                                                     double* __restrict__ az, FusedKick kick) {
-    const std::uint64_t k = static_cast<std::uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
-    for (std::uint32_t s = 0; s < splits; ++s) {
-        const std::size_t np = npad;
-        const float* p = partial + static_cast<std::size_t>(s) * 6 * np;
-        a0 += static_cast<double>(p[k]) - static_cast<double>(p[3 * np + k]);
-        a1 += static_cast<double>(p[np + k]) - static_cast<double>(p[4 * np + k]);
-        a2 += static_cast<double>(p[2 * np + k]) - static_cast<double>(p[5 * np + k]);
+// One-sided sums. A wave owns R target tiles (R lanes' worth of whole tiles, so
+// a tile's centre and extents are wave-uniform) and takes groups of
+// `per_group` source tiles; a group's sums start fresh in FP32 with their Kahan
+// compensations and are added to the wave's FP64 sums as sum - compensation, so
+// a wave leaves 24 bytes a target whatever number of groups it took (it used to
+// leave them a group: 150 MB and 0.1 ms of an evaluation at N = 20,001).
+//
+// The groups are dealt to the blocks of a target (gridDim.y) in turn: near
+// source tiles, which cost several times a far one, lie together around the
+// target in Morton order and would otherwise all fall to one block. A wave
+// finds which of its next 64 source tiles are near with one test a lane.
+//
+// The four waves of a block have target tiles of their own and meet the same
+// source tiles at about the same time, so the scalar cache serves three of the
+// four (four waves of one target on different source tiles took 1.6 times as
+// long at N = 20,001). With one block a target (gridDim.y == 1) the field is
+// written here.
+template<int R, bool kSafe, bool kRefine>
+__global__ __launch_bounds__(kBlock) void direct_fold(
+    const float4* __restrict__ packed, const float4* __restrict__ packed_lo,
+    const double4* __restrict__ centres, const float4* __restrict__ extents, std::uint32_t tiles,
+    std::uint32_t per_group, std::uint32_t groups, float eps2, double* __restrict__ partial, FieldOut out) {
+    constexpr int kWaves = kBlock / kTile;
+    __shared__ double sums[kWaves][3 * R][kTile];
+    const unsigned lane = threadIdx.x & (kTile - 1);
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kTile);
+    // Target tile r of the wave (one past the last is worked on as the last and writes nothing).
+    auto target_tile = [&](int r) { return (blockIdx.x * R + r) * kWaves + wave; };
+    float ox[R], oy[R], oz[R], lx[R], ly[R], lz[R];
+    double cx[R], cy[R], cz[R];
+    float4 ce[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const std::uint32_t tile = min(target_tile(r), tiles - 1);
+        const float4 o = packed[static_cast<std::size_t>(tile) * kTile + lane];
+        const float4 l = packed_lo[static_cast<std::size_t>(tile) * kTile + lane];
+        const double4 c = centres[tile];
+        ox[r] = o.x;
+        oy[r] = o.y;
+        oz[r] = o.z;
+        lx[r] = l.x;
+        ly[r] = l.y;
+        lz[r] = l.z;
+        cx[r] = c.x;
+        cy[r] = c.y;
+        cz[r] = c.z;
+        ce[r] = extents[tile];
     }
-    const std::uint64_t dst = order != nullptr ? order[k] : k;
-    store_field(dst, G * a0, G * a1, G * a2, ax, ay, az, kick);
+    // The lane's own FP64 sums, in LDS: touched once a group, and six registers
+    // more a target would cost the eighth wave of a SIMD.
+#pragma unroll
+    for (int c = 0; c < 3 * R; ++c) sums[wave][c][lane] = 0.0;
+    const std::uint32_t stride = gridDim.y;
+    std::uint32_t met = 0;        // source tiles taken so far
+    std::uint64_t near_bits = 0;  // of the 64 from met & ~63
+    for (std::uint32_t g = blockIdx.y; g < groups; g += stride) {
+        float sx[R], sy[R], sz[R], kx[R], ky[R], kz[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) sx[r] = sy[r] = sz[r] = kx[r] = ky[r] = kz[r] = 0.f;
+        for (std::uint32_t o = 0; o < per_group && g * per_group + o < tiles; ++o, ++met) {
+            if (met % 64 == 0) {
+                const std::uint32_t gg = g + (o + lane) / per_group * stride;
+                const std::uint32_t J = gg * per_group + (o + lane) % per_group;
+                const bool valid = gg < groups && J < tiles;
+                const double4 C = centres[valid ? J : 0];
+                const float4 E = extents[valid ? J : 0];
+                bool near = false;
+#pragma unroll
+                for (int r = 0; r < R; ++r) near = near || near_tiles(C, E, cx[r], cy[r], cz[r], ce[r]);
+                near_bits = __ballot(valid && near);
+            }
+            const bool near = ((near_bits >> (met % 64)) & 1u) != 0;
+            source_tile<R, kSafe, kRefine, true>(packed, packed_lo, centres, extents, g * per_group + o, near,
+                                                 eps2, ox, oy, oz, lx, ly, lz, cx, cy, cz, ce, sx, sy, sz, kx,
+                                                 ky, kz);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            sums[wave][3 * r][lane] += static_cast<double>(sx[r]) - static_cast<double>(kx[r]);
+            sums[wave][3 * r + 1][lane] += static_cast<double>(sy[r]) - static_cast<double>(ky[r]);
+            sums[wave][3 * r + 2][lane] += static_cast<double>(sz[r]) - static_cast<double>(kz[r]);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const std::uint32_t tile = target_tile(r);
+        if (tile >= tiles) continue;
+        const double a[3] = {sums[wave][3 * r][lane], sums[wave][3 * r + 1][lane], sums[wave][3 * r + 2][lane]};
+        const std::size_t k = static_cast<std::size_t>(tile) * kTile + lane;
+        if (gridDim.y == 1) {
+            if (k >= out.n) continue;
+            const std::uint64_t dst = out.order != nullptr ? out.order[k] : k;
+            store_field(dst, out.G * a[0], out.G * a[1], out.G * a[2], out.ax, out.ay, out.az, out.kick);
+            continue;
+        }
+        // Component c of target k from block y at partial[(3 y + c) npad + k].
+        const std::size_t np = static_cast<std::size_t>(tiles) * kTile;
+        double* const to = partial + static_cast<std::size_t>(blockIdx.y) * 3 * np + k;
+        to[0] = a[0];
+        to[np] = a[1];
+        to[2 * np] = a[2];
+    }
+}
+
+// The blocks' FP64 sums of a target, in block order.
+__global__ __launch_bounds__(kTile) void direct_reduce(const double* __restrict__ partial,
+                                                       std::uint32_t blocks, std::uint32_t tiles,
+                                                       FieldOut out) {
+    const std::uint64_t k = static_cast<std::uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (k >= out.n) return;
+    const std::size_t np = static_cast<std::size_t>(tiles) * kTile;
+    double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+#pragma unroll 8
+    for (std::uint32_t s = 0; s < blocks; ++s) {
+        const double* p = partial + static_cast<std::size_t>(s) * 3 * np + k;
+        a0 += p[0];
+        a1 += p[np];
+        a2 += p[2 * np];
+    }
+    const std::uint64_t dst = out.order != nullptr ? out.order[k] : k;
+    store_field(dst, out.G * a0, out.G * a1, out.G * a2, out.ax, out.ay, out.az, out.kick);
 }
 
 // ---- batches: many independent systems in one launch ---------------------
@@ -924,7 +970,7 @@ __device__ __forceinline__ void pairs_item(const float4* __restrict__ packed,
                         float r2 = __builtin_fmaf(dx, dx, eps2);
                         r2 = __builtin_fmaf(dy, dy, r2);
                         r2 = __builtin_fmaf(dz, dz, r2);
-                        const bool near_pair = r2 < lim && r2 > 0.f;
+                        const bool near_pair = r2 < lim && (!kSafe || r2 > 0.f);
                         close |= near_pair ? std::uint64_t{1} << step : std::uint64_t{0};
                         const float inv3 = near_pair ? 0.f : inv_cubed<kSafe, kRefine>(r2);
                         const float fj = kEqual ? inv3 : mi * inv3, fi = kEqual ? inv3 : mr * inv3;
@@ -954,6 +1000,9 @@ __device__ __forceinline__ void pairs_item(const float4* __restrict__ packed,
                 }
                 // Close pairs: at step s this lane met streamed particle
                 // (lane - s) mod 64, read back here by index.
+                const double ah[3] = {static_cast<double>(th[0]) + static_cast<double>(tl[0]),
+                                      static_cast<double>(th[1]) + static_cast<double>(tl[1]),
+                                      static_cast<double>(th[2]) + static_cast<double>(tl[2])};
                 while (close != 0) {
                     const unsigned step = __builtin_ctzll(close);
                     close &= close - 1;
@@ -963,7 +1012,7 @@ __device__ __forceinline__ void pairs_item(const float4* __restrict__ packed,
                     const float4 bl4 = packed_lo[k];
                     const float bh[3] = {b.x, b.y, b.z}, bl[3] = {bl4.x, bl4.y, bl4.z};
                     double G[3];
-                    close_pair(th, tl, bh, bl, eps2, G);
+                    close_pair(ah, bh, bl, eps2, G);
                     const double mb = kEqual ? 1.0 : static_cast<double>(b.w);
                     const double ms = static_cast<double>(mr);
                     float h, l;
@@ -1115,31 +1164,18 @@ __global__ __launch_bounds__(256) void pairs_reduce(const float* __restrict__ jp
     store_field(dst, G * a0, G * a1, G * a2, ax, ay, az, kick);
 }
 
-template<int R, bool kSafe, bool kRefine, bool kMask>
-void launch_tiles(orr_ctx* ctx, std::uint32_t blocks_i, std::uint32_t splits, const float4* packed,
-                  const float4* packed_lo, const double4* centres, const float4* extents,
-                  const std::uint32_t* mask, std::uint32_t npad, std::uint32_t tiles,
-                  std::uint32_t per_split, float eps2, float* partials) {
-    hipLaunchKernelGGL((direct_tiles<R, kSafe, kRefine, kMask>), dim3(blocks_i, splits), dim3(kBlock), 0,
-                       ctx->stream, packed, packed_lo, centres, extents, mask, npad, tiles, per_split,
-                       eps2, partials);
+template<int R>
+void launch_fold(orr_ctx* ctx, bool safe, bool refine, dim3 grid, const float4* packed,
+                 const float4* packed_lo, const double4* centres, const float4* extents,
+                 std::uint32_t tiles, std::uint32_t per_group, std::uint32_t groups, float eps2,
+                 double* partial, const FieldOut& out) {
+    auto kernel = safe ? (refine ? direct_fold<R, true, true> : direct_fold<R, true, false>)
+                       : (refine ? direct_fold<R, false, true> : direct_fold<R, false, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, ctx->stream, packed, packed_lo, centres, extents, tiles, per_group, groups, eps2, partial, out);
+    ORR_LAUNCHED("direct_fold");
 }
 
-using TilesLauncher = void (*)(orr_ctx*, std::uint32_t, std::uint32_t, const float4*,
-                               const float4*, const double4*, const float4*, const std::uint32_t*,
-                               std::uint32_t, std::uint32_t, std::uint32_t, float, float*);
-
-template<int R, bool kMask> TilesLauncher pick_mask(bool safe, bool refine) {
-    if (safe) return refine ? launch_tiles<R, true, true, kMask> : launch_tiles<R, true, false, kMask>;
-    return refine ? launch_tiles<R, false, true, kMask> : launch_tiles<R, false, false, kMask>;
-}
-
-template<int R> TilesLauncher pick(bool safe, bool refine, bool mask) {
-    return mask ? pick_mask<R, true>(safe, refine) : pick_mask<R, false>(safe, refine);
-}
-
-// Pairs of tiles flagged by a mask up to this many tiles (a 128 MiB mask);
-// beyond it the kernels test each pair themselves.
+// The pairs path's mask of near tile pairs holds up to this many tiles (128 MiB).
 constexpr std::uint32_t kMaskTiles = 32768;
 
 // The pairs path: blocks of kStay tiles, chunks of S tiles per item, slot
@@ -1231,11 +1267,25 @@ namespace {
 // near mask and pairs plan, as direct_enqueue chooses them for the context's
 // configuration.
 struct DirectShape {
-    std::uint32_t tiles = 0, npad = 0, blocks_i = 0, splits = 0, per_split = 0, words = 0;
+    std::uint32_t tiles = 0, npad = 0, words = 0;
+    // One-sided: target tiles a wave, blocks of targets, source tiles a group
+    // (summed in FP32 with one compensation) and groups, blocks a target.
     int R = 1;
-    bool masked = false;
+    std::uint32_t blocks_i = 0, per_split = 0, splits = 0, blocks_j = 1;
+    bool masked = false;  // pairs: the near mask fits
     PairPlan plan;
 };
+
+// One-sided launch: blocks of four targets, kFoldWaves waves while every block
+// has a group. Near tiles make waves uneven, so many rounds of waves: kernel and
+// fold at N = 20,001 279 us at 8192 waves, 206 at 32,768, 204 at 65,536, 213 at
+// 131,072; at 32,768 745, 596, 554 and 567 us.
+constexpr std::uint32_t kFoldWaves = 65536;
+
+void one_sided_shape(DirectShape& d) {
+    const std::uint32_t waves = d.blocks_i * (kBlock / kTile);
+    d.blocks_j = std::max(1u, std::min((kFoldWaves + waves - 1) / waves, d.splits));
+}
 
 DirectShape direct_shape(const orr_ctx* ctx, std::uint64_t n) {
     if (n > (std::uint64_t{1} << 31)) fail(ORR_ERR_LENGTH, "direct: more than 2^31 particles");
@@ -1244,7 +1294,8 @@ DirectShape direct_shape(const orr_ctx* ctx, std::uint64_t n) {
     d.npad = d.tiles * kTile;
     d.R = ctx->direct_targets_per_lane;
     d.blocks_i = (d.npad + kBlock * d.R - 1) / (kBlock * d.R);
-    // Enough blocks to fill 256 CUs several times over; each split keeps >= 1 tile.
+    // Source tiles summed together in FP32: `block_target` blocks of four target
+    // tiles times groups, each group at least one tile.
     const std::uint32_t want = ctx->direct_block_target;
     std::uint32_t splits = std::max<std::uint32_t>(1, (want + d.blocks_i - 1) / d.blocks_i);
     splits = std::min(splits, d.tiles);
@@ -1253,6 +1304,7 @@ DirectShape direct_shape(const orr_ctx* ctx, std::uint64_t n) {
     d.masked = d.tiles <= kMaskTiles;
     d.words = (d.tiles + 31) / 32;
     d.plan = pair_plan(d.tiles, d.masked, ctx->direct_pair_mode);
+    one_sided_shape(d);
     return d;
 }
 
@@ -1260,7 +1312,7 @@ DirectShape direct_shape(const orr_ctx* ctx, std::uint64_t n) {
 struct DirectBuffers {
     float4* packed = nullptr;     // [npad] {o, m}, then [npad] residuals
     double4* centres = nullptr;   // [tiles], then extents [tiles], mass ranges [tiles], uniform
-    float* partials = nullptr;    // one-sided: [splits][6][npad]; pairs: slots
+    void* partials = nullptr;     // one-sided: FP64 [blocks_j][3][npad]; pairs: slots
     std::uint32_t* mask = nullptr;  // [tiles][words] when masked
 };
 
@@ -1272,10 +1324,10 @@ std::size_t partial_buffer_bytes(const DirectShape& d) {
     const std::size_t cpart_floats = 6 * static_cast<std::size_t>(d.npad);
     return d.plan.use ? sizeof(double) * d.plan.ipart_doubles +
                             sizeof(float) * (d.plan.jpart_floats + cpart_floats)
-                      : sizeof(float) * 6 * static_cast<std::size_t>(d.npad) * d.splits;
+                      : (d.blocks_j > 1 ? sizeof(double) * 3 * static_cast<std::size_t>(d.npad) * d.blocks_j : 0);
 }
 std::size_t mask_buffer_bytes(const DirectShape& d) {
-    return d.masked ? sizeof(std::uint32_t) * static_cast<std::size_t>(d.words) * d.tiles : 0;
+    return d.plan.use ? sizeof(std::uint32_t) * static_cast<std::size_t>(d.words) * d.tiles : 0;
 }
 
 // Every launch of one evaluation on given buffers; phases timed when `timed`.
@@ -1291,8 +1343,7 @@ void direct_launch(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* 
     float4* extents = reinterpret_cast<float4*>(centres + tiles);
     float2* mass_range = reinterpret_cast<float2*>(extents + tiles);
     float* uniform = reinterpret_cast<float*>(mass_range + tiles);
-    float* partials = buf.partials;
-    std::uint32_t* mask = d.masked ? buf.mask : nullptr;
+    std::uint32_t* mask = buf.mask;
     {
         PhaseTimer t(ctx, kDirectPrepare, timed);
         hipLaunchKernelGGL(direct_prepare, dim3(tiles), dim3(kTile), 0, ctx->stream, a.x, a.y, a.z,
@@ -1302,8 +1353,6 @@ void direct_launch(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* 
             hipLaunchKernelGGL(mass_uniform, dim3(1), dim3(256), 0, ctx->stream, mass_range, tiles,
                                ctx->direct_equal_masses == 1 ? 1 : 0, uniform);
             ORR_LAUNCHED("mass_uniform");
-        }
-        if (d.masked) {
             hipLaunchKernelGGL(near_mask, dim3((tiles + kMaskRows - 1) / kMaskRows), dim3(256), 0,
                                ctx->stream, centres, extents, tiles, words, mask);
             ORR_LAUNCHED("near_mask");
@@ -1314,7 +1363,7 @@ void direct_launch(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* 
     const bool refine = ctx->direct_refine != 0;
     if (plan.use) {
         // Doubles first: every part stays aligned to its type.
-        double* ipart = reinterpret_cast<double*>(partials);
+        double* ipart = static_cast<double*>(buf.partials);
         float* jpart = reinterpret_cast<float*>(ipart + plan.ipart_doubles);
         float* cpart = jpart + plan.jpart_floats;
         {
@@ -1334,20 +1383,26 @@ void direct_launch(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* 
         }
         return;
     }
+    FieldOut out;
+    out.n = n;
+    out.order = order;
+    out.G = a.gravitational_constant;
+    out.ax = a.ax;
+    out.ay = a.ay;
+    out.az = a.az;
+    out.kick = kick;
+    double* const partial = static_cast<double*>(buf.partials);
     {
         PhaseTimer t(ctx, kDirectKernel, timed);
-        TilesLauncher launch = d.R == 1 ? pick<1>(safe, refine, d.masked)
-                             : d.R == 4 ? pick<4>(safe, refine, d.masked)
-                                        : pick<2>(safe, refine, d.masked);
-        launch(ctx, d.blocks_i, d.splits, packed, packed_lo, centres, extents, mask, npad, tiles,
-               d.per_split, eps2, partials);
-        ORR_LAUNCHED("direct_tiles");
+        const dim3 grid(d.blocks_i, d.blocks_j);
+        auto launch = d.R == 1 ? launch_fold<1> : d.R == 2 ? launch_fold<2> : launch_fold<4>;
+        launch(ctx, safe, refine, grid, packed, packed_lo, centres, extents, tiles, d.per_split, d.splits,
+               eps2, partial, out);
     }
-    {
+    if (d.blocks_j > 1) {
         PhaseTimer t(ctx, kDirectReduce, timed);
-        const std::uint32_t blocks = static_cast<std::uint32_t>((n + 255) / 256);
-        hipLaunchKernelGGL(direct_reduce, dim3(blocks), dim3(256), 0, ctx->stream, partials, d.splits,
-                           npad, n, order, a.gravitational_constant, a.ax, a.ay, a.az, kick);
+        hipLaunchKernelGGL(direct_reduce, dim3(tiles), dim3(kTile), 0, ctx->stream, partial, d.blocks_j,
+                           tiles, out);
         ORR_LAUNCHED("direct_reduce");
     }
 }
@@ -1361,12 +1416,12 @@ void direct_enqueue(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t*
     ctx->direct_packed.reserve(packed_buffer_bytes(d));
     ctx->direct_centres.reserve(centre_buffer_bytes(d));
     ctx->direct_partials.reserve(partial_buffer_bytes(d));
-    if (d.masked) ctx->direct_near.reserve(mask_buffer_bytes(d));
+    ctx->direct_near.reserve(mask_buffer_bytes(d));
     DirectBuffers buf;
     buf.packed = ctx->direct_packed.as<float4>();
     buf.centres = ctx->direct_centres.as<double4>();
-    buf.partials = ctx->direct_partials.as<float>();
-    buf.mask = d.masked ? ctx->direct_near.as<std::uint32_t>() : nullptr;
+    buf.partials = ctx->direct_partials.ptr;
+    buf.mask = ctx->direct_near.as<std::uint32_t>();
     direct_launch(ctx, a, order, d, buf, true, kick);
 }
 
@@ -1524,8 +1579,11 @@ void direct_evaluate_static(orr_ctx* ctx, const orr_direct_args& a) {
     d.plan = PairPlan{};  // the one-sided kernel
     const bool ordered = a.spatial_order != 0 && n > 64;
     const OrderSizes oz = order_sizes(n, 1, 0, false);
+    // What the groups of source tiles are sized by: room beside the other
+    // buffers for one FP32 sum and compensation a target and group (and a mask),
+    // more than the FP64 sums of a block need.
     const std::size_t fixed = aligned(packed_buffer_bytes(d)) + aligned(centre_buffer_bytes(d)) +
-                              aligned(mask_buffer_bytes(d)) +
+                              aligned(sizeof(std::uint32_t) * static_cast<std::size_t>(d.words) * d.tiles) +
                               (ordered ? aligned(oz.bbox) + 2 * aligned(oz.codes) +
                                              2 * aligned(oz.index) + aligned(oz.hist)
                                        : 0);
@@ -1538,11 +1596,11 @@ void direct_evaluate_static(orr_ctx* ctx, const orr_direct_args& a) {
         d.per_split = (d.tiles + fit - 1) / fit;
         d.splits = (d.tiles + d.per_split - 1) / d.per_split;
     }
+    one_sided_shape(d);
     Carver c{static_cast<unsigned char*>(scratch_on(ctx->device))};
     DirectBuffers buf;
     buf.packed = c.take<float4>(packed_buffer_bytes(d));
     buf.centres = c.take<double4>(centre_buffer_bytes(d));
-    buf.mask = d.masked ? c.take<std::uint32_t>(mask_buffer_bytes(d)) : nullptr;
     const std::uint32_t* order = nullptr;
     if (ordered) {
         OrderScratch ob;
@@ -1556,7 +1614,7 @@ void direct_evaluate_static(orr_ctx* ctx, const orr_direct_args& a) {
         const int cur = morton_enqueue_into(ctx, a.x, a.y, a.z, n, SegmentView{}, nullptr, 4, ob, false);
         order = ob.index[cur];
     }
-    buf.partials = c.take<float>(split_bytes * d.splits);
+    buf.partials = c.take<double>(partial_buffer_bytes(d));
     if (c.used > kStaticScratchBytes) fail(ORR_ERR_RUNTIME, "direct (static scratch): layout overflow");
     direct_launch(ctx, a, order, d, buf, false);
 }

@@ -485,3 +485,30 @@ def test_equal_mass_form_against_fp64_reference(ctx, n, mass):
     assert oracle.error_summary(rel)[0] < 2e-7
     if n % 64:
         assert all(np.array_equal(a, b) for a, b in zip(out[1], out[2]))
+
+
+@pytest.mark.parametrize("targets,block_target", [(1, 32768), (1, 3), (2, 64), (4, 8)])
+@pytest.mark.parametrize("eps", [0.0, 0.02])
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 129, 255, 256, 257, 1025])
+def test_one_sided_groups_and_blocks(ctx, n, eps, targets, block_target):
+    """One-sided sums at the edges of tiles, of blocks of four targets and of groups of
+    source tiles (one tile a group, or all in few). A term is off by at most its FP32
+    roundings (separation, square, cube, root, product: under 8 of 2^-24), so a sum by
+    that share of the sum of the terms' sizes."""
+    p = oracle.plummer(n, 40 + n)
+    x = np.stack([p.x, p.y, p.z])
+    d = x[:, None, :] - x[:, :, None]
+    r2 = (d**2).sum(0) + eps * eps
+    np.fill_diagonal(r2, np.inf)
+    t = d * (p.m * r2**-1.5)
+    default = ctx.direct_config()
+    try:
+        ctx.set_direct_config(targets_per_lane=targets, block_target=block_target, pair_mode=2)
+        s = E.HipDirectSolver(E.Softening(eps), context=ctx)
+        a = [np.zeros(n) for _ in range(3)]
+        s.evaluate((p.x, p.y, p.z), p.m, a)
+    finally:
+        ctx.set_direct_config(targets_per_lane=default["targets_per_lane"],
+                              block_target=default["block_target"], pair_mode=default["pair_mode"])
+    off = np.linalg.norm(np.stack(a) - t.sum(2), axis=0)
+    assert (off <= 8 * 2.0**-24 * np.linalg.norm(t, axis=0).sum(1)).all()
