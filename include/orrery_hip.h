@@ -143,8 +143,9 @@ ORR_API int orr_direct_static_limits(uint64_t* max_count, uint64_t* scratch_byte
  * pairs path take its equal-mass form when every particle has one mass (the
  * mass leaves the pair term and multiplies the folded sums: two multiplies
  * fewer per pair; the same bits when that mass is a power of two), 2 never.
- * small_order 1 (default) orders a system of at most 4096 particles in one
- * workgroup (one launch instead of some twenty; the same permutation, so the
+ * small_order 1 (default) orders a system of at most 20,480 particles by
+ * counting each key's rank (one launch up to 4096 particles, four above, instead
+ * of a launch per radix pass; the same permutation, so the
  * same bits), 2 never. targets_per_lane 0, refine -1, block_target 0,
  * pair_mode 0, equal_masses 0 and small_order 0 keep the current value. */
 typedef struct {

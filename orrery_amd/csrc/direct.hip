@@ -233,7 +233,10 @@ __device__ __forceinline__ void kahan_df(float h, float l, float& s, float& c) {
 //     FP64 and added to it as (hi, lo); the tile's pair then joins (s, k).
 //
 // kUnroll sets how many far-path sources are in flight (their SGPR loads
-// included).
+// included). `sources` of the tile are particles and the rest massless pads at
+// its centre, and `live` says which targets are particles: pads lie on top of
+// one another, so the near path leaves them out -- their zero terms change no
+// sum, and as close pairs they would take up to 64 FP64 evaluations a lane.
 constexpr int kRun = 16;
 // Terms of a near tile summed plainly in FP32 before each Kahan addition.
 constexpr int kNearRun = 8;
@@ -242,8 +245,8 @@ template<int R, bool kSafe, bool kRefine, bool kGivenNear = false, int kUnroll =
 __device__ __forceinline__ void source_tile(
     const float4* __restrict__ packed, const float4* __restrict__ packed_lo,
     const double4* __restrict__ centres, const float4* __restrict__ extents, std::uint32_t J,
-    bool given_near, float eps2, const float (&ox)[R], const float (&oy)[R], const float (&oz)[R],
-    const float (&lx)[R], const float (&ly)[R], const float (&lz)[R], const double (&cx)[R],
+    bool given_near, std::uint32_t sources, const bool (&live)[R], float eps2,
+    const float (&ox)[R], const float (&oy)[R], const float (&oz)[R], const float (&lx)[R], const float (&ly)[R], const float (&lz)[R], const double (&cx)[R],
     const double (&cy)[R], const double (&cz)[R], const float4 (&ce)[R], float (&sx)[R],
     float (&sy)[R], float (&sz)[R], float (&kx)[R], float (&ky)[R], float (&kz)[R]) {
     const double4 C = centres[J];
@@ -306,11 +309,11 @@ __device__ __forceinline__ void source_tile(
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         px[r] = py[r] = pz[r] = pkx[r] = pky[r] = pkz[r] = 0.f;
-        lim[r] = close_limit(ce[r].w, E.w, eps2);
+        lim[r] = live[r] ? close_limit(ce[r].w, E.w, eps2) : -1.f;
         close[r][0] = close[r][1] = 0;
     }
 #pragma unroll 1
-    for (int j0 = 0; j0 < kTile; j0 += kNearRun) {
+    for (int j0 = 0; j0 < static_cast<int>(sources); j0 += kNearRun) {
         if (j0 == kTile / 2) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
@@ -351,15 +354,33 @@ __device__ __forceinline__ void source_tile(
             kahan(qz[r], pz[r], pkz[r]);
         }
     }
+    // What the pads' runs of zero terms would do: one addition of zero moves a
+    // compensation into its sum where it is large enough to show, more change
+    // nothing.
+    auto add_zero = [&](int r) {
+        kahan(0.f, px[r], pkx[r]);
+        kahan(0.f, py[r], pky[r]);
+        kahan(0.f, pz[r], pkz[r]);
+    };
+    if (sources + kNearRun <= kTile) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) add_zero(r);
+    }
     // The close pairs, each lane over its own (few): sources read by index.
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const double t[3] = {static_cast<double>(th[r][0]) + static_cast<double>(tl[r][0]),
                              static_cast<double>(th[r][1]) + static_cast<double>(tl[r][1]),
                              static_cast<double>(th[r][2]) + static_cast<double>(tl[r][2])};
-        std::uint64_t bits = static_cast<std::uint64_t>(close[r][0]) << 32 | close[r][1];
+        // The first source to the highest bit (the runs taken fill `taken` bits,
+        // the last 32 of them or fewer in close[1]), and no pads.
+        const std::uint32_t taken = (sources + kNearRun - 1) / kNearRun * kNearRun;
+        std::uint64_t bits = static_cast<std::uint64_t>(close[r][0]) << 32 |
+                             static_cast<std::uint64_t>(close[r][1]) << (taken > 32 ? 64 - taken : 32 - taken);
+        if (taken <= 32) bits <<= 32;
+        bits &= ~std::uint64_t{0} << (kTile - sources);
         while (bits != 0) {
-            const int j = __builtin_clzll(bits);  // the first source is the highest bit
+            const int j = __builtin_clzll(bits);
             bits &= ~(std::uint64_t{1} << (63 - j));
             const float4 q = src[j];
             const float4 ql = src_lo[j];
@@ -374,6 +395,12 @@ __device__ __forceinline__ void source_tile(
             kahan_df(h, l, py[r], pky[r]);
             split(mq * G[2], h, l);
             kahan_df(h, l, pz[r], pkz[r]);
+        }
+        if (sources < kTile) {
+            // The pads, at the tile's centre, are close pairs or none of them is.
+            const float dx = -th[r][0] - tl[r][0], dy = -th[r][1] - tl[r][1], dz = -th[r][2] - tl[r][2];
+            const float r2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, eps2)));
+            if (r2 < lim[r] && (!kSafe || r2 > 0.f)) add_zero(r);
         }
     }
 #pragma unroll
@@ -477,9 +504,11 @@ __global__ __launch_bounds__(kBlock) void direct_fold(
     float ox[R], oy[R], oz[R], lx[R], ly[R], lz[R];
     double cx[R], cy[R], cz[R];
     float4 ce[R];
+    bool live[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const std::uint32_t tile = min(target_tile(r), tiles - 1);
+        live[r] = static_cast<std::uint64_t>(tile) * kTile + lane < out.n;
         const float4 o = packed[static_cast<std::size_t>(tile) * kTile + lane];
         const float4 l = packed_lo[static_cast<std::size_t>(tile) * kTile + lane];
         const double4 c = centres[tile];
@@ -499,6 +528,7 @@ __global__ __launch_bounds__(kBlock) void direct_fold(
 #pragma unroll
     for (int c = 0; c < 3 * R; ++c) sums[wave][c][lane] = 0.0;
     const std::uint32_t stride = gridDim.y;
+    const std::uint32_t last = static_cast<std::uint32_t>(out.n - (static_cast<std::uint64_t>(tiles) - 1) * kTile);
     std::uint32_t met = 0;        // source tiles taken so far
     std::uint64_t near_bits = 0;  // of the 64 from met & ~63
     for (std::uint32_t g = blockIdx.y; g < groups; g += stride) {
@@ -518,7 +548,9 @@ __global__ __launch_bounds__(kBlock) void direct_fold(
                 near_bits = __ballot(valid && near);
             }
             const bool near = ((near_bits >> (met % 64)) & 1u) != 0;
-            source_tile<R, kSafe, kRefine, true>(packed, packed_lo, centres, extents, g * per_group + o, near,
+            const std::uint32_t J = g * per_group + o;
+            const std::uint32_t sources = J + 1 < tiles ? kTile : last;
+            source_tile<R, kSafe, kRefine, true>(packed, packed_lo, centres, extents, J, near, sources, live,
                                                  eps2, ox, oy, oz, lx, ly, lz, cx, cy, cz, ce, sx, sy, sz, kx,
                                                  ky, kz);
         }
@@ -623,7 +655,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
     const std::uint32_t first = __builtin_amdgcn_readfirstlane(blockIdx.x * (kBlock / kTile) + threadIdx.x / kTile);
     for (std::uint32_t next = first; next < items; next += waves) {
         const uint4 it = item[next];
-        const float eps2 = eps2_of[tile[it.x].z];
+        const uint4 own = tile[it.x];
+        const float eps2 = eps2_of[own.z];
+        const bool live[1] = {lane < own.y};
         const std::uint32_t k = it.x * kTile + lane;
         const float4 o = packed[k];
         const float4 l = packed_lo[k];
@@ -635,7 +669,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         float sx[1] = {0.f}, sy[1] = {0.f}, sz[1] = {0.f}, kx[1] = {0.f}, ky[1] = {0.f},
               kz[1] = {0.f};
         for (std::uint32_t J = it.y; J < it.z; ++J)
-            source_tile<1, kSafe, kRefine, false, kItemUnroll>(packed, packed_lo, centres, extents, J, false, eps2,
+            source_tile<1, kSafe, kRefine, false, kItemUnroll>(packed, packed_lo, centres, extents, J, false,
+                                                        tile[J].y, live, eps2,
                                                         ox, oy, oz, lx, ly, lz, cx, cy, cz, ce, sx,
                                                         sy, sz, kx, ky, kz);
         float* out = partial + static_cast<std::size_t>(it.w) * 6 * kTile;
@@ -1099,12 +1134,13 @@ __global__ __launch_bounds__(kBlock) void direct_complement(const float4* __rest
     const float lx[1] = {l.x}, ly[1] = {l.y}, lz[1] = {l.z};
     const double cx[1] = {c.x}, cy[1] = {c.y}, cz[1] = {c.z};
     const float4 ce[1] = {extents[t]};
+    const bool live[1] = {true};
     float sx[1] = {0.f}, sy[1] = {0.f}, sz[1] = {0.f}, kx[1] = {0.f}, ky[1] = {0.f}, kz[1] = {0.f};
     const std::uint32_t* row = mask + static_cast<std::size_t>(t) * words;
     const std::uint32_t b0 = t / kStay * kStay, b1 = min(b0 + kStay, tiles);
     for (std::uint32_t J = b0; J < b1; ++J) {
         const bool near = ((row[J / 32] >> (J & 31u)) & 1u) != 0;
-        source_tile<1, kSafe, kRefine, true>(packed, packed_lo, centres, extents, J, near, eps2, ox,
+        source_tile<1, kSafe, kRefine, true>(packed, packed_lo, centres, extents, J, near, kTile, live, eps2, ox,
                                              oy, oz, lx, ly, lz, cx, cy, cz, ce, sx, sy, sz, kx, ky, kz);
     }
     const std::size_t np = static_cast<std::size_t>(tiles) * kTile;
@@ -1437,30 +1473,63 @@ std::size_t direct_batch_bytes(std::uint64_t tiles, std::uint64_t slots) {
 
 void direct_evaluate(orr_ctx* ctx, const orr_direct_args& a, const FusedKick& kick) {
     if (a.count == 0) return;
-    const std::uint32_t* order = nullptr;
-    if (a.spatial_order != 0 && a.count > 64) {
-        // The Morton order is some nine short launches: replayed as a graph (its
-        // phases untimed); the three direct launches stay eager and timed.
-        std::vector<unsigned char> key;
-        key_add(key, a.x);
-        key_add(key, a.y);
-        key_add(key, a.z);
-        key_add(key, a.count);
-        // Compact tiles need only the top 32 bits of the 63-bit codes: the four
-        // upper radix passes of eight, or for a small system the same order
-        // from one workgroup.
-        const bool small = ctx->direct_small_order == 1 && a.count <= kSmallOrder;
-        key_add(key, small);
-        run_captured(ctx, ctx->direct_graph, std::move(key), [&] {
-            if (small) {
-                morton_enqueue_small(ctx, a.x, a.y, a.z, a.count, 4);
-            } else {
-                morton_enqueue(ctx, a.x, a.y, a.z, a.count, 4);
-            }
-        }, true);
-        order = ctx->order_index.as<std::uint32_t>();
+    const bool ordered = a.spatial_order != 0 && a.count > 64;
+    // Compact tiles need only the top 32 bits of the 63-bit codes: the four
+    // upper radix passes of eight, or for a small system the same order by
+    // counting ranks.
+    const bool small = ctx->direct_small_order == 1 && a.count <= kRankOrder;
+    auto enqueue_order = [&] {
+        if (small) {
+            morton_enqueue_small(ctx, a.x, a.y, a.z, a.count);
+        } else {
+            morton_enqueue(ctx, a.x, a.y, a.z, a.count, 4);
+        }
+    };
+    auto order = [&]() -> const std::uint32_t* {
+        return ordered ? ctx->order_index.as<std::uint32_t>() : nullptr;
+    };
+    std::vector<unsigned char> key;
+    key_add(key, a.x);
+    key_add(key, a.y);
+    key_add(key, a.z);
+    key_add(key, a.count);
+    key_add(key, small);
+    if (ctx->timing) {
+        // The order's short launches as one replayed graph, untimed; the direct
+        // launches eager and timed.
+        if (ordered) run_captured(ctx, ctx->direct_graph, std::move(key), enqueue_order, true);
+        direct_enqueue(ctx, a, order(), kick);
+        return;
     }
-    direct_enqueue(ctx, a, order, kick);
+    // A small system's launches outrun the host: the whole evaluation as one
+    // graph (N = 1000: 56 us, 66 with the order alone as a graph). Without an
+    // order there are two launches, cheaper than a graph; beyond kSmallOrder
+    // the launches are long enough for the host to stay ahead of them.
+    if (!ordered || a.count > kSmallOrder) {
+        if (ordered) enqueue_order();
+        direct_enqueue(ctx, a, order(), kick);
+        return;
+    }
+    key_add(key, a.m);
+    key_add(key, a.ax);
+    key_add(key, a.ay);
+    key_add(key, a.az);
+    key_add(key, a.softening_squared);
+    key_add(key, a.gravitational_constant);
+    key_add(key, ordered);
+    key_add(key, kick.vx);
+    key_add(key, kick.vy);
+    key_add(key, kick.vz);
+    key_add(key, kick.s);
+    key_add(key, ctx->direct_targets_per_lane);
+    key_add(key, ctx->direct_refine);
+    key_add(key, ctx->direct_block_target);
+    key_add(key, ctx->direct_pair_mode);
+    key_add(key, ctx->direct_equal_masses);
+    run_captured(ctx, ctx->direct_graph, std::move(key), [&] {
+        if (ordered) enqueue_order();
+        direct_enqueue(ctx, a, order(), kick);
+    });
 }
 
 void direct_batch_enqueue(orr_ctx* ctx, const double* x, const double* y, const double* z,

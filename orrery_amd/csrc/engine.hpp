@@ -132,7 +132,7 @@ struct orr_ctx {
     int direct_pair_mode = 1;
     // 1: the pairs path's equal-mass form where the masses allow it, 2: never.
     int direct_equal_masses = 1;
-    int direct_small_order = 1;  // 1: one-workgroup ordering up to kSmallOrder particles, 2: never
+    int direct_small_order = 1;  // 1: ordering by rank up to kRankOrder particles, 2: never
     int sort_mode = 1;  // Morton sort: 1 one-sweep passes, 2 histogram + scan + scatter per pass
     // Barnes-Hut walk configuration (orr_ctx_set_tree_config); 0 chooses by size.
     int walk_targets_per_lane = 0;
@@ -354,11 +354,16 @@ std::size_t ctx_device_bytes(const orr_ctx* ctx);
 // code's top bits only (stable within equal tops), enough for compact tiles.
 void morton_enqueue(orr_ctx* ctx, const double* x, const double* y, const double* z,
                     std::uint64_t n, int first_digit = 0);
-// morton_enqueue's index (and cube) for n <= kSmallOrder and first_digit >= 4 in
-// one launch: the same permutation; ctx->order_codes is left as it was.
+// morton_enqueue's index (and cube) by the codes' top 32 bits (first_digit 4)
+// for n <= kRankOrder, by counting each key's rank: one launch up to
+// kSmallOrder, four up to kRankOrder; the same permutation. ctx->order_codes
+// holds no 64-bit codes afterwards.
 constexpr std::uint64_t kSmallOrder = 4096;
+// Order and launch gaps, rank counting against radix passes: 33 against 66 us at
+// 8192 particles, 48 / 81 at 16,384, 65 / 79 at 20,001, 95 / 83 at 24,576.
+constexpr std::uint64_t kRankOrder = 20480;
 void morton_enqueue_small(orr_ctx* ctx, const double* x, const double* y, const double* z,
-                          std::uint64_t n, int first_digit);
+                          std::uint64_t n);
 // Copies the cube {origin, size} computed by the last morton_enqueue (syncs).
 void morton_cube(orr_ctx* ctx, double cube[4]);
 

@@ -607,43 +607,104 @@ __global__ __launch_bounds__(kBlock) void radix_onesweep(const std::uint64_t* __
     }
 }
 
-// Small systems in one workgroup: extrema, cube, codes and the order by the
-// codes' digits from first_digit up, instead of nine short launches.
-// The multi-kernel order is a stable sort by those digits, that is a sort by
-// (code >> 8 first_digit, index), a key unique per element; a bitonic network
-// over the packed keys sorts them to the same permutation. first_digit >= 4
-// keeps the digits within 32 bits beside the 32-bit index.
-constexpr int kSmallThreads = 1024;
-constexpr int kSmallSlots = static_cast<int>(kSmallOrder) / kSmallThreads;  // keys per thread
-// Positions: 6 lane bits, 2 slot bits, 4 wave bits.
-static_assert(kSmallOrder == 4096 && kSmallThreads == 1024 && kSmallSlots == 4, "small-sort layout");
+// ---- small systems: order by rank ------------------------------------------------
+//
+// The multi-kernel order is a stable sort by the codes' digits from first_digit
+// up, that is a sort by (code >> 8 first_digit, index): a key unique per
+// element, whose position is the number of smaller keys. Counting them is n^2
+// compares, 32 bits wide where first_digit >= 4, with no dependence between
+// passes: 20 us at 16,384 keys against some 65 us of radix launches, each bound
+// by its own latency. A wave ranks kRankKeys keys of its own against all codes
+// in LDS, 64 a step: every lane counts the codes of its stride that lie before
+// the key, and the lanes' counts are added.
+constexpr int kRankThreads = 1024;
+constexpr int kRankWaves = kRankThreads / 64;
 
-// Compare-exchange of a key with its partner's: the smaller one where this
-// position keeps the minimum, else the larger.
-__device__ __forceinline__ unsigned long long keep(unsigned long long mine, unsigned long long other,
-                                                   bool keep_min) {
-    const bool other_less = other < mine;
-    return other_less == keep_min ? other : mine;
+// Before key i, code c: codes equal to c at a lower index, or lower codes. The
+// 64 codes from j0 are all before i's 64, all after, or its own.
+__device__ __forceinline__ std::uint32_t wave_total(std::uint32_t v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
 }
 
-__global__ __launch_bounds__(kSmallThreads) void morton_small(const double* __restrict__ x,
-                                                              const double* __restrict__ y,
-                                                              const double* __restrict__ z,
-                                                              std::uint32_t n, int first_digit,
-                                                              double* __restrict__ cube_out,
-                                                              std::uint32_t* __restrict__ index) {
-    __shared__ unsigned long long keys[kSmallOrder];
-    __shared__ double wave_ext[kSmallThreads / 64][6];
+// codes: n of them in LDS, the last 64 filled up with ~0 (a code's top bit is
+// clear). Writes index[rank of i] = i for the wave's keys first .. first + kKeys - 1.
+template<int kKeys>
+__device__ void rank_keys(const std::uint32_t* codes, std::uint32_t n, std::uint32_t first,
+                          std::uint32_t* __restrict__ index) {
+    const std::uint32_t lane = threadIdx.x & 63;
+    std::uint32_t key[kKeys], count[kKeys];
+#pragma unroll
+    for (int k = 0; k < kKeys; ++k) {
+        key[k] = codes[min(first + k, n - 1)];
+        count[k] = 0;
+    }
+    // The wave's keys lie in one run of 64: first is a multiple of kKeys, a power of two.
+    const std::uint32_t own = first & ~63u, padded = (n + 63) & ~63u;
+    for (std::uint32_t j = 0; j < own; j += 64) {
+        const std::uint32_t c = codes[j + lane];
+#pragma unroll
+        for (int k = 0; k < kKeys; ++k) count[k] += c <= key[k] ? 1u : 0u;
+    }
+    {
+        const std::uint32_t c = codes[own + lane];
+#pragma unroll
+        for (int k = 0; k < kKeys; ++k) {
+            count[k] += c < key[k] || (c == key[k] && own + lane < first + k) ? 1u : 0u;
+        }
+    }
+    for (std::uint32_t j = own + 64; j < padded; j += 64) {
+        const std::uint32_t c = codes[j + lane];
+#pragma unroll
+        for (int k = 0; k < kKeys; ++k) count[k] += c < key[k] ? 1u : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < kKeys; ++k) {
+        const std::uint32_t rank = wave_total(count[k]);
+        if (lane == 0 && first + k < n) index[rank] = first + k;
+    }
+}
+
+// The 32 bits of a position's code from digit 4 up, as encode computes them.
+__device__ __forceinline__ std::uint32_t top_code(double px, double py, double pz, const double* cube,
+                                                  double scale) {
+    if (!(cube[3] > 0)) return 0;
+    const std::uint64_t code = (spread_bits(to_grid(px, cube[0], scale)) << 2) |
+                               (spread_bits(to_grid(py, cube[1], scale)) << 1) |
+                               spread_bits(to_grid(pz, cube[2], scale));
+    return static_cast<std::uint32_t>(code >> 32);
+}
+
+// Up to kSmallOrder particles in one launch: every block finds the extrema, the
+// cube and all codes itself (a few positions a thread), then ranks a key a wave.
+__global__ __launch_bounds__(kRankThreads) void morton_small(const double* __restrict__ x,
+                                                             const double* __restrict__ y,
+                                                             const double* __restrict__ z,
+                                                             std::uint32_t n, double* __restrict__ cube_out,
+                                                             std::uint32_t* __restrict__ index) {
+    constexpr int kSlots = static_cast<int>(kSmallOrder) / kRankThreads;
+    __shared__ std::uint32_t codes[kSmallOrder];
+    __shared__ double wave_ext[kRankWaves][6];
     __shared__ double cube[4];
     const std::uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const double inf = __builtin_huge_val();
     double e[6] = {inf, inf, inf, -inf, -inf, -inf};
-    for (std::uint32_t i = t; i < n; i += kSmallThreads) {
-        const double v[3] = {x[i], y[i], z[i]};
+    double v[kSlots][3];
+#pragma unroll
+    for (int r = 0; r < kSlots; ++r) {
+        const std::uint32_t i = t + r * kRankThreads;
+        const std::uint32_t from = i < n ? i : 0;
+        v[r][0] = x[from];
+        v[r][1] = y[from];
+        v[r][2] = z[from];
+    }
+#pragma unroll
+    for (int r = 0; r < kSlots; ++r) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            e[c] = v[c] < e[c] ? v[c] : e[c];
-            e[3 + c] = v[c] > e[3 + c] ? v[c] : e[3 + c];
+            e[c] = v[r][c] < e[c] ? v[r][c] : e[c];
+            e[3 + c] = v[r][c] > e[3 + c] ? v[r][c] : e[3 + c];
         }
     }
     // Extrema are exact, so folding them in any order gives the same values.
@@ -666,97 +727,50 @@ __global__ __launch_bounds__(kSmallThreads) void morton_small(const double* __re
         for (int c = 0; c < 3; ++c) {
             lo[c] = wave_ext[0][c];
             hi[c] = wave_ext[0][3 + c];
-            for (std::uint32_t w = 1; w < kSmallThreads / 64; ++w) {
+            for (int w = 1; w < kRankWaves; ++w) {
                 lo[c] = wave_ext[w][c] < lo[c] ? wave_ext[w][c] : lo[c];
                 hi[c] = wave_ext[w][3 + c] > hi[c] ? wave_ext[w][3 + c] : hi[c];
             }
         }
         make_cube(lo, hi, cube);
-        for (int c = 0; c < 4; ++c) cube_out[c] = cube[c];
+        if (blockIdx.x == 0) {
+            for (int c = 0; c < 4; ++c) cube_out[c] = cube[c];
+        }
     }
     __syncthreads();
-    // Codes as encode computes them, packed (top digits, index); padding last.
-    // Thread t holds the positions whose bits 0-5 are its lane, 6-7 the slot
-    // r and 8-11 its wave: bit b of a position is exchanged in 12 - b stages,
-    // so the low bits, the busiest, stay in the wave or the thread.
-    auto pos = [&](int r) { return lane | (static_cast<std::uint32_t>(r) << 6) | (wave << 8); };
-    const double size = cube[3];
-    const double scale = static_cast<double>(kGrid) / size;
-    const int shift = 8 * first_digit;
-    unsigned long long v[kSmallSlots];
+    const double scale = static_cast<double>(kGrid) / cube[3];
 #pragma unroll
-    for (int r = 0; r < kSmallSlots; ++r) {
-        const std::uint32_t i = pos(r);
-        unsigned long long key = ~0ull;
-        if (i < n) {
-            std::uint64_t code = 0;
-            if (size > 0) {
-                code = (spread_bits(to_grid(x[i], cube[0], scale)) << 2) |
-                       (spread_bits(to_grid(y[i], cube[1], scale)) << 1) |
-                       spread_bits(to_grid(z[i], cube[2], scale));
-            }
-            key = ((code >> shift) << 32) | i;
-        }
-        v[r] = key;
+    for (int r = 0; r < kSlots; ++r) {
+        const std::uint32_t i = t + r * kRankThreads;
+        codes[i] = i < n ? top_code(v[r][0], v[r][1], v[r][2], cube, scale) : ~0u;
     }
-    // Bitonic sort, ascending, of all kSmallOrder positions: partners 256 or
-    // more apart (another wave) through LDS, 64 or 128 apart in the same
-    // thread, under 64 apart by wave shuffles.
-    for (std::uint32_t k = 2; k <= kSmallOrder; k <<= 1) {
-        std::uint32_t j = k >> 1;
-        if (j >= 256) {
-            __syncthreads();  // the last round's reads of keys are done
-#pragma unroll
-            for (int r = 0; r < kSmallSlots; ++r) keys[pos(r)] = v[r];
-            __syncthreads();
-            for (; j >= 256; j >>= 1) {
-#pragma unroll
-                for (int r = 0; r < kSmallSlots; ++r) {
-                    const std::uint32_t i = pos(r);
-                    const std::uint32_t partner = i ^ j;
-                    if (partner > i) {
-                        const unsigned long long a = keys[i], b = keys[partner];
-                        const bool ascending = (i & k) == 0;
-                        if ((a > b) == ascending) {
-                            keys[i] = b;
-                            keys[partner] = a;
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-#pragma unroll
-            for (int r = 0; r < kSmallSlots; ++r) v[r] = keys[pos(r)];
-        }
-        for (; j >= 64; j >>= 1) {
-            const int jr = static_cast<int>(j >> 6);
-#pragma unroll
-            for (int r = 0; r < kSmallSlots; ++r) {
-                if ((r & jr) != 0) continue;
-                const std::uint32_t i = pos(r);
-                const bool ascending = (i & k) == 0;
-                const unsigned long long a = v[r], b = v[r | jr];
-                if ((a > b) == ascending) {
-                    v[r] = b;
-                    v[r | jr] = a;
-                }
-            }
-        }
-        for (; j > 0; j >>= 1) {
-#pragma unroll
-            for (int r = 0; r < kSmallSlots; ++r) {
-                const std::uint32_t i = pos(r);
-                const unsigned long long other = __shfl_xor(v[r], static_cast<int>(j), 64);
-                const bool keep_min = ((i & j) == 0) == ((i & k) == 0);
-                v[r] = keep(v[r], other, keep_min);
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < kSmallSlots; ++r) {
-        const std::uint32_t i = pos(r);
-        if (i < n) index[i] = static_cast<std::uint32_t>(v[r]);
-    }
+    __syncthreads();
+    rank_keys<1>(codes, n, blockIdx.x * kRankWaves + wave, index);
+}
+
+// Codes of a system too large for every block to compute them all.
+__global__ __launch_bounds__(kBlock) void encode_top(const double* __restrict__ x,
+                                                     const double* __restrict__ y,
+                                                     const double* __restrict__ z, std::uint32_t n,
+                                                     const double* __restrict__ cube,
+                                                     std::uint32_t* __restrict__ codes) {
+    const std::uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const double c[4] = {cube[0], cube[1], cube[2], cube[3]};
+    codes[i] = top_code(x[i], y[i], z[i], c, static_cast<double>(kGrid) / c[3]);
+}
+
+constexpr int kRankKeys = 4;  // keys a wave ranks together from the same reads
+
+__global__ __launch_bounds__(kRankThreads) void morton_rank(const std::uint32_t* __restrict__ in,
+                                                            std::uint32_t n,
+                                                            std::uint32_t* __restrict__ index) {
+    extern __shared__ std::uint32_t all_codes[];
+    const std::uint32_t padded = (n + 63) & ~63u;
+    for (std::uint32_t i = threadIdx.x; i < padded; i += kRankThreads) all_codes[i] = i < n ? in[i] : ~0u;
+    __syncthreads();
+    const std::uint32_t wave = blockIdx.x * kRankWaves + threadIdx.x / 64;
+    if (wave * kRankKeys < n) rank_keys<kRankKeys>(all_codes, n, wave * kRankKeys, index);
 }
 
 }  // namespace
@@ -925,17 +939,45 @@ int morton_enqueue_into(orr_ctx* ctx, const double* x, const double* y, const do
 }
 
 void morton_enqueue_small(orr_ctx* ctx, const double* x, const double* y, const double* z,
-                          std::uint64_t n, int first_digit) {
+                          std::uint64_t n) {
     if (n == 0) return;
-    if (n > kSmallOrder) fail(ORR_ERR_INVALID_ARGUMENT, "morton_enqueue_small: more than 4096 particles");
-    if (first_digit < 4) fail(ORR_ERR_INVALID_ARGUMENT, "morton_enqueue_small: first_digit must be at least 4");
-    ctx->order_bbox.reserve(4 * sizeof(double));
+    if (n > kRankOrder) fail(ORR_ERR_INVALID_ARGUMENT, "morton_enqueue_small: too many particles");
+    const std::uint32_t n32 = static_cast<std::uint32_t>(n);
     ctx->order_index.reserve(sizeof(std::uint32_t) * n);
+    if (n <= kSmallOrder) {
+        ctx->order_bbox.reserve(4 * sizeof(double));
+        PhaseTimer t(ctx, kSort);
+        hipLaunchKernelGGL(morton_small, dim3((n32 + kRankWaves - 1) / kRankWaves), dim3(kRankThreads), 0,
+                           ctx->stream, x, y, z, n32, ctx->order_bbox.as<double>(),
+                           ctx->order_index.as<std::uint32_t>());
+        ORR_LAUNCHED("morton_small");
+        return;
+    }
+    const OrderSizes sz = order_sizes(n, 1, 0, false);
+    ctx->order_bbox.reserve(sz.bbox);
+    ctx->order_codes.reserve(sz.codes);
+    double* cube = ctx->order_bbox.as<double>();
+    double* partial = cube + 4;
+    {
+        PhaseTimer t(ctx, kBbox);
+        hipLaunchKernelGGL(bbox_partial, dim3(sz.bbox_blocks), dim3(kBlock), 0, ctx->stream, x, y, z, n, partial);
+        ORR_LAUNCHED("bbox_partial");
+        hipLaunchKernelGGL(bbox_final, dim3(1), dim3(kBlock), 0, ctx->stream, partial, sz.bbox_blocks, cube);
+        ORR_LAUNCHED("bbox_final");
+    }
+    std::uint32_t* codes = ctx->order_codes.as<std::uint32_t>();
+    {
+        PhaseTimer t(ctx, kEncode);
+        hipLaunchKernelGGL(encode_top, dim3((n32 + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream, x, y, z,
+                           n32, cube, codes);
+        ORR_LAUNCHED("encode_top");
+    }
     PhaseTimer t(ctx, kSort);
-    hipLaunchKernelGGL(morton_small, dim3(1), dim3(kSmallThreads), 0, ctx->stream, x, y, z,
-                       static_cast<std::uint32_t>(n), first_digit, ctx->order_bbox.as<double>(),
+    constexpr std::uint32_t kPerBlock = kRankWaves * kRankKeys;
+    hipLaunchKernelGGL(morton_rank, dim3((n32 + kPerBlock - 1) / kPerBlock), dim3(kRankThreads),
+                       sizeof(std::uint32_t) * ((n32 + 63) & ~63u), ctx->stream, codes, n32,
                        ctx->order_index.as<std::uint32_t>());
-    ORR_LAUNCHED("morton_small");
+    ORR_LAUNCHED("morton_rank");
 }
 
 void morton_cube(orr_ctx* ctx, double cube[4]) {

@@ -512,3 +512,24 @@ def test_one_sided_groups_and_blocks(ctx, n, eps, targets, block_target):
                               block_target=default["block_target"], pair_mode=default["pair_mode"])
     off = np.linalg.norm(np.stack(a) - t.sum(2), axis=0)
     assert (off <= 8 * 2.0**-24 * np.linalg.norm(t, axis=0).sum(1)).all()
+
+
+@pytest.mark.parametrize("n", [66, 1023, 1025, 4095, 4097, 4159, 8192, 20479, 20480, 20481])
+@pytest.mark.parametrize("layout", ["cube", "half on one point"])
+def test_rank_order_is_the_radix_order(ctx, n, layout):
+    """Ordering by rank against the radix passes at the edges of its launch (one key and
+    four keys a wave, ragged last waves, the largest size and one beyond): the same
+    permutation, so the same forces bit for bit, with equal codes told apart by index."""
+    r = np.random.default_rng(n)
+    pos = [r.uniform(-1, 1, n) for _ in range(3)]
+    if layout != "cube":
+        for a in pos:
+            a[r.permutation(n)[: n // 2]] = 0.25
+    results = []
+    try:
+        for small in (1, 2):
+            ctx.set_direct_config(small_order=small, pair_mode=2)
+            results.append(evaluate(ctx, tuple(pos), np.full(n, 1.0 / n), eps=0.05)[0])
+    finally:
+        ctx.set_direct_config(small_order=1, pair_mode=1)
+    np.testing.assert_array_equal(np.stack(results[0]), np.stack(results[1]))
