@@ -146,7 +146,8 @@ ORR_API int orr_direct_static_limits(uint64_t* max_count, uint64_t* scratch_byte
  * small_order 1 (default) orders a system of at most 20,480 particles by
  * counting each key's rank (one launch up to 4096 particles, four above, instead
  * of a launch per radix pass; the same permutation, so the
- * same bits), 2 never. targets_per_lane 0, refine -1, block_target 0,
+ * same bits) and takes whole steps of at most 256 particles in one workgroup
+ * (the same bits again), 2 neither. targets_per_lane 0, refine -1, block_target 0,
  * pair_mode 0, equal_masses 0 and small_order 0 keep the current value. */
 typedef struct {
     int32_t targets_per_lane;

@@ -512,6 +512,19 @@ int orr_system_step(orr_system* s, const orr_step_config* c, double dt, uint64_t
         check_config(c);
         use_device(s->ctx);
         if (s->count == 0) return;
+        if (c->solver == 0) {
+            orr::SystemArrays arrays{};
+            for (int k = 0; k < 3; ++k) {
+                arrays.x[k] = s->array(k);
+                arrays.v[k] = s->array(3 + k);
+                arrays.a[k] = s->array(6 + k);
+            }
+            arrays.m = s->array(9);
+            if (orr::direct_tiny_steps(s->ctx, arrays, s->count, *c, dt, steps)) {
+                s->ctx->sync();
+                return;
+            }
+        }
         auto one_step = [&] {
             if (c->integrator == 2) {
                 rk4_step(s, *c, dt);

@@ -41,9 +41,11 @@
 #include <cmath>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 #include "close_pair.hpp"
 #include "engine.hpp"
+#include "morton_code.hpp"
 
 namespace orr {
 namespace {
@@ -599,6 +601,202 @@ __global__ __launch_bounds__(kTile) void direct_reduce(const double* __restrict_
     }
     const std::uint64_t dst = out.order != nullptr ? out.order[k] : k;
     store_field(dst, out.G * a0, out.G * a1, out.G * a2, out.ax, out.ay, out.az, out.kick);
+}
+
+// ---- tiny systems: whole steps in one workgroup ----------------------------------
+//
+// Up to kTinyTiles tiles a step is five or six launches of a few microseconds
+// each, 16 to 43 us that no launch fills. One workgroup does it all instead, any
+// number of steps in one launch: wave (t, J) of tiles^2 waves takes the pairs of
+// target tile t and source tile J, thread i < n holds particle i's state in
+// registers, and the ordered, packed tiles live in LDS. Every piece of
+// arithmetic is the launches' own -- the cube, codes and order (morton_code.hpp),
+// pack_tile, near_tiles, source_tile, the FP64 addition of the tiles' sums in
+// order, the unfused kicks and drifts -- so the steps are the same bits.
+// Bound by one workgroup's latency: a velocity Verlet step of two bodies 33 ->
+// 2.8 us, of 64 particles 33 -> 11, of 128 65 -> 18, of 256 72 -> 29.
+constexpr int kTinyTiles = 4;
+constexpr std::uint32_t kTinyMax = kTinyTiles * kTile;
+
+struct TinyArgs {
+    double *x[3] = {}, *v[3] = {}, *a[3] = {};
+    const double* m = nullptr;
+    std::uint32_t n = 0, steps = 0;
+    int mode = 0;      // 0: the field only, 1: kick-drift-kick substeps, 2: Runge-Kutta 4
+    int substeps = 1;  // mode 1
+    bool ordered = false;
+    float eps2 = 0.f;
+    double G = 1.0;
+    double kick[3] = {}, drift[3] = {};  // mode 1, per substep
+    double dt = 0.0;                     // mode 2
+};
+
+__device__ __forceinline__ double unfused(double a, double s, double b) {
+#pragma clang fp contract(off)
+    return a + s * b;
+}
+
+template<bool kSafe, bool kRefine, bool kRk4>
+__global__ __launch_bounds__(kTinyTiles * kTinyTiles * kTile) void direct_tiny(TinyArgs A) {
+    __shared__ float4 packed[kTinyMax], packed_lo[kTinyMax];
+    __shared__ double4 centres[kTinyTiles];
+    __shared__ float4 extents[kTinyTiles];
+    __shared__ double pos[4][kTinyMax];               // x y z m in tile order
+    __shared__ double sums[kTinyTiles][3][kTinyMax];  // [source tile][component][target]
+    __shared__ double wave_ext[kTinyTiles][6];
+    __shared__ std::uint32_t codes[kTinyMax], ranks[kTinyMax];
+    const std::uint32_t n = A.n, tiles = (n + kTile - 1) / kTile;
+    const std::uint32_t i = threadIdx.x, lane = i & (kTile - 1);
+    const std::uint32_t wave = __builtin_amdgcn_readfirstlane(i / kTile);
+    const bool mine = i < n;
+    double x[3] = {0, 0, 0}, v[3] = {0, 0, 0}, a[3] = {0, 0, 0};
+    const double m = mine ? A.m[i] : 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        if (mine) x[c] = A.x[c][i];
+        if (mine && A.mode != 0) {
+            v[c] = A.v[c][i];
+            a[c] = A.a[c][i];
+        }
+    }
+    // a = the field of the positions x.
+    auto field = [&] {
+        std::uint32_t at = i;  // the particle's place in tile order
+        if (A.ordered) {
+            if (wave < tiles) {
+                const double inf = __builtin_huge_val();
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const double lo = wave_min(mine ? x[c] : inf), hi = wave_max(mine ? x[c] : -inf);
+                    if (lane == 0) {
+                        wave_ext[wave][c] = lo;
+                        wave_ext[wave][3 + c] = hi;
+                    }
+                }
+            }
+            if (i < kTinyMax) ranks[i] = 0;
+            __syncthreads();
+            double lo[3], hi[3], cube[4];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                lo[c] = wave_ext[0][c];
+                hi[c] = wave_ext[0][3 + c];
+                for (std::uint32_t w = 1; w < tiles; ++w) {
+                    lo[c] = wave_ext[w][c] < lo[c] ? wave_ext[w][c] : lo[c];
+                    hi[c] = wave_ext[w][3 + c] > hi[c] ? wave_ext[w][3 + c] : hi[c];
+                }
+            }
+            make_cube(lo, hi, cube);
+            if (i < tiles * kTile) {
+                codes[i] = mine ? top_code(x[0], x[1], x[2], cube, static_cast<double>(kGrid) / cube[3]) : ~0u;
+            }
+            __syncthreads();
+            // Rank: keys (code, index) before particle k's, the waves of one tile
+            // of particles taking a tile of codes each.
+            const std::uint32_t k = wave % tiles * kTile + lane, j0 = wave / tiles * kTile;
+            if (k < n) {
+                const std::uint32_t key = codes[k];
+                std::uint32_t before = 0;
+#pragma unroll 8
+                for (std::uint32_t j = j0; j < j0 + kTile; ++j) {
+                    const std::uint32_t c = codes[j];
+                    before += c < key || (c == key && j < k) ? 1u : 0u;
+                }
+                atomicAdd(&ranks[k], before);
+            }
+            __syncthreads();
+            if (mine) at = ranks[i];
+        }
+        if (mine) {
+            pos[0][at] = x[0];
+            pos[1][at] = x[1];
+            pos[2][at] = x[2];
+            pos[3][at] = m;
+        }
+        __syncthreads();
+        if (wave < tiles) {
+            pack_tile(mine ? pos[0][i] : 0.0, mine ? pos[1][i] : 0.0, mine ? pos[2][i] : 0.0,
+                      mine ? pos[3][i] : 0.0, mine, i, wave, packed, packed_lo, centres, extents);
+        }
+        __syncthreads();
+        const std::uint32_t t = wave / tiles, J = wave % tiles, k = t * kTile + lane;
+        const float4 o = packed[k], l = packed_lo[k];
+        const double4 C = centres[t];
+        const float ox[1] = {o.x}, oy[1] = {o.y}, oz[1] = {o.z};
+        const float lx[1] = {l.x}, ly[1] = {l.y}, lz[1] = {l.z};
+        const double cx[1] = {C.x}, cy[1] = {C.y}, cz[1] = {C.z};
+        const float4 ce[1] = {extents[t]};
+        const bool live[1] = {k < n};
+        float sx[1] = {0.f}, sy[1] = {0.f}, sz[1] = {0.f}, kx[1] = {0.f}, ky[1] = {0.f}, kz[1] = {0.f};
+        const std::uint32_t sources = J + 1 < tiles ? kTile : n - (tiles - 1) * kTile;
+        source_tile<1, kSafe, kRefine, false, 8>(packed, packed_lo, centres, extents, J, false, sources, live,
+                                                 A.eps2, ox, oy, oz, lx, ly, lz, cx, cy, cz, ce, sx, sy, sz, kx,
+                                                 ky, kz);
+        sums[J][0][k] = static_cast<double>(sx[0]) - static_cast<double>(kx[0]);
+        sums[J][1][k] = static_cast<double>(sy[0]) - static_cast<double>(ky[0]);
+        sums[J][2][k] = static_cast<double>(sz[0]) - static_cast<double>(kz[0]);
+        __syncthreads();
+        if (mine) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                double total = 0.0;
+                for (std::uint32_t w = 0; w < tiles; ++w) total += sums[w][c][at];
+                a[c] = A.G * total;
+            }
+        }
+    };
+    // One evaluation a turn: what comes before it and after it by the turn's
+    // place in its step.
+    double x0[3], v0[3], slope_x[3], slope_v[3];
+    const std::uint32_t per_step = kRk4 ? 4 : A.substeps, turns = A.mode == 0 ? 1 : A.steps * per_step;
+    std::uint32_t p = 0;
+#pragma unroll 1
+    for (std::uint32_t turn = 0; turn < turns; ++turn) {
+        if constexpr (kRk4) {
+            // runge_kutta4.cpp:64-139, as rk4_kernel's four operations.
+            const double scale = p < 2 ? A.dt / 2 : p == 2 ? A.dt : A.dt / 6;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                if (p == 0) {
+                    x0[c] = x[c];
+                    v0[c] = slope_x[c] = v[c];
+                    slope_v[c] = a[c];
+                }
+                x[c] = unfused(x0[c], scale, p == 3 ? slope_x[c] : v[c]);
+                v[c] = unfused(v0[c], scale, p == 3 ? slope_v[c] : a[c]);
+            }
+        } else if (A.mode != 0) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                v[c] = unfused(v[c], A.kick[p], a[c]);
+                x[c] = unfused(x[c], A.drift[p], v[c]);
+            }
+        }
+        field();
+        if constexpr (kRk4) {
+            const double weight = p < 2 ? 2.0 : 1.0;
+            if (p < 3) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    slope_x[c] = unfused(slope_x[c], weight, v[c]);
+                    slope_v[c] = unfused(slope_v[c], weight, a[c]);
+                }
+            }
+        } else if (A.mode != 0) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) v[c] = unfused(v[c], A.kick[p], a[c]);
+        }
+        p = p + 1 == per_step ? 0 : p + 1;
+    }
+    if (!mine) return;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        A.a[c][i] = a[c];
+        if (A.mode != 0) {
+            A.x[c][i] = x[c];
+            A.v[c][i] = v[c];
+        }
+    }
 }
 
 // ---- batches: many independent systems in one launch ---------------------
@@ -1471,9 +1669,87 @@ std::size_t direct_batch_bytes(std::uint64_t tiles, std::uint64_t slots) {
     return packed_bytes(tiles) + centre_bytes(tiles) + slot_bytes(slots);
 }
 
+namespace {
+
+// Whether a system's evaluations are direct_tiny's: one source tile a group and
+// one target tile a wave, as the launches would take them, and no phase to time.
+bool tiny_applies(const orr_ctx* ctx, std::uint64_t n) {
+    if (n == 0 || n > kTinyMax || ctx->timing || ctx->direct_small_order != 1) return false;
+    const DirectShape d = direct_shape(ctx, n);
+    return d.R == 1 && d.per_split == 1 && !d.plan.use;
+}
+
+void tiny_launch(orr_ctx* ctx, const TinyArgs& args, double softening_squared) {
+    const std::uint32_t tiles = (args.n + kTile - 1) / kTile;
+    const bool safe = !(softening_squared > 0), refine = ctx->direct_refine != 0;
+    auto pick = [&](auto rk4) {
+        constexpr bool kRk4 = decltype(rk4)::value;
+        return safe ? (refine ? direct_tiny<true, true, kRk4> : direct_tiny<true, false, kRk4>)
+                    : (refine ? direct_tiny<false, true, kRk4> : direct_tiny<false, false, kRk4>);
+    };
+    auto kernel = args.mode == 2 ? pick(std::true_type{}) : pick(std::false_type{});
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(tiles * tiles * kTile), 0, ctx->stream, args);
+    ORR_LAUNCHED("direct_tiny");
+}
+
+}  // namespace
+
+bool direct_tiny_steps(orr_ctx* ctx, const SystemArrays& s, std::uint64_t n, const orr_step_config& c,
+                       double dt, std::uint64_t steps) {
+    if (!tiny_applies(ctx, n)) return false;
+    TinyArgs t;
+    for (int k = 0; k < 3; ++k) {
+        t.x[k] = s.x[k];
+        t.v[k] = s.v[k];
+        t.a[k] = s.a[k];
+    }
+    t.m = s.m;
+    t.n = static_cast<std::uint32_t>(n);
+    t.ordered = n > kTile;
+    t.eps2 = static_cast<float>(c.softening_squared);
+    t.G = c.gravitational_constant;
+    t.dt = dt;
+    if (c.integrator == 2) {
+        t.mode = 2;
+    } else {
+        t.mode = 1;
+        t.substeps = c.integrator == 1 ? 3 : 1;
+        const double w[3] = {kOuterWeight, kInnerWeight, kOuterWeight};
+        for (int p = 0; p < t.substeps; ++p) {
+            t.drift[p] = c.integrator == 1 ? w[p] * dt : dt;
+            t.kick[p] = t.drift[p] / 2;
+        }
+    }
+    // A launch of a few hundred steps lasts some milliseconds: no kernel holds
+    // the device for long.
+    constexpr std::uint64_t kStepsPerLaunch = 256;
+    while (steps > 0) {
+        t.steps = static_cast<std::uint32_t>(std::min(steps, kStepsPerLaunch));
+        tiny_launch(ctx, t, c.softening_squared);
+        steps -= t.steps;
+    }
+    return true;
+}
+
 void direct_evaluate(orr_ctx* ctx, const orr_direct_args& a, const FusedKick& kick) {
     if (a.count == 0) return;
     const bool ordered = a.spatial_order != 0 && a.count > 64;
+    if (kick.vx == nullptr && tiny_applies(ctx, a.count)) {
+        TinyArgs t;
+        t.x[0] = const_cast<double*>(a.x);
+        t.x[1] = const_cast<double*>(a.y);
+        t.x[2] = const_cast<double*>(a.z);
+        t.a[0] = a.ax;
+        t.a[1] = a.ay;
+        t.a[2] = a.az;
+        t.m = a.m;
+        t.n = static_cast<std::uint32_t>(a.count);
+        t.ordered = ordered;
+        t.eps2 = static_cast<float>(a.softening_squared);
+        t.G = a.gravitational_constant;
+        tiny_launch(ctx, t, a.softening_squared);
+        return;
+    }
     // Compact tiles need only the top 32 bits of the 63-bit codes: the four
     // upper radix passes of eight, or for a small system the same order by
     // counting ranks.

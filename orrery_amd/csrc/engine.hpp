@@ -239,6 +239,15 @@ __device__ __forceinline__ double kick_update(double v, double s, double a) {
 void direct_enqueue(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* order,
                     const FusedKick& kick = FusedKick{});
 
+// direct.hip: `steps` steps of a system of at most a few tiles, all in one
+// workgroup (enqueued, no synchronisation). False, with nothing done, where the
+// system is too large or the context's settings ask for the launches of their own.
+struct SystemArrays {
+    double *x[3], *v[3], *a[3], *m;
+};
+bool direct_tiny_steps(orr_ctx* ctx, const SystemArrays& s, std::uint64_t n, const orr_step_config& c,
+                       double dt, std::uint64_t steps);
+
 // direct.hip, batched: the direct systems of a batch as one tile space.
 // Tables are device arrays; tile/item/slot meaning is given in direct.hip.
 struct DirectBatchView {

@@ -456,3 +456,30 @@ def test_potential_at_tile_edges(ctx, n, eps):
     want = oracle.diagnostics(p, eps * eps)["potential"]
     s.close()
     assert abs(got - want) <= (n + 16) * 2.0**-53 * abs(want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("integrator", ["velocity-verlet", "yoshida4", "rk4"])
+@pytest.mark.parametrize("eps", [0.0, 0.02])
+@pytest.mark.parametrize("n", [1, 2, 7, 8, 9, 63, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257])
+def test_tiny_steps_equal_launched_steps(ctx, integrator, eps, n):
+    """Whole steps in one workgroup (up to 256 particles, one to sixteen waves) against
+    the launches they stand for (which small_order 2 asks for): the same bits after
+    steps of two sizes, and after more steps than one launch takes."""
+    p = oracle.plummer(n, n + 5)
+    cfg = E.StepConfig(integrator=integrator, softening=eps)
+    ends = []
+    try:
+        for small in (1, 2):
+            ctx.set_direct_config(small_order=small)
+            s = E.DeviceSystem(ctx, n)
+            s.upload(*p.arrays())
+            s.refresh(cfg)
+            s.step(cfg, 1e-3, 7)
+            s.step(cfg, 2e-3, 260 if n in (2, 65) else 2)
+            ends.append(s.download())
+            s.close()
+    finally:
+        ctx.set_direct_config(small_order=1)
+    for key in ends[0]:
+        np.testing.assert_array_equal(ends[0][key], ends[1][key], err_msg=key)
