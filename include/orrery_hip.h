@@ -86,6 +86,14 @@ ORR_API int orr_malloc(orr_ctx* ctx, uint64_t bytes, void** device_out);
 ORR_API int orr_free(orr_ctx* ctx, void* device);
 ORR_API int orr_upload(orr_ctx* ctx, void* device_dst, const void* host_src, uint64_t bytes);
 ORR_API int orr_download(orr_ctx* ctx, void* host_dst, const void* device_src, uint64_t bytes);
+/* Several host arrays of `count` doubles to or from device arrays at once (at
+ * most 10): small ones through a pinned buffer of the context in one transfer.
+ * An upload is ordered before later work of the context and has read the host
+ * arrays when it returns; a download follows earlier work and has filled them. */
+ORR_API int orr_upload_rows(orr_ctx* ctx, double* const* dst, const double* const* src, uint32_t rows,
+                            uint64_t count);
+ORR_API int orr_download_rows(orr_ctx* ctx, double* const* dst, double* const* src, uint32_t rows,
+                              uint64_t count);
 ORR_API int orr_memset(orr_ctx* ctx, void* device_dst, int32_t value, uint64_t bytes);
 
 /* ---- direct summation --------------------------------------------------- */

@@ -144,6 +144,8 @@ SIGNATURES = {
     "orr_free": [_vp, _vp],
     "orr_upload": [_vp, _vp, _vp, ctypes.c_uint64],
     "orr_download": [_vp, _vp, _vp, ctypes.c_uint64],
+    "orr_upload_rows": [_vp, _vp, _vp, ctypes.c_uint32, ctypes.c_uint64],
+    "orr_download_rows": [_vp, _vp, _vp, ctypes.c_uint32, ctypes.c_uint64],
     "orr_memset": [_vp, _vp, ctypes.c_int32, ctypes.c_uint64],
     "orr_direct_eval": [_vp, ctypes.POINTER(OrrDirectArgs)],
     "orr_direct_eval_static": [_vp, ctypes.POINTER(OrrDirectArgs)],

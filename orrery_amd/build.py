@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIBRARY = os.path.join(HERE, "liborrery_hip.so")
 SOURCES = ["context.hip", "capi.hip", "direct.hip", "morton.hip", "scan.hip", "tree.hip", "batch.hip", "serve.hip", "io.hip",
-           "integrate.hip", "probes.hip"]
+           "integrate.hip", "stage.hip", "probes.hip"]
 # Host-only translation units, compiled by the host compiler: the seeded
 # initial-condition sampler must make the same libm calls, unfused, as the
 # reference's CPU build.

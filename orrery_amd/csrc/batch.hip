@@ -684,11 +684,15 @@ int orr_batch_upload(orr_batch* b, uint32_t system, const double* x, const doubl
         orr::use_device(b);
         const std::uint64_t begin = b->first[s], count = b->first[s + 1] - begin;
         const double* src[10] = {x, y, z, vx, vy, vz, nullptr, nullptr, nullptr, m};
+        const double* from[10];
+        double* to[10];
+        int rows = 0;
         for (int k = 0; k < 10; ++k) {
-            if (src[k] == nullptr || count == 0) continue;
-            ORR_HIP(hipMemcpyAsync(b->array(k) + begin, src[k], count * sizeof(double),
-                                   hipMemcpyHostToDevice, b->dctx->stream));
+            if (src[k] == nullptr) continue;
+            from[rows] = src[k];
+            to[rows++] = b->array(k) + begin;
         }
+        orr::stage_upload(b->dctx, to, from, rows, count);
         orr::sync_all(b);
     });
 }
@@ -702,12 +706,14 @@ int orr_batch_download(orr_batch* b, uint32_t system, double* x, double* y, doub
         orr::sync_all(b);
         const std::uint64_t begin = b->first[s], count = b->first[s + 1] - begin;
         double* dst[9] = {x, y, z, vx, vy, vz, ax, ay, az};
+        double *from[9], *to[9];
+        int rows = 0;
         for (int k = 0; k < 9; ++k) {
-            if (dst[k] == nullptr || count == 0) continue;
-            ORR_HIP(hipMemcpyAsync(dst[k], b->array(k) + begin, count * sizeof(double),
-                                   hipMemcpyDeviceToHost, b->dctx->stream));
+            if (dst[k] == nullptr) continue;
+            from[rows] = b->array(k) + begin;
+            to[rows++] = dst[k];
         }
-        b->dctx->sync();
+        orr::stage_download(b->dctx, to, from, rows, count);
     });
 }
 

@@ -237,6 +237,29 @@ int orr_download(orr_ctx* ctx, void* dst, const void* src, uint64_t bytes) {
     });
 }
 
+int orr_upload_rows(orr_ctx* ctx, double* const* dst, const double* const* src, uint32_t rows,
+                    uint64_t count) {
+    return guarded([&] {
+        require(ctx != nullptr && rows <= orr::kStageRows, "null context or more than 10 rows");
+        use_device(ctx);
+        if (rows == 0 || count == 0) return;
+        require(dst != nullptr && src != nullptr, "null argument");
+        for (uint32_t k = 0; k < rows; ++k) require(dst[k] != nullptr && src[k] != nullptr, "null row");
+        orr::stage_upload(ctx, dst, src, static_cast<int>(rows), count);
+    });
+}
+
+int orr_download_rows(orr_ctx* ctx, double* const* dst, double* const* src, uint32_t rows, uint64_t count) {
+    return guarded([&] {
+        require(ctx != nullptr && rows <= orr::kStageRows, "null context or more than 10 rows");
+        use_device(ctx);
+        if (rows == 0 || count == 0) return;
+        require(dst != nullptr && src != nullptr, "null argument");
+        for (uint32_t k = 0; k < rows; ++k) require(dst[k] != nullptr && src[k] != nullptr, "null row");
+        orr::stage_download(ctx, dst, src, static_cast<int>(rows), count);
+    });
+}
+
 int orr_memset(orr_ctx* ctx, void* dst, int32_t value, uint64_t bytes) {
     return guarded([&] {
         require(ctx != nullptr && (bytes == 0 || dst != nullptr), "null argument");
@@ -472,11 +495,15 @@ int orr_system_upload(orr_system* s, const double* x, const double* y, const dou
         require(s != nullptr, "null system");
         use_device(s->ctx);
         const double* src[10] = {x, y, z, vx, vy, vz, nullptr, nullptr, nullptr, m};
+        const double* from[10];
+        double* to[10];
+        int rows = 0;
         for (int k = 0; k < 10; ++k) {
-            if (src[k] == nullptr || s->count == 0) continue;
-            ORR_HIP(hipMemcpyAsync(s->array(k), src[k], s->count * sizeof(double),
-                                   hipMemcpyHostToDevice, s->ctx->stream));
+            if (src[k] == nullptr) continue;
+            from[rows] = src[k];
+            to[rows++] = s->array(k);
         }
+        orr::stage_upload(s->ctx, to, from, rows, s->count);
         s->ctx->sync();
     });
 }
@@ -487,12 +514,14 @@ int orr_system_download(orr_system* s, double* x, double* y, double* z, double* 
         require(s != nullptr, "null system");
         use_device(s->ctx);
         double* dst[9] = {x, y, z, vx, vy, vz, ax, ay, az};
+        double *from[9], *to[9];
+        int rows = 0;
         for (int k = 0; k < 9; ++k) {
-            if (dst[k] == nullptr || s->count == 0) continue;
-            ORR_HIP(hipMemcpyAsync(dst[k], s->array(k), s->count * sizeof(double),
-                                   hipMemcpyDeviceToHost, s->ctx->stream));
+            if (dst[k] == nullptr) continue;
+            from[rows] = s->array(k);
+            to[rows++] = dst[k];
         }
-        s->ctx->sync();
+        orr::stage_download(s->ctx, to, from, rows, s->count);
     });
 }
 

@@ -146,6 +146,7 @@ void free_context(orr_ctx* ctx) noexcept {
     drop_captured(ctx->tree_graph);
     drop_captured(ctx->direct_graph);
     for (Buffer* b : ctx->buffers()) b->release();
+    ctx->staging.release();
     for (auto& p : ctx->pending) {
         (void)hipEventDestroy(p.start);
         (void)hipEventDestroy(p.stop);

@@ -12,6 +12,7 @@
 #include <cstddef>
 #include <array>
 #include <functional>
+#include <mutex>
 #include <cstdint>
 #include <new>
 #include <stdexcept>
@@ -171,6 +172,22 @@ struct orr_ctx {
         hipGraphExec_t exec = nullptr;
     };
     Captured tree_graph, direct_graph;
+
+    // The pinned buffer of small host transfers (stage.hip), at most
+    // kStageBytes; `busy` while a launch may still read it. The lock covers it
+    // for callers that move data of one context from several threads.
+    struct Staging {
+        void* ptr = nullptr;
+        std::size_t bytes = 0;
+        bool busy = false;
+        std::mutex lock;
+        void release() noexcept {
+            if (ptr != nullptr) (void)hipHostFree(ptr);
+            ptr = nullptr;
+            bytes = 0;
+        }
+    };
+    Staging staging;
     // True while a run_captured sequence is being captured: a run_captured
     // reached from inside it then enqueues its work inline (into the same
     // capture) instead of launching or capturing a graph of its own.
@@ -238,6 +255,18 @@ __device__ __forceinline__ double kick_update(double v, double s, double a) {
 // direct.hip: enqueue the direct sum (no synchronisation).
 void direct_enqueue(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* order,
                     const FusedKick& kick = FusedKick{});
+
+// stage.hip: `rows` host arrays of `count` doubles to or from device arrays, in
+// the order of the context's stream. An upload has read the host arrays when it
+// returns; a download waits for the stream and has filled them.
+constexpr int kStageRows = 10;
+// A system's state out and in, pinned rows against nine or seven pageable
+// copies: 29 / 176 and 27 / 65 us at 1000 particles, 82 / 177 and 57 / 96 at
+// 16,384, 529 / 559 and 144 / 146 at 65,536 (4.5 MiB); beyond, uploads are slower.
+constexpr std::size_t kStageBytes = std::size_t{4} << 20;
+void stage_upload(orr_ctx* ctx, double* const* device, const double* const* host, int rows,
+                  std::uint64_t count);
+void stage_download(orr_ctx* ctx, double* const* host, double* const* device, int rows, std::uint64_t count);
 
 // direct.hip: `steps` steps of a system of at most a few tiles, all in one
 // workgroup (enqueued, no synchronisation). False, with nothing done, where the

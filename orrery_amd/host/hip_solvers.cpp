@@ -63,22 +63,33 @@ public:
             capacity_ = n;
         }
         const std::span<const Real> in[4] = {positions.x, positions.y, positions.z, masses};
-        for (int k = 0; k < 4; ++k) upload(buffers_[k], in[k]);
         std::array<double*, 7> out{};
         for (int k = 0; k < 7; ++k) out[k] = static_cast<double*>(buffers_[k]);
+        if constexpr (std::is_same_v<Real, double>) {
+            const double* from[4];
+            for (int k = 0; k < 4; ++k) from[k] = in[k].data();
+            check(orr_upload_rows(ctx_, out.data(), from, 4, n));
+        } else {
+            for (int k = 0; k < 4; ++k) upload(buffers_[k], in[k]);
+        }
         return out;
     }
 
     void download(core::Vec3Span<Real> accelerations) {
         const std::span<Real> out[3] = {accelerations.x, accelerations.y, accelerations.z};
-        for (int k = 0; k < 3; ++k) {
-            if constexpr (std::is_same_v<Real, double>) {
-                check(orr_download(ctx_, out[k].data(), buffers_[4 + k], out[k].size() * sizeof(double)));
-            } else {
-                host_.resize(out[k].size());
-                check(orr_download(ctx_, host_.data(), buffers_[4 + k], host_.size() * sizeof(double)));
-                for (Index i = 0; i < host_.size(); ++i) out[k][i] = static_cast<Real>(host_[i]);
+        if constexpr (std::is_same_v<Real, double>) {
+            double *to[3], *from[3];
+            for (int k = 0; k < 3; ++k) {
+                to[k] = out[k].data();
+                from[k] = static_cast<double*>(buffers_[4 + k]);
             }
+            check(orr_download_rows(ctx_, to, from, 3, out[0].size()));
+            return;
+        }
+        for (int k = 0; k < 3; ++k) {
+            host_.resize(out[k].size());
+            check(orr_download(ctx_, host_.data(), buffers_[4 + k], host_.size() * sizeof(double)));
+            for (Index i = 0; i < host_.size(); ++i) out[k][i] = static_cast<Real>(host_[i]);
         }
     }
 

@@ -116,6 +116,23 @@ class Context:
         C.check(self._lib.orr_download(self.handle, dst.ctypes.data_as(ctypes.c_void_p),
                                        ctypes.c_void_p(src), dst.nbytes))
 
+    def upload_rows(self, dst, src) -> None:
+        """Equally long contiguous FP64 host arrays to device addresses (orr_upload_rows)."""
+        n = len(src[0])
+        assert all(len(a) == n and a.dtype == np.float64 and a.flags.c_contiguous for a in src)
+        rows = ctypes.c_void_p * len(src)
+        C.check(self._lib.orr_upload_rows(self.handle, rows(*dst), rows(*(a.ctypes.data for a in src)),
+                                          len(src), n))
+
+    def download_rows(self, dst, src) -> None:
+        """Device addresses to equally long contiguous FP64 host arrays (orr_download_rows)."""
+        n = len(dst[0])
+        assert all(len(a) == n and a.dtype == np.float64 and a.flags.c_contiguous and a.flags.writeable
+                   for a in dst)
+        rows = ctypes.c_void_p * len(dst)
+        C.check(self._lib.orr_download_rows(self.handle, rows(*(a.ctypes.data for a in dst)), rows(*src),
+                                            len(dst), n))
+
     # -- direct kernel configuration (autotuner knob) -----------------------
     def set_direct_config(self, targets_per_lane: int = 0, refine: int = -1, block_target: int = 0,
                           pair_mode: int = 0, equal_masses: int = 0, small_order: int = 0) -> None:
@@ -225,6 +242,20 @@ class _Staging:
             self.capacity = cap
         return self.arrays
 
+    def put(self, positions, masses) -> None:
+        host = [np.ascontiguousarray(a, dtype=np.float64) for a in (*positions, masses)]
+        self.ctx.upload_rows([a.ptr for a in self.arrays[:4]], host)
+
+    def get(self, accelerations) -> None:
+        """Straight into arrays that can take it, else by way of a copy."""
+        direct = [isinstance(a, np.ndarray) and a.ndim == 1 and a.dtype == np.float64
+                  and a.flags.c_contiguous and a.flags.writeable for a in accelerations]
+        out = [a if ok else np.empty(len(a)) for a, ok in zip(accelerations, direct)]
+        self.ctx.download_rows(out, [a.ptr for a in self.arrays[4:]])
+        for a, o, ok in zip(accelerations, out, direct):
+            if not ok:
+                a[:] = o
+
 
 def _check_spans(positions, masses, accelerations):
     x, y, z = positions
@@ -296,14 +327,10 @@ class HipDirectSolver:
             self._tally(0)
             return
         d = self._staging.reserve(n)
-        for dev, host in zip(d[:4], (*positions, masses)):
-            self.ctx.upload(dev.ptr, np.ascontiguousarray(host, dtype=np.float64))
+        self._staging.put(positions, masses)
         args = self._args(tuple(a.ptr for a in d), n)
         C.check(C.load().orr_direct_eval(self.ctx.handle, ctypes.byref(args)))
-        for dev, host in zip(d[4:], accelerations):
-            out = np.empty(n)
-            self.ctx.download(out, dev.ptr)
-            host[:] = out
+        self._staging.get(accelerations)
         self._tally(n)
 
     def _tally(self, n: int) -> None:
@@ -396,14 +423,10 @@ class HipTreeSolver:
             self._count.evaluations += 1
             return
         d = self._staging.reserve(n)
-        for dev, host in zip(d[:4], (*positions, masses)):
-            self.ctx.upload(dev.ptr, np.ascontiguousarray(host, dtype=np.float64))
+        self._staging.put(positions, masses)
         args = self._args(tuple(a.ptr for a in d), n)
         C.check(C.load().orr_tree_eval(self.ctx.handle, ctypes.byref(args), ctypes.byref(self._stats)))
-        for dev, host in zip(d[4:], accelerations):
-            out = np.empty(n)
-            self.ctx.download(out, dev.ptr)
-            host[:] = out
+        self._staging.get(accelerations)
         self._tally()
 
     def _tally(self) -> None:

@@ -483,3 +483,21 @@ def test_tiny_steps_equal_launched_steps(ctx, integrator, eps, n):
         ctx.set_direct_config(small_order=1)
     for key in ends[0]:
         np.testing.assert_array_equal(ends[0][key], ends[1][key], err_msg=key)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 255, 257, 58254, 58255, 74898, 74899])
+def test_state_round_trip_at_the_staging_limit(ctx, n):
+    """Up and down unchanged on either side of 4 MiB of rows (nine out, seven in)."""
+    r = np.random.default_rng(n)
+    arrays = [r.standard_normal(n) for _ in range(7)]
+    s = E.DeviceSystem(ctx, n)
+    sent = [a.copy() for a in arrays]
+    s.upload(*arrays)
+    for a in arrays:
+        a[:] = np.nan  # the upload has read its source when it returns
+    back = s.download()
+    s.close()
+    for key, a in zip(("x", "y", "z", "vx", "vy", "vz"), sent):
+        np.testing.assert_array_equal(back[key], a)
+    assert not any(back[k].any() for k in ("ax", "ay", "az"))
