@@ -58,8 +58,8 @@ constexpr std::uint8_t kNoBoundary = 22;
 constexpr int kMaxChildren = 8;                 // octants
 constexpr std::uint32_t kNoChild = 0xffffffffu;
 // Spare float4 entries past the last particle of leaf_rel: a leaf's sources are
-// read in rounds of four.
-constexpr std::size_t kLeafPad = 3;
+// read in rounds of four, one round ahead.
+constexpr std::size_t kLeafPad = 4;
 // The fewest targets a walk wave holds.
 constexpr std::uint64_t kMinLanes = 16;
 
@@ -524,15 +524,47 @@ __device__ __forceinline__ void kahan(float p, float& s, float& c) {
     s = t;
 }
 
-// Up to this many full (64-lane) walk waves -- two per SIMD of the 256 CUs --
-// half-lane waves are faster (quadrupole walk, two-disc collision: 1.088 ->
-// 0.981 ms at N = 65,536, 1.328 -> 1.265 ms at 131,072); above it they are
-// slower (1.35 -> 1.83 ms at 262,144): the walk is bound by issue, not by
-// latency, once each SIMD has a few waves. Up to a quarter of a wave per SIMD,
-// waves of 16 targets (monopole walk of a 16,384-particle Plummer sphere: 64
-// targets a wave 0.566, 32 0.521, 16 0.470 ms).
-constexpr std::uint64_t kHalfLaneWaves = 2 * 4 * 256;
-constexpr std::uint64_t kQuarterLaneWaves = 256;
+// Targets a wave, and waves that share the walk of a group of targets (parts),
+// by the launch's full (64-lane) waves. Walk in ms, Plummer spheres (P) and
+// two-disc collisions (D), opening angle 0.5 or 0.6, monopoles (m) or quadrupoles (q),
+// as {16 targets, 1 part}, {32, 1}, {16, 8}, {16, 4}, {32, 2}, and from 65,536 on
+// {32, 1}, {64, 1}, {32, 2}:
+//   1000 Pq  0.145 0.153 0.049 0.065           28,000 Pq 0.690 0.727   -   0.676 0.582
+//   4096 Pq  0.336 0.372 0.125 0.156           49,152 Pq 0.828 0.828   -   1.153 0.690
+//   8192 Dm  0.263 0.277 0.118 0.167           60,000 Dm 0.505 0.492   -   0.837 0.418
+//   8192 Pq  0.490 0.539 0.231 0.221           65,536 Dq 0.822 0.896 0.758
+//   10,240 Pm 0.392 0.427 0.243 0.188          73,728 Pq 0.974 1.013 0.922
+//   16,384 Pm 0.447 0.483 0.417 0.259          81,920 Dq 0.863 0.912 0.892
+//   24,576 Pq 0.678 0.705   -   0.505 0.534    98,304 Pq 1.026 1.062 1.140
+//   24,576 Dm 0.473 0.493   -   0.358 0.373    106,496 Pq 1.062 1.017 1.151
+// More parts pay while the launch leaves the SIMDs short of waves; past that
+// the nodes walked twice, and the room in LDS, cost more than they hide.
+struct WalkShape {
+    int lanes, parts;
+};
+constexpr std::uint64_t kEightPartWaves = 128;
+constexpr std::uint64_t kFourPartWaves = 384;
+constexpr std::uint64_t kTwoPartWaves = 1152;
+constexpr std::uint64_t kHalfLaneWaves = 1600;
+WalkShape walk_shape(std::uint64_t full_waves) {
+    if (full_waves <= kEightPartWaves) return {16, 8};
+    if (full_waves <= kFourPartWaves) return {16, 4};
+    if (full_waves <= kTwoPartWaves) return {32, 2};
+    return {full_waves <= kHalfLaneWaves ? 32 : 64, 1};
+}
+
+// Runs a part of a split walk has room for: as many as let all groups of the
+// launch be on the chip at once (the 160 KB of LDS of a CU over its share of
+// the groups, less 4 KB for the kernel's own), within a block's 64 KB.
+// Too few make a part wait for the one before it (4096 particles, eight parts,
+// quadrupoles: 24 runs 0.243, 32 runs 0.169 ms), too many make a group wait for a
+// place (49,152 particles, two parts of 32 targets: 48 runs 0.762, 64 runs,
+// which leave room for five groups of six on a CU, 0.926 ms).
+std::uint32_t split_runs(std::uint32_t groups, std::uint32_t run_bytes) {
+    constexpr std::uint32_t kLds = 160 << 10, kBlockLds = 64 << 10, kOwn = 4 << 10, kCus = 256;
+    const std::uint32_t share = std::min(kLds / ((groups + kCus - 1) / kCus), kBlockLds) - kOwn;
+    return std::max(share / run_bytes, 4u);
+}
 
 // Workgroups are dispatched to the 8 XCDs in turn (block b to XCD b mod 8),
 // and each XCD has its own L2. Neighbouring targets in Morton order visit the
@@ -601,31 +633,23 @@ __device__ __forceinline__ void accept(WalkTarget& t, float mass, const float4& 
     }
 }
 
-// Four consecutive leaf particles in scalar registers.
+// Four consecutive leaf particles. The last round of a leaf still loads four
+// (leaf_rel holds kLeafPad spare entries past the last particle).
 struct LeafRound {
     float4 q[4];
 };
 __device__ __forceinline__ LeafRound load_round(const float4* __restrict__ leaf_rel, std::uint32_t j) {
-    // Four sources from one base, so that their scalar loads are one load. A
-    // last round of fewer than four still loads four (leaf_rel holds kLeafPad
-    // spare entries past the last particle).
     const float4* const q = leaf_rel + j;
-    LeafRound v{{q[0], q[1], q[2], q[3]}};
-    return v;
-}
-__device__ __forceinline__ void pin(const LeafRound& v) {
-    asm volatile("" ::"s"(v.q[0].x), "s"(v.q[0].y), "s"(v.q[0].z), "s"(v.q[0].w), "s"(v.q[1].x), "s"(v.q[1].y),
-                 "s"(v.q[1].z), "s"(v.q[1].w), "s"(v.q[2].x), "s"(v.q[2].y), "s"(v.q[2].z), "s"(v.q[2].w),
-                 "s"(v.q[3].x), "s"(v.q[3].y), "s"(v.q[3].z), "s"(v.q[3].w));
+    return LeafRound{{q[0], q[1], q[2], q[3]}};
 }
 
-// Particle-particle terms of leaf [b, e) for one target, then the partial is
-// Kahan-added. The target is re-expressed against the leaf's centre cb in FP64
-// (ca: the centre of the target's own leaf).
+// Particle-particle terms of leaf [b, e) for one target. The target is
+// re-expressed against the leaf's centre cb in FP64 (ca: the centre of the
+// target's own leaf).
 template<bool kSafe>
 __device__ __forceinline__ void leaf_pairs(WalkTarget& t, const double4& cb, double cax, double cay,
                                            double caz, const float4* __restrict__ leaf_rel,
-                                           std::uint32_t b, std::uint32_t e, float eps2) {
+                                           std::uint32_t b, std::uint32_t e, float eps2, std::uint32_t lane0) {
     const float tx = t.oi.x - static_cast<float>(cb.x - cax);
     const float ty = t.oi.y - static_cast<float>(cb.y - cay);
     const float tz = t.oi.z - static_cast<float>(cb.z - caz);
@@ -642,27 +666,35 @@ __device__ __forceinline__ void leaf_pairs(WalkTarget& t, const double4& cb, dou
         t.pz = __builtin_fmaf(f, dz, t.pz);
     };
     // Whole rounds without a branch between the four terms, whose chains then
-    // overlap; the sums still take them in index order.
+    // overlap; the sums still take them in index order. `lane0` is a zero the
+    // compiler cannot see through: the sources come through the vector cache,
+    // where loads return in order and a round can be on its way while the one
+    // before it is summed. Read through the scalar cache, every round is a
+    // miss (a leaf is a few lines that few waves share), waited for in full,
+    // and pushes out the node records (16,384 particles, 16 targets a wave:
+    // walk 0.488 -> 0.455 ms; 262,144 and 2,097,152 the same).
     std::uint32_t j = b;
-    for (; j + 4 <= e; j += 4) {
-        const LeafRound v = load_round(leaf_rel, j);
-        pin(v);
+    LeafRound v = load_round(leaf_rel, j + lane0);
+    while (j + 4 <= e) {
+        const LeafRound w = load_round(leaf_rel, j + 4 + lane0);
         pair(v.q[0]);
         pair(v.q[1]);
         pair(v.q[2]);
         pair(v.q[3]);
+        v = w;
+        j += 4;
     }
     if (j < e) {
-        const LeafRound v = load_round(leaf_rel, j);
-        pin(v);
         pair(v.q[0]);
         if (j + 1 < e) pair(v.q[1]);
         if (j + 2 < e) pair(v.q[2]);
     }
+}
+
+__device__ __forceinline__ void kahan(WalkTarget& t) {
     kahan(t.px, t.sx, t.kx);
     kahan(t.py, t.sy, t.ky);
     kahan(t.pz, t.sz, t.kz);
-    t.px = t.py = t.pz = 0.f;
 }
 
 // A wave's stack of pending sibling lists, level d in lane d of a few vector
@@ -670,7 +702,11 @@ __device__ __forceinline__ void leaf_pairs(WalkTarget& t, const double4& cb, dou
 // execution mask); the lane select goes through m0, since the instruction can
 // read only one scalar register.
 __device__ __forceinline__ void lane_write(std::uint32_t& reg, std::uint32_t value, std::uint32_t lane) {
-    asm("s_mov_b32 m0, %2\n\ts_nop 0\n\tv_writelane_b32 %0, %1, m0" : "+v"(reg) : "s"(value), "s"(lane) : "m0");
+    asm("s_mov_b32 m0, %2\n\ts_nop 0\n\tv_writelane_b32 %0, %1, m0"
+        : "+v"(reg)
+        : "s"(__builtin_amdgcn_readfirstlane(static_cast<int>(value))),
+          "s"(__builtin_amdgcn_readfirstlane(static_cast<int>(lane)))
+        : "m0");
 }
 __device__ __forceinline__ std::uint32_t lane_read(std::uint32_t reg, std::uint32_t lane) {
     return static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(reg), static_cast<int>(lane)));
@@ -697,6 +733,20 @@ __device__ void add_counts(unsigned long long* __restrict__ stats, std::uint32_t
     atomicAdd(&st[3], slots);
 }
 
+// How much of a target's walk lies within d nodes of its own leaf, in the
+// depth-first order: the cells a walk opens on each level lie around the
+// target at the scale of that level, so the visits thin out as 1 / d beyond the
+// nearest few hundred nodes, all of which it visits. Only the balance of a
+// split walk rests on it. kNearNodes 256 to 2048 measured alike (16,384
+// particles in four parts: walk 0.29 to 0.33 ms).
+constexpr float kNearNodes = 512.f;
+__device__ __forceinline__ float walk_weight(float d) {
+    return d <= kNearNodes ? d : kNearNodes * (1.f + __logf(d / kNearNodes));
+}
+__device__ __forceinline__ float walk_reach(float weight) {
+    return weight <= kNearNodes ? weight : kNearNodes * __expf(weight / kNearNodes - 1.f);
+}
+
 // Wave-coherent walk. Each of the first kLanes lanes owns kR targets (wave w
 // owns the kLanes kR sorted particles from kLanes kR w, target r of lane l
 // being kLanes r + l; with kLanes = 32 the other half of the wave holds none,
@@ -714,18 +764,45 @@ __device__ void add_counts(unsigned long long* __restrict__ stats, std::uint32_t
 //
 // kMany: the targets may belong to several systems (a batch); the systems of
 // a wave's targets are then walked one after another.
-template<int kR, bool kSafe, bool kQuad, int kLanes, bool kMany>
-__global__ __launch_bounds__(kBlock) void tree_walk(
+//
+// kSplit > 1: a group of targets is walked by kSplit waves, the parts, each a
+// range of the nodes. With one wave a group, a small launch leaves a SIMD a
+// wave or two, which issue at half the rate a SIMD can and wait out every load,
+// and the launch lasts as long as its slowest wave (16,384 particles, 1024 waves of 16
+// targets: 0.30 ms on average, 0.51 the slowest, 183 running after three
+// quarters of the time). A target's partial sum starts at zero after each leaf
+// it visits, so its walk is a row of runs, leaf to leaf, that do not depend on
+// one another: a part computes the runs that begin at a leaf among its nodes,
+// each to its end, which may lie among the next part's (`tail`). Its own
+// first nodes, up to the first leaf, are the part before's run; it walks them
+// only to find that leaf. The runs of part 0 go into the Kahan sums as they
+// end; those of the others wait in LDS until the sums of the part before are
+// there, then go in in order: the sums see the same partials in the same
+// order, and the results are the same bits. A part whose room in LDS is full
+// waits for the part before it and then adds its runs directly; part 0 waits
+// for nobody, so every wait ends. A visit is counted by the part that owns the node.
+//
+// The one-wave walk of one system is held to 64 vector registers, eight waves
+// a SIMD (of 67 it would take; 2,097,152 particles: 8.6 -> 8.3 ms).
+template<int kR, bool kSafe, bool kQuad, int kLanes, bool kMany, int kSplit>
+__global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
+                             kSplit == 1 && kR == 1 && !kMany ? 8 : 1) void tree_walk(
     const WalkNode* __restrict__ nodes, const QuadF* __restrict__ quads,
     const double4* __restrict__ node_geo,
     const float4* __restrict__ root_rel, const float4* __restrict__ leaf_rel,
     const std::uint32_t* __restrict__ leaf_of, const std::uint32_t* __restrict__ index,
     const std::uint32_t* __restrict__ counters, const std::uint32_t* __restrict__ seg_of,
     const std::uint32_t* __restrict__ seg_start, const std::uint32_t* __restrict__ first_node,
-    std::uint32_t n, float eps2, double G,
+    std::uint32_t n, float eps2, double G, std::uint32_t runs,
     double* __restrict__ ax, double* __restrict__ ay, double* __restrict__ az,
     unsigned long long* __restrict__ stats, unsigned long long* __restrict__ wave_stats) {
-    const std::uint32_t wave = xcd_block(blockIdx.x, gridDim.x) * (kBlock / 64) + threadIdx.x / 64;
+    static_assert(kSplit == 1 || kR == 1);
+    // The parts of a split walk have the same targets.
+    constexpr int kSlots = kSplit == 1 ? kBlock : 64;
+    const std::uint32_t wave = kSplit == 1
+                                   ? xcd_block(blockIdx.x, gridDim.x) * (kBlock / 64) + threadIdx.x / 64
+                                   : xcd_block(blockIdx.x, gridDim.x);
+    const std::uint32_t part = kSplit == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const std::uint32_t lane = threadIdx.x & 63;
     const std::uint32_t M = counters[0];
     WalkTarget t[kR];
@@ -734,7 +811,14 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
     // Each lane's targets' own leaf centres, read at every leaf visit: held in
     // LDS rather than registers (12 KB a block at two targets a lane) or
     // re-read from memory at each visit. A lane reads only its own slots.
-    __shared__ double s_own[kR][3][kBlock];
+    __shared__ double s_own[kR][3][kSlots];
+    // What the parts of a split walk hand on: the chain of Kahan sums, the
+    // counts, and who has finished.
+    extern __shared__ float s_runs[];
+    __shared__ float s_chain[6][kLanes];
+    __shared__ unsigned long long s_count[kSplit][4];
+    __shared__ std::uint32_t s_done[kSplit];
+    const std::uint32_t slot = kSplit == 1 ? threadIdx.x : lane;
 #pragma unroll
     for (int r = 0; r < kR; ++r) {
         const std::uint32_t i = wave * (kLanes * kR) + kLanes * r + lane;
@@ -744,24 +828,68 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
         t[r].oi = leaf_rel[ic];
         t[r].own = leaf_of[ic];
         const double4 ca = node_geo[t[r].own];
-        s_own[r][0][threadIdx.x] = ca.x;
-        s_own[r][1][threadIdx.x] = ca.y;
-        s_own[r][2][threadIdx.x] = ca.z;
+        if (part == 0) {
+            s_own[r][0][slot] = ca.x;
+            s_own[r][1][slot] = ca.y;
+            s_own[r][2][slot] = ca.z;
+        }
         seg[r] = kMany ? seg_of[ic] : 0u;
         todo[r] = __ballot(valid);
         t[r].sx = t[r].sy = t[r].sz = t[r].kx = t[r].ky = t[r].kz = 0.f;
         t[r].px = t[r].py = t[r].pz = 0.f;
         t[r].pc = 0;
     }
+    if constexpr (kSplit > 1) {
+        if (threadIdx.x < kSplit) s_done[threadIdx.x] = 0;
+        __syncthreads();
+    }
     // An FP32 instruction with a scalar operand issues at half the rate of one
     // that reads only vector registers: eps^2 enters every term.
     asm volatile("" : "+v"(eps2));
+    std::uint32_t lane0 = 0;  // leaf_pairs
+    asm volatile("" : "+v"(lane0));
     std::uint32_t steps = 0;
     std::uint32_t systems = 0;   // systems walked by this wave
     std::uint32_t seg0 = 0;      // the first of them
     // Particle-particle terms, and the visits that accepted nothing (leaves
     // and opened cells); accepted nodes are counted per target.
     unsigned long long pp = 0, stopped = 0;
+    // A split walk: the runs kept for the replay, whether the sums so far are
+    // here yet (`direct`), and the targets whose last run ends with the walk.
+    std::uint32_t kept = 0;
+    bool direct = part == 0;
+    std::uint64_t last_run = 0;
+    float* const my_runs = s_runs + (part == 0 ? 0u : part - 1) * (runs * 3u * kLanes) + lane;
+    auto keep_run = [&](WalkTarget& w) {
+        float* const run = my_runs + kept * (3u * kLanes);
+        run[0] = w.px;
+        run[kLanes] = w.py;
+        run[2 * kLanes] = w.pz;
+        ++kept;
+    };
+    // The sums of the parts before this one, then this part's runs so far.
+    auto join_chain = [&] {
+        // Not an atomic load: one in the walk would keep the node records out of
+        // the scalar cache.
+        while (*static_cast<volatile std::uint32_t*>(&s_done[part - 1]) == 0) __builtin_amdgcn_s_sleep(1);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        WalkTarget& w = t[0];
+        if (lane < kLanes) {
+            w.sx = s_chain[0][lane];
+            w.sy = s_chain[1][lane];
+            w.sz = s_chain[2][lane];
+            w.kx = s_chain[3][lane];
+            w.ky = s_chain[4][lane];
+            w.kz = s_chain[5][lane];
+        }
+        for (std::uint32_t e = 0; e < kept; ++e) {
+            const float* const run = my_runs + e * (3u * kLanes);
+            kahan(run[0], w.sx, w.kx);
+            kahan(run[kLanes], w.sy, w.ky);
+            kahan(run[2 * kLanes], w.sz, w.kz);
+        }
+        direct = true;
+    };
     while (true) {
         std::uint32_t own_seg = 0;
         std::uint64_t mask[kR];
@@ -801,79 +929,14 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
         for (int r = 0; r < kR; ++r) st_lo[r] = st_hi[r] = 0;
         std::uint32_t depth = 0, end = 0;  // the outermost list ends nowhere
         std::uint32_t cur = kMany ? __builtin_amdgcn_readfirstlane(first_node[seg_start[own_seg]]) : 0u;
-        // cur only ever grows, so the loop ends whatever the records hold.
-        while (cur < M) {
-            ++steps;
-            const float4 na = nodes[cur].a;
-            const uint4 nb = nodes[cur].b;
-            float4 qa{}, qb{};
-            if constexpr (kQuad) {
-                qa = quads[cur].a;
-                qb = quads[cur].b;
-            }
-            // Every scalar load of the iteration is issued here and waited for once;
-            // left to itself the compiler sinks them into the branches below, one
-            // dependent wait each.
-            asm volatile("" ::"s"(na.x), "s"(na.y), "s"(na.z), "s"(na.w), "s"(nb.x), "s"(nb.y), "s"(nb.z),
-                         "s"(nb.w));
-            if constexpr (kQuad) {
-                asm volatile("" ::"s"(qa.x), "s"(qa.y), "s"(qa.z), "s"(qa.w), "s"(qb.x), "s"(qb.y),
-                             "s"(qb.z), "s"(qb.w));
-            }
-            const float acc = __builtin_bit_cast(float, nb.x);
-            std::uint64_t rest[kR], any = 0;
-#pragma unroll
-            for (int r = 0; r < kR; ++r) {
-                rest[r] = 0;
-                if (kR > 1 && mask[r] == 0) continue;
-                float dx, dy, dz;
-                const float r2 = separation(t[r], na, dx, dy, dz);
-                const std::uint64_t far = __ballot(r2 >= acc) & mask[r];
-                rest[r] = mask[r] & ~far;
-                any |= rest[r];
-                if (__builtin_amdgcn_inverse_ballot_w64(far)) {
-                    accept<kSafe, kQuad>(t[r], na.w, qa, qb, dx, dy, dz, r2, eps2);
-                    ++t[r].pc;
-                }
-            }
-            // The successor when nothing opens: an escape index always lies past its
-            // node; the maximum only keeps a corrupted record from looping.
-            const std::uint32_t step = cur + 1;
-            const std::uint32_t next = max(nb.y, step);
-            std::uint32_t go = next;
-            if (any != 0) {
-                if (nb.w != 0) {
-                    const double4 cb = node_geo[cur];
-                    const std::uint32_t b = nb.z, e = nb.z + nb.w;
-#pragma unroll
-                    for (int r = 0; r < kR; ++r) {
-                        if (rest[r] == 0) continue;
-                        const std::uint32_t here = __popcll(rest[r]);
-                        stopped += here;
-                        pp += static_cast<unsigned long long>(here) * nb.w -
-                              __popcll(__ballot(t[r].own == cur) & rest[r]);
-                        if (__builtin_amdgcn_inverse_ballot_w64(rest[r])) {
-                            leaf_pairs<kSafe>(t[r], cb, s_own[r][0][threadIdx.x], s_own[r][1][threadIdx.x],
-                                              s_own[r][2][threadIdx.x], leaf_rel, b, e, eps2);
-                        }
-                    }
-                } else {
-                    // Open: the children for those that did, then everyone here
-                    // goes on at `next`.
-                    lane_write(st_end, end, depth);
-#pragma unroll
-                    for (int r = 0; r < kR; ++r) {
-                        stopped += __popcll(rest[r]);
-                        lane_write(st_lo[r], static_cast<std::uint32_t>(mask[r]), depth);
-                        lane_write(st_hi[r], static_cast<std::uint32_t>(mask[r] >> 32), depth);
-                        mask[r] = rest[r];
-                    }
-                    ++depth;  // at most 21 levels
-                    end = next;
-                    go = step;
-                }
-            }
-            cur = go;
+        std::uint32_t stop = M;
+        // A split walk: the targets whose current run is this part's, and
+        // those still walking.
+        std::uint64_t open = 0, alive = ~std::uint64_t{0};
+        bool tail = false;
+        std::uint32_t main_steps = 0, main_pc = 0;
+        unsigned long long main_pp = 0, main_stopped = 0;
+        auto up = [&] {
             // The end of one or more sibling lists: back to the masks of the
             // lists they lie in (cur > 0, so never past the outermost).
             while (cur == end) {
@@ -883,15 +946,230 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
                 for (int r = 0; r < kR; ++r) {
                     mask[r] = static_cast<std::uint64_t>(lane_read(st_lo[r], depth)) |
                               static_cast<std::uint64_t>(lane_read(st_hi[r], depth)) << 32;
+                    if constexpr (kSplit > 1) mask[r] &= alive;
                 }
             }
+        };
+        auto open_cell = [&](std::uint32_t next, const std::uint64_t (&rest)[kR]) {
+            lane_write(st_end, end, depth);
+#pragma unroll
+            for (int r = 0; r < kR; ++r) {
+                lane_write(st_lo[r], static_cast<std::uint32_t>(mask[r]), depth);
+                lane_write(st_hi[r], static_cast<std::uint32_t>(mask[r] >> 32), depth);
+                mask[r] = rest[r];
+            }
+            ++depth;  // at most 21 levels
+            end = next;
+        };
+        if constexpr (kSplit > 1) {
+            const std::uint32_t first = static_cast<std::uint32_t>(__builtin_ctzll(mask[0]));
+            const std::uint32_t last = 63u - static_cast<std::uint32_t>(__builtin_clzll(mask[0]));
+            const std::uint32_t at = wave * kLanes + (kSplit == 2 ? first : (first + last) / 2);
+            const std::uint32_t home = __builtin_amdgcn_readfirstlane(leaf_of[at]);
+            const std::uint32_t root = cur;
+            const std::uint32_t system_end = kMany ? seg_start[own_seg + 1] : n;
+            const std::uint32_t node_end =
+                system_end < n ? __builtin_amdgcn_readfirstlane(first_node[system_end]) : M;
+            const float left = walk_weight(static_cast<float>(home - root));
+            const float right = walk_weight(static_cast<float>(node_end - home));
+            // The node at which part k begins.
+            auto cut = [&](std::uint32_t k) {
+                if (kSplit == 2) return home;
+                const float w = (left + right) * static_cast<float>(k) / kSplit - left;
+                const float d = w < 0 ? -walk_reach(-w) : walk_reach(w);
+                const float node = fminf(fmaxf(static_cast<float>(home) + d, static_cast<float>(root)),
+                                         static_cast<float>(node_end));
+                return static_cast<std::uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(node)));
+            };
+            if (part + 1 < kSplit) stop = cut(part + 1);
+            open = part == 0 ? mask[0] : 0;
+            const std::uint32_t begin = part > 0 ? cut(part) : 0u;
+            if (part > 0) {
+                // Down to this part's first node.
+                while (cur < begin) {
+                    const float4 na = nodes[cur].a;
+                    const uint4 nb = nodes[cur].b;
+                    const std::uint32_t next = max(nb.y, cur + 1);
+                    if (next <= begin) {
+                        cur = next;
+                        continue;
+                    }
+                    float dx, dy, dz;
+                    const float r2 = separation(t[0], na, dx, dy, dz);
+                    const std::uint64_t rest[kR] = {mask[0] & ~__ballot(r2 >= __builtin_bit_cast(float, nb.x))};
+                    if (rest[0] == 0) {
+                        cur = next;
+                        up();
+                        break;
+                    }
+                    open_cell(next, rest);
+                    ++cur;
+                }
+                depth = __builtin_amdgcn_readfirstlane(depth);
+                end = __builtin_amdgcn_readfirstlane(end);
+            }
+        }
+        while (true) {
+            // cur only ever grows, so the loop ends whatever the records hold.
+            while (cur < stop) {
+                ++steps;
+                const float4 na = nodes[cur].a;
+                const uint4 nb = nodes[cur].b;
+                float4 qa{}, qb{};
+                if constexpr (kQuad) {
+                    qa = quads[cur].a;
+                    qb = quads[cur].b;
+                }
+                // Every scalar load of the iteration is issued here and waited for once;
+                // left to itself the compiler sinks them into the branches below, one
+                // dependent wait each.
+                asm volatile("" ::"s"(na.x), "s"(na.y), "s"(na.z), "s"(na.w), "s"(nb.x), "s"(nb.y), "s"(nb.z),
+                             "s"(nb.w));
+                if constexpr (kQuad) {
+                    asm volatile("" ::"s"(qa.x), "s"(qa.y), "s"(qa.z), "s"(qa.w), "s"(qb.x), "s"(qb.y),
+                                 "s"(qb.z), "s"(qb.w));
+                }
+                const float acc = __builtin_bit_cast(float, nb.x);
+                std::uint64_t rest[kR], any = 0;
+#pragma unroll
+                for (int r = 0; r < kR; ++r) {
+                    rest[r] = 0;
+                    if (kR > 1 && mask[r] == 0) continue;
+                    float dx, dy, dz;
+                    const float r2 = separation(t[r], na, dx, dy, dz);
+                    const std::uint64_t far = __ballot(r2 >= acc) & mask[r];
+                    rest[r] = mask[r] & ~far;
+                    any |= rest[r];
+                    if (__builtin_amdgcn_inverse_ballot_w64(far)) {
+                        accept<kSafe, kQuad>(t[r], na.w, qa, qb, dx, dy, dz, r2, eps2);
+                        ++t[r].pc;
+                    }
+                }
+                // The successor when nothing opens: an escape index always lies past its
+                // node; the maximum only keeps a corrupted record from looping.
+                const std::uint32_t step = cur + 1;
+                const std::uint32_t next = max(nb.y, step);
+                std::uint32_t go = next;
+                if (any != 0) {
+                    if (nb.w != 0) {
+                        const double4 cb = node_geo[cur];
+                        const std::uint32_t b = nb.z, e = nb.z + nb.w;
+#pragma unroll
+                        for (int r = 0; r < kR; ++r) {
+                            if (rest[r] == 0) continue;
+                            const std::uint32_t here = __popcll(rest[r]);
+                            stopped += here;
+                            pp += static_cast<unsigned long long>(here) * nb.w -
+                                  __popcll(__ballot(t[r].own == cur) & rest[r]);
+                            if (__builtin_amdgcn_inverse_ballot_w64(rest[r])) {
+                                leaf_pairs<kSafe>(t[r], cb, s_own[r][0][slot], s_own[r][1][slot],
+                                                  s_own[r][2][slot], leaf_rel, b, e, eps2, lane0);
+                                if constexpr (kSplit == 1) {
+                                    kahan(t[r]);
+                                } else if (__builtin_amdgcn_inverse_ballot_w64(open)) {
+                                    if (direct) {
+                                        kahan(t[r]);
+                                    } else {
+                                        keep_run(t[r]);
+                                    }
+                                }
+                                t[r].px = t[r].py = t[r].pz = 0.f;
+                            }
+                            if constexpr (kSplit > 1) {
+                                if (tail) {
+                                    open &= ~rest[r];
+                                    alive = open;
+                                    mask[r] &= open;
+                                    if (open == 0) stop = 0;
+                                } else {
+                                    open |= rest[r];
+                                }
+                                if (!direct && __ballot(kept == runs) != 0) {
+                                    join_chain();
+                                }
+                            }
+                        }
+                    } else {
+                        // Open: the children for those that did, then everyone here
+                        // goes on at `next`.
+#pragma unroll
+                        for (int r = 0; r < kR; ++r) stopped += __popcll(rest[r]);
+                        open_cell(next, rest);
+                        go = step;
+                    }
+                }
+                cur = go;
+                up();
+            }
+            if constexpr (kSplit == 1) break;
+            if (tail || part + 1 == kSplit || open == 0) break;
+            // Past this part's nodes: only the runs already open go on, each to
+            // its end. The part that owns these nodes counts them.
+            tail = true;
+            main_steps = steps;
+            main_pp = pp;
+            main_stopped = stopped;
+            main_pc = t[0].pc;
+            alive = open;
+            mask[0] &= open;
+            stop = M;
+        }
+        if constexpr (kSplit > 1) {
+            if (tail) {
+                steps = main_steps;
+                pp = main_pp;
+                stopped = main_stopped;
+                t[0].pc = main_pc;
+            }
+            last_run |= open;
+        }
+    }
+    if constexpr (kSplit > 1) {
+        if (__builtin_amdgcn_inverse_ballot_w64(last_run)) {
+            if (direct) {
+                kahan(t[0]);
+            } else {
+                keep_run(t[0]);
+            }
+        }
+        if (!direct) join_chain();
+    } else {
+#pragma unroll
+        for (int r = 0; r < kR; ++r) kahan(t[r]);
+    }
+    // Counts: a wave inside one system writes its sums to its own slot, summed
+    // per system by walk_counts (atomics on one address would serialise every
+    // wave); a wave spanning systems adds them per system.
+    const unsigned long long pc = accepted(t);
+    unsigned long long count[4] = {pp, pc, pc + stopped, steps};
+    const bool mixed = kMany && systems > 1;
+    if (mixed) {
+        if (lane == 0) add_counts(stats, seg0, pp, pc, pc + stopped, count[3] * (kR * kLanes) / 64);
+        for (int c = 0; c < 4; ++c) count[c] = 0;
+    }
+    if constexpr (kSplit > 1) {
+        if (part + 1 < kSplit) {
+            if (lane < kLanes) {
+                s_chain[0][lane] = t[0].sx;
+                s_chain[1][lane] = t[0].sy;
+                s_chain[2][lane] = t[0].sz;
+                s_chain[3][lane] = t[0].kx;
+                s_chain[4][lane] = t[0].ky;
+                s_chain[5][lane] = t[0].kz;
+            }
+            if (lane == 0) {
+                for (int c = 0; c < 4; ++c) s_count[part][c] = count[c];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            if (lane == 0) *static_cast<volatile std::uint32_t*>(&s_done[part]) = 1;
+            return;
+        }
+        for (int q = 0; q + 1 < kSplit; ++q) {
+            for (int c = 0; c < 4; ++c) count[c] += s_count[q][c];
         }
     }
 #pragma unroll
     for (int r = 0; r < kR; ++r) {
-        kahan(t[r].px, t[r].sx, t[r].kx);
-        kahan(t[r].py, t[r].sy, t[r].ky);
-        kahan(t[r].pz, t[r].sz, t[r].kz);
         const std::uint32_t i = wave * (kLanes * kR) + kLanes * r + lane;
         if (lane < kLanes && i < n) {
             const std::uint32_t dst = index[i];
@@ -900,20 +1178,12 @@ __global__ __launch_bounds__(kBlock) void tree_walk(
             az[dst] = G * (static_cast<double>(t[r].sz) - static_cast<double>(t[r].kz));
         }
     }
-    // Counts: a wave inside one system writes its sums to its own slot, summed
-    // per system by walk_counts (atomics on one address would serialise every
-    // wave); a wave spanning systems adds them per system.
-    unsigned long long* mine_slot = wave_stats + 4 * static_cast<std::size_t>(wave);
-    const unsigned long long pc = accepted(t), visits = pc + stopped;
     if (lane == 0) {
-        // Lane-target slots, 64 per count.
-        const unsigned long long slots = static_cast<unsigned long long>(steps) * (kR * kLanes) / 64;
-        const bool mixed = kMany && systems > 1;
-        if (mixed) add_counts(stats, seg0, pp, pc, visits, slots);
-        mine_slot[0] = mixed ? 0 : pp;
-        mine_slot[1] = mixed ? 0 : pc;
-        mine_slot[2] = mixed ? 0 : visits;
-        mine_slot[3] = mixed ? 0 : slots;
+        unsigned long long* mine_slot = wave_stats + 4 * static_cast<std::size_t>(wave);
+        mine_slot[0] = count[0];
+        mine_slot[1] = count[1];
+        mine_slot[2] = count[2];
+        mine_slot[3] = count[3] * (kR * kLanes) / 64;  // lane-target slots, 64 per count
     }
 }
 
@@ -998,7 +1268,7 @@ std::size_t layout_bytes(std::uint64_t n, std::size_t nodes, bool quadrupole, st
     const std::size_t counters = 16 + 8 * 4 * static_cast<std::size_t>(segments) +
                                  8 * ((n + kBlock - 1) / kBlock) +
                                  32 * (kBlock / 64) * (((64 / kMinLanes) * n + kBlock - 1) / kBlock) + 512;
-    return per_particle + per_node + counters + 22 * 256 + 64;
+    return per_particle + per_node + counters + 22 * 256 + 48;
 }
 
 Layout layout(orr_ctx* ctx, std::uint64_t n, std::size_t nodes, bool quadrupole, std::uint32_t segments,
@@ -1134,44 +1404,55 @@ void tree_enqueue(orr_ctx* ctx, const orr_tree_args& a, const SegmentView& segs,
         // One target a lane at every size (2^21 particles, quadrupoles: 8.3 ms
         // with one or two; below, one is faster); two only when configured.
         const int R = ctx->walk_targets_per_lane != 0 ? ctx->walk_targets_per_lane : 1;
-        // Fewer targets a wave for a small launch (more waves, each over a
-        // tighter group of targets); zero in the context means choose by that
-        // rule. A target's walk and sums do not depend on which targets share
-        // its wave, so the results are the same bits either way.
+        // Fewer targets a wave and several waves a group for a small launch;
+        // zero in the context means choose by that rule. A target's walk and
+        // sums do not depend on which targets share its wave nor on the parts,
+        // so the results are the same bits either way.
         const std::uint64_t full_waves = (n + 64u * R - 1) / (64u * R);
-        const int lanes = ctx->walk_lanes != 0 ? ctx->walk_lanes
-                          : full_waves <= kQuarterLaneWaves && R == 1 ? 16
-                          : full_waves <= kHalfLaneWaves ? 32 : 64;
-        using Walk = decltype(&tree_walk<1, true, true, 64, false>);
-        auto many = [&](auto r, auto l, auto sv, auto q) -> Walk {
-            constexpr int kRr = decltype(r)::value, kLl = decltype(l)::value;
+        const WalkShape shape = ctx->walk_lanes != 0 || R != 1
+                                    ? WalkShape{ctx->walk_lanes != 0 ? ctx->walk_lanes
+                                                : full_waves <= kHalfLaneWaves ? 32 : 64, 1}
+                                    : walk_shape(full_waves);
+        const int lanes = shape.lanes, split = shape.parts;
+        using Walk = decltype(&tree_walk<1, true, true, 64, false, 1>);
+        auto many = [&](auto r, auto l, auto p, auto sv, auto q) -> Walk {
+            constexpr int kRr = decltype(r)::value, kLl = decltype(l)::value, kP = decltype(p)::value;
             constexpr bool kS = decltype(sv)::value, kQ = decltype(q)::value;
-            return seg_of != nullptr ? tree_walk<kRr, kS, kQ, kLl, true> : tree_walk<kRr, kS, kQ, kLl, false>;
+            return seg_of != nullptr ? tree_walk<kRr, kS, kQ, kLl, true, kP>
+                                     : tree_walk<kRr, kS, kQ, kLl, false, kP>;
         };
         using Yes = std::true_type;
         using No = std::false_type;
-        auto pick = [&](auto r, auto l) -> Walk {
-            return safe ? (quad ? many(r, l, Yes{}, Yes{}) : many(r, l, Yes{}, No{}))
-                        : (quad ? many(r, l, No{}, Yes{}) : many(r, l, No{}, No{}));
+        auto pick = [&](auto r, auto l, auto p) -> Walk {
+            return safe ? (quad ? many(r, l, p, Yes{}, Yes{}) : many(r, l, p, Yes{}, No{}))
+                        : (quad ? many(r, l, p, No{}, Yes{}) : many(r, l, p, No{}, No{}));
         };
         using One = std::integral_constant<int, 1>;
         using Two = std::integral_constant<int, 2>;
+        using Four = std::integral_constant<int, 4>;
+        using Eight = std::integral_constant<int, 8>;
         using Quarter = std::integral_constant<int, 16>;
         using Half = std::integral_constant<int, 32>;
         using Full = std::integral_constant<int, 64>;
-        const Walk walk = R == 2 ? (lanes == 32 ? pick(Two{}, Half{}) : pick(Two{}, Full{}))
-                                 : (lanes == 16 ? pick(One{}, Quarter{})
-                                                : lanes == 32 ? pick(One{}, Half{}) : pick(One{}, Full{}));
+        const Walk walk = R == 2         ? (lanes == 32 ? pick(Two{}, Half{}, One{}) : pick(Two{}, Full{}, One{}))
+                          : split == 8   ? pick(One{}, Quarter{}, Eight{})
+                          : split == 4   ? pick(One{}, Quarter{}, Four{})
+                          : split == 2   ? pick(One{}, Half{}, Two{})
+                          : lanes == 32  ? pick(One{}, Half{}, One{})
+                                         : pick(One{}, Full{}, One{});
         const std::uint32_t per_wave = static_cast<std::uint32_t>(lanes * R);
-        const std::uint32_t per_block = (kBlock / 64) * per_wave;
+        const std::uint32_t groups = split == 1 ? kBlock / 64 : 1;  // a block
+        const std::uint32_t per_block = groups * per_wave;
         const std::uint32_t walk_blocks = (n32 + per_block - 1) / per_block;
-        hipLaunchKernelGGL(walk, dim3(walk_blocks), dim3(kBlock), 0, ctx->stream, L.walk, L.quadf,
-                           L.geo, L.root_rel, L.leaf_rel, L.leaf_of, index, L.c32, seg_of,
-                           seg_start, L.first_node, n32, eps2, a.gravitational_constant, a.ax,
+        const std::uint32_t run_bytes = 12u * static_cast<std::uint32_t>(lanes * (split - 1));
+        const std::uint32_t runs = split == 1 ? 0 : split_runs(walk_blocks, run_bytes);
+        hipLaunchKernelGGL(walk, dim3(walk_blocks), dim3(split == 1 ? kBlock : 64 * split),
+                           static_cast<std::size_t>(runs) * run_bytes, ctx->stream, L.walk, L.quadf, L.geo, L.root_rel, L.leaf_rel, L.leaf_of, index, L.c32, seg_of,
+                           seg_start, L.first_node, n32, eps2, a.gravitational_constant, runs, a.ax,
                            a.ay, a.az, counts64, L.wave_stats);
         ORR_LAUNCHED("tree_walk");
         hipLaunchKernelGGL(walk_counts, dim3(segs.count), dim3(kBlock), 0, ctx->stream,
-                           L.wave_stats, walk_blocks * (kBlock / 64), per_wave, seg_start, counts64);
+                           L.wave_stats, walk_blocks * groups, per_wave, seg_start, counts64);
         ORR_LAUNCHED("walk_counts");
     }
 }

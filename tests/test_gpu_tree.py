@@ -360,6 +360,31 @@ def test_replayed_evaluations_are_bitwise(ctx):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,leaf,theta", [
+    (3, 1, 0.0), (17, 1, 0.6), (300, 1, 0.0), (3000, 1, 0.0), (3000, 1, 0.3),  # far more runs than a part has room for
+    (8192, 8, 0.5), (8193, 8, 0.5), (24576, 4, 0.5), (24577, 4, 0.5), (30000, 1, 0.5),
+    (73728, 32, 0.7), (73729, 32, 0.7), (102400, 32, 0.7), (102401, 32, 0.7)])
+def test_walk_in_parts_is_the_walk_in_one(ctx, n, leaf, theta):
+    """Eight, four and two waves a group of targets against one: the same accelerations
+    and counts bit for bit, on both sides of each line between them, in ragged last
+    groups, and where the parts run out of room and wait for one another."""
+    p = oracle.disc_collision(n, 11) if n % 2 else oracle.plummer(n, 11)
+    out = []
+    try:
+        for lanes in (-1, 64):
+            ctx.set_tree_config(lanes=lanes)
+            s = E.HipTreeSolver(E.TreeParameters(theta, leaf, quadrupole=n < 10000), E.Softening(0.01), context=ctx)
+            a = [np.zeros(n) for _ in range(3)]
+            s.evaluate((p.x, p.y, p.z), p.m, a)
+            c = s.interaction_count()
+            out.append((np.stack(a), c.particle_particle, c.particle_cell, s.node_visits()))
+    finally:
+        ctx.set_tree_config(lanes=-1)
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("quadrupole", [False, True])
 @pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 65, 1000, 16384, 16385, 131072, 131073])
 def test_waves_chosen_by_size_walk_as_full_waves(ctx, n, quadrupole):
