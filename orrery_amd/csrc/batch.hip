@@ -43,7 +43,7 @@ namespace orr {
 namespace {
 
 constexpr std::uint32_t kTile = 64;
-constexpr std::uint32_t kChunk = 2048;  // particles per bounding-box chunk
+constexpr std::uint32_t kChunk = kSystemChunk;  // particles per bounding-box chunk
 
 // v += scale[system] a, the kick of integrators/velocity_verlet.cpp:20-38 (one
 // multiply, one add, unfused) with each particle's own system's scale. Tree
@@ -103,6 +103,7 @@ struct orr_batch {
     std::uint32_t *dstart = nullptr, *dchunks = nullptr, *dchunk_first = nullptr;
     std::uint32_t *tstart = nullptr, *tchunks = nullptr, *tchunk_first = nullptr;
     std::uint32_t dchunk_count = 0, tchunk_count = 0;
+    std::uint64_t dlongest = 0, tlongest = 0;  // particles of the largest system of each branch
     std::uint32_t tiles = 0, items = 0, slots = 0;
     std::uint64_t direct_pairs = 0;
     bool safe = false;
@@ -163,6 +164,7 @@ void plan(orr_batch* b) {
     std::vector<std::uint32_t> dchunks, tchunks, dchunk_first(b->D + 1), tchunk_first(b->T + 1);
 
     b->direct_pairs = 0;
+    b->dlongest = b->tlongest = 0;
     b->safe = false;
     std::uint32_t slots = 0;
     for (std::uint32_t s = 0; s < S; ++s) {
@@ -189,6 +191,8 @@ void plan(orr_batch* b) {
             chunks.push_back(static_cast<std::uint32_t>(c - base));
             chunks.push_back(static_cast<std::uint32_t>(std::min(end, c + kChunk) - base));
         }
+        std::uint64_t& longest = direct ? b->dlongest : b->tlongest;
+        longest = std::max(longest, end - begin);
         chunk_first[local + 1] = static_cast<std::uint32_t>(chunks.size() / 3);
         if (!direct) {
             tstart[local] = static_cast<std::uint32_t>(begin - base);
@@ -283,7 +287,8 @@ void kick_all(orr_batch* b, const double* scale, double* v0, double* v1, double*
 void evaluate_direct(orr_batch* b) {
     if (b->n_direct == 0) return;
     orr_ctx* ctx = b->dctx;
-    const SegmentView segs{b->D, b->dstart, b->seg_of, b->dchunks, b->dchunk_first, b->dchunk_count};
+    const SegmentView segs{b->D, b->dstart, b->seg_of, b->dchunks, b->dchunk_first, b->dchunk_count,
+                           b->dlongest};
     morton_enqueue_segments(ctx, b->array(0), b->array(1), b->array(2), b->n_direct, segs);
     DirectBatchView v;
     v.count = b->n_direct;
@@ -321,7 +326,7 @@ void evaluate_tree(orr_batch* b) {
     a.leaf_capacity = b->leaf_capacity;
     a.quadrupole = b->cfg.quadrupole;
     const SegmentView segs{b->T, b->tstart, b->seg_of + base, b->tchunks, b->tchunk_first,
-                           b->tchunk_count};
+                           b->tchunk_count, b->tlongest};
     tree_evaluate_segments(b->tctx, a, segs, nullptr, nullptr);
 }
 

@@ -300,10 +300,12 @@ struct SegmentView {
     std::uint32_t count = 1;
     const std::uint32_t* start = nullptr;        // [count + 1] first particle of each system
     const std::uint32_t* seg_of = nullptr;       // [n] system of each particle
-    const std::uint32_t* chunks = nullptr;       // [chunk_count][3] {system, begin, end}
+    const std::uint32_t* chunks = nullptr;       // [chunk_count][3] {system, begin, end}, kSystemChunk each but a system's last
     const std::uint32_t* chunk_first = nullptr;  // [count + 1] first chunk of each system
     std::uint32_t chunk_count = 0;
+    std::uint64_t longest = 0;                   // particles of the largest system (0: not known)
 };
+constexpr std::uint32_t kSystemChunk = 2048;
 
 // morton.hip, segmented: one cube per system (cubes at ctx->order_bbox[4 * s]),
 // order by (system, code, index). Systems keep their particle ranges. With

@@ -10,7 +10,8 @@
 //   * a stable LSD radix sort starting from identity order reproduces the
 //     (code, index) lexicographic total order (morton.hpp:155-175).
 //
-// Sort: 8 passes of 8-bit digits. By default one launch counts the digits of
+// Sort: systems of up to kMergeOrder particles in chunks sorted in LDS and merged
+// by rank; larger ones in 8 passes of 8-bit digits. By default one launch counts the digits of
 // every pass and each pass is one scatter that finds the blocks before it by
 // decoupled look-back; the multi-kernel form (per pass: histogram -> device-wide
 // exclusive scan -> scatter) gives the same permutation and stays selectable.
@@ -21,6 +22,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 #include <utility>
 
 #include "engine.hpp"
@@ -573,9 +575,264 @@ __global__ __launch_bounds__(kBlock) void radix_onesweep(const std::uint64_t* __
     }
 }
 
+// ---- chunks sorted in LDS, merged by rank -----------------------------------------
+//
+// Up to kMergeOrder particles a system, the eight to ten radix passes (12 to 19 us
+// each, bound by their own latency) become two launches. One workgroup
+// computes the codes of a chunk of kChunkKeys particles and sorts them in LDS;
+// then every key's position is its own rank plus the number of keys that each
+// other chunk of its system holds before it, found by binary search: equal
+// codes count where their chunk, and so their index, comes first. The order
+// is the radix passes': (system, code, index).
+constexpr int kChunkThreads = 1024;
+constexpr std::uint32_t kChunkKeys = 2 * kChunkThreads;
+static_assert(kChunkKeys == kSystemChunk);
+// Two chunks' searches cost as much at any size, so the merge grows as the
+// square of a system, the passes hardly: cube, codes and order, ms, merged
+// against passes: 4096 particles 0.034 against 0.115, 16,384 0.034 and 0.117,
+// 65,536 0.059 and 0.13, 98,304 0.080 and 0.155, 196,608 0.149 and some 0.17,
+// 262,144 0.227 and 0.199.
+constexpr std::uint32_t kMergeOrder = 196608;
+
+// The value of the lane whose number differs by kMask, within a wave.
+template<int kMask>
+__device__ __forceinline__ std::uint32_t xor_lane(std::uint32_t v) {
+    auto dpp = [](std::uint32_t u, auto ctrl) {
+        return static_cast<std::uint32_t>(
+            __builtin_amdgcn_mov_dpp(static_cast<int>(u), decltype(ctrl)::value, 0xf, 0xf, true));
+    };
+    if constexpr (kMask == 1) return dpp(v, std::integral_constant<int, 0xb1>{});    // quad_perm 1,0,3,2
+    else if constexpr (kMask == 2) return dpp(v, std::integral_constant<int, 0x4e>{});  // quad_perm 2,3,0,1
+    else if constexpr (kMask == 3) return dpp(v, std::integral_constant<int, 0x1b>{});  // quad_perm 3,2,1,0
+    else if constexpr (kMask == 7) return dpp(v, std::integral_constant<int, 0x141>{});   // row_half_mirror
+    else if constexpr (kMask == 8) return dpp(v, std::integral_constant<int, 0x128>{});   // row_ror 8
+    else if constexpr (kMask == 15) return dpp(v, std::integral_constant<int, 0x140>{});  // row_mirror
+    else if constexpr (kMask == 4) return xor_lane<7>(xor_lane<3>(v));
+    else return static_cast<std::uint32_t>(__shfl_xor(static_cast<int>(v), kMask, 64));
+}
+template<int kMask>
+__device__ __forceinline__ std::uint64_t xor_lane(std::uint64_t v) {
+    return static_cast<std::uint64_t>(xor_lane<kMask>(static_cast<std::uint32_t>(v >> 32))) << 32 |
+           xor_lane<kMask>(static_cast<std::uint32_t>(v));
+}
+
+// Elements 2 t (a) and 2 t + 1 (b) of thread t, kChunkKeys in all, ascending: a
+// bitonic network whose comparators all point the same way. A merge of runs of
+// kRun / 2 starts by comparing element i with i ^ (kRun - 1), then i ^ j for j =
+// kRun / 4 down to 1. Threads less than a wave apart exchange through lane moves,
+// the rest (10 of 66 stages) through `swap`, in LDS.
+template<int kMask>
+__device__ __forceinline__ void sort_stage(std::uint64_t& a, std::uint64_t& b, bool crossed,
+                                           std::uint64_t* swap) {
+    const std::uint32_t t = threadIdx.x;
+    // The lower of two threads keeps the smaller keys; they differ first in the top bit of the mask.
+    constexpr std::uint32_t kTop = 1u << (31 - __builtin_clz(static_cast<unsigned>(kMask)));
+    const bool low = (t & kTop) == 0;
+    std::uint64_t pa, pb;
+    if constexpr (kMask < 64) {
+        pa = xor_lane<kMask>(a);
+        pb = xor_lane<kMask>(b);
+    } else {
+        __syncthreads();
+        swap[t] = a;
+        swap[kChunkThreads + t] = b;
+        __syncthreads();
+        pa = swap[t ^ kMask];
+        pb = swap[kChunkThreads + (t ^ kMask)];
+    }
+    const std::uint64_t oa = crossed ? pb : pa, ob = crossed ? pa : pb;
+    a = (oa < a) == low ? oa : a;
+    b = (ob < b) == low ? ob : b;
+}
+__device__ __forceinline__ void sort_two(std::uint64_t& a, std::uint64_t& b) {
+    const std::uint64_t lo = a < b ? a : b, hi = a < b ? b : a;
+    a = lo;
+    b = hi;
+}
+template<int kStride>  // in threads
+__device__ __forceinline__ void half_cleaners(std::uint64_t& a, std::uint64_t& b, std::uint64_t* swap) {
+    if constexpr (kStride >= 1) {
+        sort_stage<kStride>(a, b, false, swap);
+        half_cleaners<kStride / 2>(a, b, swap);
+    }
+}
+template<int kRun>
+__device__ __forceinline__ void merge_runs(std::uint64_t& a, std::uint64_t& b, std::uint64_t* swap) {
+    if constexpr (kRun > 2) {
+        merge_runs<kRun / 2>(a, b, swap);
+        sort_stage<kRun / 2 - 1>(a, b, true, swap);
+        half_cleaners<kRun / 8>(a, b, swap);
+    }
+    sort_two(a, b);
+}
+
+// Block b: the codes of chunk b's particles, sorted, at the chunk's own place in
+// keys and vals. `below` masks the code bits the order leaves out.
+//
+// A key in the network is the upper 53 bits of a code above the particle's place
+// in the chunk, so keys are distinct and need no payload. Codes that differ
+// only below those bits (cells 2^-17.7 of the cube) are put right after, if any are out of
+// order, by sorting once more by (first position of the equal 53 bits, lower bits, place).
+__global__ __launch_bounds__(kChunkThreads) void chunk_sort(
+    const double* __restrict__ x, const double* __restrict__ y, const double* __restrict__ z,
+    const double* __restrict__ m, std::uint32_t n, const double* __restrict__ partial,
+    std::uint32_t partials, const std::uint32_t* __restrict__ chunks,
+    const std::uint32_t* __restrict__ chunk_first, std::uint64_t below, double* __restrict__ cubes,
+    std::uint64_t* __restrict__ keys, std::uint32_t* __restrict__ vals, double4* __restrict__ aos) {
+    constexpr std::uint32_t kPlaceBits = 11, kLowBits = 10;
+    static_assert(kChunkKeys == 1u << kPlaceBits);
+    __shared__ std::uint64_t s_code[kChunkKeys];
+    __shared__ std::uint64_t s_swap[kChunkKeys];
+    __shared__ double s_cube[4];
+    __shared__ double s_box[6];
+    __shared__ std::uint32_t s_fix;
+    const std::uint32_t t = threadIdx.x;
+    std::uint32_t seg = 0, begin = blockIdx.x * kChunkKeys, end = min(n, begin + kChunkKeys);
+    std::uint32_t p0 = 0, p1 = partials;
+    if (chunks != nullptr) {
+        seg = chunks[3 * blockIdx.x];
+        begin = chunks[3 * blockIdx.x + 1];
+        end = chunks[3 * blockIdx.x + 2];
+        p0 = chunk_first[seg];
+        p1 = chunk_first[seg + 1];
+    }
+    const std::uint32_t count = end - begin;
+    // The system's extrema from its partial ones (exact, in any order), 32 threads a component.
+    if (t < 6 * 32) {
+        const std::uint32_t c = t / 32;
+        const double inf = __builtin_huge_val();
+        double v = c < 3 ? inf : -inf;
+        for (std::uint32_t p = p0 + t % 32; p < p1; p += 32) {
+            const double w = partial[6 * static_cast<std::size_t>(p) + c];
+            v = (c < 3 ? w < v : w > v) ? w : v;
+        }
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) {
+            const double w = __shfl_xor(v, off, 64);
+            v = (c < 3 ? w < v : w > v) ? w : v;
+        }
+        if (t % 32 == 0) s_box[c] = v;
+    }
+    if (t == 0) s_fix = 0;
+    __syncthreads();
+    if (t == 0) {
+        make_cube(s_box, s_box + 3, s_cube);
+        if (begin == (chunks != nullptr ? chunks[3 * p0 + 1] : 0u)) {
+            for (int c = 0; c < 4; ++c) cubes[4 * static_cast<std::size_t>(seg) + c] = s_cube[c];
+        }
+    }
+    __syncthreads();
+    const double size = s_cube[3];
+    const double scale = static_cast<double>(kGrid) / size;
+    std::uint64_t a = ~0ull, b = ~0ull;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const std::uint32_t place = t + r * kChunkThreads;
+        if (place >= count) continue;
+        const std::size_t i = static_cast<std::size_t>(begin) + place;
+        const double px = x[i], py = y[i], pz = z[i];
+        std::uint64_t code = 0;
+        if (size > 0) {
+            code = (spread_bits(to_grid(px, s_cube[0], scale)) << 2) |
+                   (spread_bits(to_grid(py, s_cube[1], scale)) << 1) | spread_bits(to_grid(pz, s_cube[2], scale));
+        }
+        if (aos != nullptr) aos[i] = make_double4(px, py, pz, m[i]);
+        code &= ~below;
+        s_code[place] = code;
+        (r == 0 ? a : b) = (code >> kLowBits) << kPlaceBits | place;
+    }
+    merge_runs<kChunkKeys>(a, b, s_swap);
+    constexpr std::uint64_t kPlaceMask = kChunkKeys - 1;
+    constexpr std::uint32_t kLowMask = (1u << kLowBits) - 1;
+    auto low_of = [&](std::uint64_t key) {
+        return static_cast<std::uint32_t>(s_code[key & kPlaceMask]) & kLowMask;
+    };
+    __syncthreads();
+    s_swap[2 * t] = a;
+    s_swap[2 * t + 1] = b;
+    __syncthreads();
+    // Pads (all ones) lie past the last key.
+    auto out_of_order = [&](std::uint64_t u, std::uint64_t v) {
+        return u >> kPlaceBits == v >> kPlaceBits && low_of(u) > low_of(v);
+    };
+    if ((2 * t + 1 < count && out_of_order(a, b)) ||
+        (2 * t + 2 < count && out_of_order(b, s_swap[2 * t + 2]))) {
+        s_fix = 1;
+    }
+    __syncthreads();
+    if (s_fix != 0) {
+        auto again = [&](std::uint64_t key, std::uint32_t at) -> std::uint64_t {
+            if (at >= count) return ~std::uint64_t{0};
+            const std::uint64_t run = key & ~kPlaceMask;
+            std::uint32_t first = 0;  // keys below the run
+            for (std::uint32_t step = kChunkKeys / 2; step > 0; step >>= 1) {
+                if (s_swap[first + step - 1] < run) first += step;
+            }
+            return static_cast<std::uint64_t>(first) << (kLowBits + kPlaceBits) |
+                   static_cast<std::uint64_t>(low_of(key)) << kPlaceBits | (key & kPlaceMask);
+        };
+        a = again(a, 2 * t);
+        b = again(b, 2 * t + 1);
+        __syncthreads();
+        merge_runs<kChunkKeys>(a, b, s_swap);
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const std::uint32_t at = 2 * t + r;
+        if (at >= count) continue;
+        const std::uint32_t place = static_cast<std::uint32_t>((r == 0 ? a : b) & kPlaceMask);
+        keys[static_cast<std::size_t>(begin) + at] = s_code[place];
+        vals[static_cast<std::size_t>(begin) + at] = begin + place;
+    }
+}
+
+// Every key to its position in its system: one thread a key, the searches of
+// kMergeAhead chunks on their way together.
+constexpr int kMergeAhead = 8;
+__global__ __launch_bounds__(kBlock) void chunk_merge(
+    const std::uint64_t* __restrict__ keys_in, const std::uint32_t* __restrict__ vals_in, std::uint32_t n,
+    const std::uint32_t* __restrict__ seg_of, const std::uint32_t* __restrict__ seg_start,
+    std::uint64_t* __restrict__ keys_out, std::uint32_t* __restrict__ vals_out) {
+    const std::uint32_t p = blockIdx.x * kBlock + threadIdx.x;
+    if (p >= n) return;
+    std::uint32_t lo = 0, hi = n;
+    if (seg_of != nullptr) {
+        const std::uint32_t seg = seg_of[p];
+        lo = seg_start[seg];
+        hi = seg_start[seg + 1];
+    }
+    const std::uint64_t key = keys_in[p];
+    const std::uint32_t val = vals_in[p];
+    const std::uint32_t own = (p - lo) / kChunkKeys, chunks = (hi - lo + kChunkKeys - 1) / kChunkKeys;
+    std::uint32_t position = lo + (p - lo) % kChunkKeys;
+    for (std::uint32_t c = 0; c < chunks; c += kMergeAhead) {
+        std::uint32_t found[kMergeAhead], begin[kMergeAhead], length[kMergeAhead];
+#pragma unroll
+        for (int u = 0; u < kMergeAhead; ++u) {
+            found[u] = 0;
+            begin[u] = lo + (c + u) * kChunkKeys;
+            length[u] = c + u >= chunks || c + u == own ? 0 : min(hi - begin[u], kChunkKeys);
+        }
+        for (std::uint32_t step = kChunkKeys; step > 0; step >>= 1) {
+#pragma unroll
+            for (int u = 0; u < kMergeAhead; ++u) {
+                // Past the chunk's end: any key, and no step. No branch, so that the loads overlap.
+                const bool inside = found[u] + step <= length[u];
+                const std::uint64_t other = keys_in[inside ? begin[u] + found[u] + step - 1 : p];
+                const bool before = c + u < own ? other <= key : other < key;
+                found[u] += inside && before ? step : 0;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kMergeAhead; ++u) position += found[u];
+    }
+    keys_out[position] = key;
+    vals_out[position] = val;
+}
+
 // ---- small systems: order by rank ------------------------------------------------
 //
-// The multi-kernel order is a stable sort by the codes' digits from first_digit
+// The order is a stable sort by the codes' digits from first_digit
 // up, that is a sort by (code >> 8 first_digit, index): a key unique per
 // element, whose position is the number of smaller keys. Counting them is n^2
 // compares, 32 bits wide where first_digit >= 4, with no dependence between
@@ -815,19 +1072,26 @@ int morton_enqueue_into(orr_ctx* ctx, const double* x, const double* y, const do
     const std::uint32_t sort_blocks = sz.sort_blocks;
     double* cube = b.bbox;  // cubes[4 * segment]
     double* partial = cube + 4 * static_cast<std::size_t>(segs.count);
+    const std::uint64_t longest = segmented ? segs.longest : n;
+    const bool merged = ctx->sort_mode == 1 && longest > 0 && longest <= kMergeOrder;
     {
         PhaseTimer t(ctx, kBbox, timed);
         if (segmented) {
             hipLaunchKernelGGL(bbox_chunks, dim3(segs.chunk_count), dim3(kBlock), 0, ctx->stream, x, y,
                                z, segs.chunks, partial);
             ORR_LAUNCHED("bbox_chunks");
+        }
+        if (segmented && !merged) {
             hipLaunchKernelGGL(bbox_segments, dim3((segs.count + kBlock - 1) / kBlock), dim3(kBlock), 0,
                                ctx->stream, partial, segs.chunk_first, segs.count, cube);
             ORR_LAUNCHED("bbox_segments");
-        } else {
+        }
+        if (!segmented) {
             hipLaunchKernelGGL(bbox_partial, dim3(bbox_blocks), dim3(kBlock), 0, ctx->stream, x, y, z,
                                n, partial);
             ORR_LAUNCHED("bbox_partial");
+        }
+        if (!segmented && !merged) {
             hipLaunchKernelGGL(bbox_final, dim3(1), dim3(kBlock), 0, ctx->stream, partial,
                                bbox_blocks, cube);
             ORR_LAUNCHED("bbox_final");
@@ -836,6 +1100,26 @@ int morton_enqueue_into(orr_ctx* ctx, const double* x, const double* y, const do
     std::uint64_t* const* keys = b.codes;
     std::uint32_t* const* vals = b.index;
     const std::uint32_t* seg_of = segmented ? segs.seg_of : nullptr;
+    if (merged) {
+        const std::uint32_t n32 = static_cast<std::uint32_t>(n);
+        const std::uint32_t chunk_count = segmented ? segs.chunk_count : (n32 + kChunkKeys - 1) / kChunkKeys;
+        const bool one_each = longest <= kChunkKeys;
+        {
+            PhaseTimer t(ctx, kEncode, timed);
+            hipLaunchKernelGGL(chunk_sort, dim3(chunk_count), dim3(kChunkThreads), 0, ctx->stream, x, y, z, m, n32,
+                               partial, bbox_blocks, segmented ? segs.chunks : nullptr, segs.chunk_first,
+                               (std::uint64_t{1} << (8 * first_digit)) - 1, cube, keys[one_each ? 0 : 1],
+                               vals[one_each ? 0 : 1], m != nullptr ? b.aos : nullptr);
+            ORR_LAUNCHED("chunk_sort");
+        }
+        PhaseTimer t(ctx, kSort, timed);
+        if (!one_each) {
+            hipLaunchKernelGGL(chunk_merge, dim3((n32 + kBlock - 1) / kBlock), dim3(kBlock), 0, ctx->stream,
+                               keys[1], vals[1], n32, seg_of, segs.start, keys[0], vals[0]);
+            ORR_LAUNCHED("chunk_merge");
+        }
+        return 0;
+    }
     {
         PhaseTimer t(ctx, kEncode, timed);
         hipLaunchKernelGGL(encode, dim3(static_cast<std::uint32_t>((n + kBlock - 1) / kBlock)),

@@ -84,3 +84,36 @@ def test_one_sweep_beyond_resident_blocks(ctx):
     n = 8_388_608
     x, y, z = (rng.standard_normal(n) for _ in range(3))
     check(ctx, x, y, z)
+
+
+@pytest.mark.parametrize("n,spread,corners", [
+    (2048, 0.0, 0), (2048, 2.0**-19, 2), (2047, 2.0**-20, 2), (4100, 2.0**-19, 2), (4100, 2.0**-18, 300),
+    (20000, 2.0**-19, 9000), (6145, 0.0, 1), (196608, 1.0, 0), (196609, 1.0, 0), (90001, 2.0**-19, 50000)])
+def test_chunks_merged_by_rank(ctx, n, spread, corners):
+    """Codes that agree in their upper 53 bits and differ below, or not at all, inside a
+    chunk and across chunks; pads in the last chunk; both sides of the line to the passes."""
+    rng = np.random.default_rng(n)
+    pts = 0.3 + spread * rng.random((n, 3))
+    at = rng.permutation(n)[:corners]
+    pts[at] = rng.random((corners, 3))
+    if corners > 1:
+        pts[at[0]] = 0.0
+        pts[at[1]] = 1.0
+    check(ctx, *(np.ascontiguousarray(pts[:, k]) for k in range(3)))
+
+
+@pytest.mark.parametrize("n", [20481, 65537, 196608])
+def test_order_by_top_digits_either_way(ctx, n):
+    """The direct sum orders by a code's upper half and index: the same sums bit for bit from either sort."""
+    p = oracle.disc_collision(n, 5)
+    out = []
+    try:
+        for mode in (1, 2):
+            ctx.set_tree_config(sort_mode=mode)
+            s = E.HipDirectSolver(E.Softening(0.01), context=ctx)
+            a = [np.zeros(n) for _ in range(3)]
+            s.evaluate((p.x, p.y, p.z), p.m, a)
+            out.append(np.stack(a))
+    finally:
+        ctx.set_tree_config(sort_mode=1)
+    np.testing.assert_array_equal(out[0], out[1])
