@@ -80,19 +80,21 @@ struct QuadF {
 __device__ inline std::uint32_t grid_stride_start() { return blockIdx.x * blockDim.x + threadIdx.x; }
 __device__ inline std::uint32_t grid_stride_step() { return gridDim.x * blockDim.x; }
 
-__global__ void clear_counters(std::uint32_t* __restrict__ c32, unsigned long long* __restrict__ c64,
-                               std::uint32_t count64) {
-    if (threadIdx.x < 4) c32[threadIdx.x] = 0;
-    if (c64 != nullptr) {
-        for (std::uint32_t k = threadIdx.x; k < count64; k += blockDim.x) c64[k] = 0;
-    }
-}
-
 // d(k) from adjacent sorted codes; 0 where a system starts (each system of a
-// batch is its own tree, and a level-0 boundary ends every window at it).
+// batch is its own tree, and a level-0 boundary ends every window at it). The
+// first block also clears the counters of the launches to come.
 __global__ __launch_bounds__(kBlock) void tree_levels(const std::uint64_t* __restrict__ codes,
                                                       const std::uint32_t* __restrict__ seg_of,
-                                                      std::uint32_t n, std::uint8_t* __restrict__ d) {
+                                                      std::uint32_t n, std::uint8_t* __restrict__ d,
+                                                      std::uint32_t* __restrict__ c32,
+                                                      unsigned long long* __restrict__ c64,
+                                                      std::uint32_t count64) {
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < 4) c32[threadIdx.x] = 0;
+        if (c64 != nullptr) {
+            for (std::uint32_t k = threadIdx.x; k < count64; k += kBlock) c64[k] = 0;
+        }
+    }
     const std::uint32_t k = blockIdx.x * kBlock + threadIdx.x;
     if (k >= n) return;
     if (k == 0 || (seg_of != nullptr && seg_of[k] != seg_of[k - 1])) {
@@ -230,9 +232,8 @@ __global__ __launch_bounds__(kBlock) void tree_chains(
 }
 
 // One block: leaf count and depth from the per-block slots.
-__global__ __launch_bounds__(kBlock) void tree_counts(const uint2* __restrict__ block_counts,
-                                                      std::uint32_t blocks,
-                                                      std::uint32_t* __restrict__ counters) {
+__device__ void tree_counts(const uint2* __restrict__ block_counts, std::uint32_t blocks,
+                            std::uint32_t* __restrict__ counters) {
     __shared__ unsigned s_total[kBlock], s_deep[kBlock];
     unsigned total = 0, deep = 0;
     for (std::uint32_t b = threadIdx.x; b < blocks; b += kBlock) {
@@ -327,12 +328,24 @@ __device__ inline std::uint32_t walk_escape(std::uint32_t next, std::uint32_t ce
     return cell_end >= system_end ? 0xffffffffu : next;
 }
 
+// A value that another workgroup of the same launch reads (on any XCD): stored
+// past this XCD's L2, and loaded past the reader's.
+__device__ __forceinline__ void share(double* p, double v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double shared_value(const double* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ inline void finish_node(std::uint32_t node, double mass, double cx, double cy, double cz,
                                    const double4 geo, double theta, const double* __restrict__ cube,
                                    bool leaf, std::uint32_t begin, std::uint32_t count,
                                    std::uint32_t next, double4* __restrict__ moment,
                                    WalkNode* __restrict__ walk) {
-    moment[node] = make_double4(cx, cy, cz, mass);
+    share(&moment[node].x, cx);
+    share(&moment[node].y, cy);
+    share(&moment[node].z, cz);
+    share(&moment[node].w, mass);
     // octree.cpp:370-371 and :374-387.
     const double ox = cx - geo.x, oy = cy - geo.y, oz = cz - geo.z;
     const double offset = sqrt((ox * ox) + (oy * oy) + (oz * oz));
@@ -367,7 +380,7 @@ __device__ inline void add_displaced(double q[6], double mass, double dx, double
 
 __device__ inline void store_quad(std::uint32_t node, const double q[6], double* __restrict__ quad64,
                                   QuadF* __restrict__ quadf) {
-    for (int k = 0; k < 6; ++k) quad64[6 * static_cast<std::size_t>(node) + k] = q[k];
+    for (int k = 0; k < 6; ++k) share(&quad64[6 * static_cast<std::size_t>(node) + k], q[k]);
     QuadF f;
     f.a = make_float4(static_cast<float>(q[0]), static_cast<float>(q[1]), static_cast<float>(q[2]),
                       static_cast<float>(q[3]));
@@ -375,17 +388,137 @@ __device__ inline void store_quad(std::uint32_t node, const double q[6], double*
     quadf[node] = f;
 }
 
-// octree.cpp:91-135 (leaf): index-order sums, fallback to the first particle;
-// with quadrupoles, the displaced moments of the particles about the centre of mass.
-__global__ __launch_bounds__(kBlock) void leaf_moments(
+// Every internal node's children in DFS order (the next chain from node + 1 to
+// the node's own next), side by side for the moments, and what the climb
+// needs: the parent of every node, and how many children an internal node
+// still waits for. These two lie in memory nothing else uses yet: an internal
+// node's moment (the parent in the first word, the count in the second), a
+// leaf's row of `children`. The last block sums the leaf counts meanwhile.
+__device__ __forceinline__ std::uint32_t* link_words(double4* moment, std::uint32_t node) {
+    return reinterpret_cast<std::uint32_t*>(&moment[node]);
+}
+__global__ __launch_bounds__(kBlock) void tree_links(
+    std::uint32_t* __restrict__ counters, const std::uint8_t* __restrict__ node_level,
+    const std::uint8_t* __restrict__ leaf_level_of_first, const std::uint32_t* __restrict__ node_begin,
+    const std::uint32_t* __restrict__ node_next, const uint2* __restrict__ block_counts,
+    std::uint32_t blocks, std::uint32_t* __restrict__ children, double4* __restrict__ moment) {
+    if (blockIdx.x + 1 == gridDim.x) {
+        tree_counts(block_counts, blocks, counters);
+        return;
+    }
+    const std::uint32_t M = counters[0];
+    const std::uint32_t stride = (gridDim.x - 1) * kBlock;
+    for (std::uint32_t node = grid_stride_start(); node < M; node += stride) {
+        const unsigned level = node_level[node];
+        const bool leaf = level == leaf_level_of_first[node_begin[node]];
+        std::uint32_t* const row = children + static_cast<std::size_t>(kMaxChildren) * node;
+        if (level == 0) *(leaf ? row : link_words(moment, node)) = kNoChild;
+        if (leaf) continue;
+        const std::uint32_t end = node_next[node];
+        std::uint32_t k = 0;
+        for (std::uint32_t c = node + 1; c < end && k < kMaxChildren; c = max(node_next[c], c + 1)) {
+            row[k++] = c;
+            const bool leaf_child = node_level[c] == leaf_level_of_first[node_begin[c]];
+            *(leaf_child ? children + static_cast<std::size_t>(kMaxChildren) * c : link_words(moment, c)) = node;
+        }
+        link_words(moment, node)[1] = k;
+        for (; k < kMaxChildren; ++k) row[k] = kNoChild;
+    }
+}
+
+// octree.cpp:142-185 (internal): children in DFS order; quadrupoles by the
+// parallel-axis theorem, children's moments first.
+__device__ void internal_moments(
+    std::uint32_t node, const std::uint32_t* __restrict__ node_begin,
+    const std::uint32_t* __restrict__ node_count, const std::uint32_t* __restrict__ node_next,
+    const std::uint32_t* __restrict__ children, const double4* __restrict__ node_geo, double theta,
+    const double* __restrict__ cube, std::uint32_t system_end, double4* __restrict__ moment,
+    WalkNode* __restrict__ walk, double* __restrict__ quad64, QuadF* __restrict__ quadf) {
+    // The children's indices, then their moments, loaded side by side; the
+    // sums below still run in DFS order.
+    const std::uint32_t* list = children + static_cast<std::size_t>(kMaxChildren) * node;
+    std::uint32_t child[kMaxChildren];
+    double4 cms[kMaxChildren];
+#pragma unroll
+    for (int k = 0; k < kMaxChildren; ++k) child[k] = list[k];
+#pragma unroll
+    for (int k = 0; k < kMaxChildren; ++k) {
+        const double* m = &moment[child[k] == kNoChild ? node : child[k]].x;
+        cms[k] = make_double4(shared_value(m), shared_value(m + 1), shared_value(m + 2), shared_value(m + 3));
+    }
+    double mass = 0, wx = 0, wy = 0, wz = 0, mx = 0, my = 0, mz = 0;
+    std::uint32_t count = 0;
+#pragma unroll
+    for (int k = 0; k < kMaxChildren; ++k) {
+        if (child[k] == kNoChild) continue;
+        const double4 cm = cms[k];
+        mass += cm.w;
+        wx += cm.x * cm.w;
+        wy += cm.y * cm.w;
+        wz += cm.z * cm.w;
+        mx += cm.x;
+        my += cm.y;
+        mz += cm.z;
+        ++count;
+    }
+    double cx, cy, cz;
+    if (mass > 0) {
+        cx = wx / mass;
+        cy = wy / mass;
+        cz = wz / mass;
+    } else {
+        const double k = static_cast<double>(count == 0 ? 1 : count);
+        cx = mx / k;
+        cy = my / k;
+        cz = mz / k;
+    }
+    const std::uint32_t b = node_begin[node];
+    finish_node(node, mass, cx, cy, cz, node_geo[node], theta, cube, false, b, 0,
+                walk_escape(node_next[node], b + node_count[node], system_end), moment, walk);
+    if (quad64 != nullptr) {
+        double q[6] = {0, 0, 0, 0, 0, 0};
+        // Four children's moments on their way together: one latency, not four.
+#pragma unroll
+        for (int k = 0; k < kMaxChildren; k += 4) {
+            double cq[4][6];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const std::uint32_t c = child[k + u] == kNoChild ? node : child[k + u];
+#pragma unroll
+                for (int j = 0; j < 6; ++j) cq[u][j] = shared_value(quad64 + 6 * static_cast<std::size_t>(c) + j);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (child[k + u] == kNoChild) continue;
+                for (int j = 0; j < 6; ++j) q[j] += cq[u][j];
+                const double4 cm = cms[k + u];
+                add_displaced(q, cm.w, cm.x - cx, cm.y - cy, cm.z - cz);
+            }
+        }
+        store_quad(node, q, quad64, quadf);
+    }
+}
+
+// All moments in one launch. One thread a leaf, octree.cpp:91-135: index-order
+// sums, fallback to the first particle; with quadrupoles, the displaced
+// moments of the particles about the centre of mass. Then up the tree: the
+// thread whose child was the last one a node waited for computes the node and
+// goes on to its parent; the others are done, and no thread waits. Which
+// thread comes last does not change what it computes. A launch a level, 21 of
+// them, cost 3 to 10 us each, most over levels that have no nodes: all
+// moments of 16,384 particles 70 -> 33 us, of 65,536 72 -> 34, with
+// quadrupoles of 262,144 126 -> 71 and of 2,097,152 264 -> 225. Plain stores
+// between agent-scope fences instead of stores and loads past the L2: 33 -> 35
+// and 225 -> 1120 us.
+__global__ __launch_bounds__(kBlock) void tree_moments(
     const std::uint32_t* __restrict__ counters, const std::uint8_t* __restrict__ node_level,
     const std::uint8_t* __restrict__ leaf_level_of_first, const std::uint32_t* __restrict__ node_begin,
     const std::uint32_t* __restrict__ node_count, const std::uint32_t* __restrict__ node_next,
-    const double4* __restrict__ node_geo, const double4* __restrict__ sorted, double theta,
+    const std::uint32_t* __restrict__ children, const double4* __restrict__ node_geo,
+    const double4* __restrict__ sorted, double theta,
     const double* __restrict__ cubes, const std::uint32_t* __restrict__ seg_of,
     const std::uint32_t* __restrict__ seg_start, std::uint32_t n,
-    double4* __restrict__ moment, WalkNode* __restrict__ walk,
-    double* __restrict__ quad64, QuadF* __restrict__ quadf) {
+    double4* moment, WalkNode* __restrict__ walk, double* quad64, QuadF* __restrict__ quadf) {
     const std::uint32_t M = counters[0];
     for (std::uint32_t node = grid_stride_start(); node < M; node += grid_stride_step()) {
         const std::uint32_t b = node_begin[node];
@@ -395,6 +528,7 @@ __global__ __launch_bounds__(kBlock) void leaf_moments(
         const std::uint32_t system_end = seg_start != nullptr ? seg_start[seg + 1] : n;
         const std::uint32_t e = b + node_count[node];
         double mass = 0, wx = 0, wy = 0, wz = 0;
+#pragma unroll 4
         for (std::uint32_t i = b; i < e; ++i) {
             const double4 p = sorted[i];
             mass += p.w;
@@ -416,103 +550,26 @@ __global__ __launch_bounds__(kBlock) void leaf_moments(
                     walk_escape(node_next[node], e, system_end), moment, walk);
         if (quad64 != nullptr) {
             double q[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 4
             for (std::uint32_t i = b; i < e; ++i) {
                 const double4 p = sorted[i];
                 add_displaced(q, p.w, p.x - cx, p.y - cy, p.z - cz);
             }
             store_quad(node, q, quad64, quadf);
         }
-    }
-}
-
-// The children of every internal node in DFS order (the next chain from
-// node + 1 to the node's own next), written once for all levels in one launch
-// so that the per-level moment passes load them side by side instead of
-// following the chain one dependent load at a time.
-__global__ __launch_bounds__(kBlock) void tree_children(
-    const std::uint32_t* __restrict__ counters, const std::uint8_t* __restrict__ node_level,
-    const std::uint8_t* __restrict__ leaf_level_of_first, const std::uint32_t* __restrict__ node_begin,
-    const std::uint32_t* __restrict__ node_next, std::uint32_t* __restrict__ children) {
-    const std::uint32_t M = counters[0];
-    for (std::uint32_t node = grid_stride_start(); node < M; node += grid_stride_step()) {
-        if (node_level[node] == leaf_level_of_first[node_begin[node]]) continue;  // a leaf
-        const std::uint32_t end = node_next[node];
-        std::uint32_t* out = children + static_cast<std::size_t>(kMaxChildren) * node;
-        int k = 0;
-        for (std::uint32_t c = node + 1; c < end && k < kMaxChildren; c = max(node_next[c], c + 1)) out[k++] = c;
-        for (; k < kMaxChildren; ++k) out[k] = kNoChild;
-    }
-}
-
-// octree.cpp:142-185 (internal): children in DFS order via the next chain;
-// quadrupoles by the parallel-axis theorem, children's moments first.
-__global__ __launch_bounds__(kBlock) void internal_moments(
-    unsigned level, const std::uint32_t* __restrict__ counters,
-    const std::uint8_t* __restrict__ node_level, const std::uint8_t* __restrict__ leaf_level_of_first,
-    const std::uint32_t* __restrict__ node_begin, const std::uint32_t* __restrict__ node_count,
-    const std::uint32_t* __restrict__ node_next, const std::uint32_t* __restrict__ children,
-    const double4* __restrict__ node_geo, double theta, const double* __restrict__ cubes,
-    const std::uint32_t* __restrict__ seg_of, const std::uint32_t* __restrict__ seg_start,
-    std::uint32_t n, double4* __restrict__ moment,
-    WalkNode* __restrict__ walk, double* __restrict__ quad64, QuadF* __restrict__ quadf) {
-    const std::uint32_t M = counters[0];
-    for (std::uint32_t node = grid_stride_start(); node < M; node += grid_stride_step()) {
-        if (node_level[node] != level) continue;
-        const std::uint32_t b = node_begin[node];
-        if (leaf_level_of_first[b] == level) continue;  // a leaf
-        const std::uint32_t seg = seg_of != nullptr ? seg_of[b] : 0u;
-        const double* cube = cubes + 4 * static_cast<std::size_t>(seg);
-        const std::uint32_t system_end = seg_start != nullptr ? seg_start[seg + 1] : n;
-        // The children's indices, then their moments, loaded side by side; the
-        // sums below still run in DFS order.
-        const std::uint32_t* list = children + static_cast<std::size_t>(kMaxChildren) * node;
-        std::uint32_t child[kMaxChildren];
-        double4 cms[kMaxChildren];
-#pragma unroll
-        for (int k = 0; k < kMaxChildren; ++k) child[k] = list[k];
-#pragma unroll
-        for (int k = 0; k < kMaxChildren; ++k) {
-            if (child[k] != kNoChild) cms[k] = moment[child[k]];
-        }
-        double mass = 0, wx = 0, wy = 0, wz = 0, mx = 0, my = 0, mz = 0;
-        std::uint32_t count = 0;
-#pragma unroll
-        for (int k = 0; k < kMaxChildren; ++k) {
-            if (child[k] == kNoChild) continue;
-            const double4 cm = cms[k];
-            mass += cm.w;
-            wx += cm.x * cm.w;
-            wy += cm.y * cm.w;
-            wz += cm.z * cm.w;
-            mx += cm.x;
-            my += cm.y;
-            mz += cm.z;
-            ++count;
-        }
-        double cx, cy, cz;
-        if (mass > 0) {
-            cx = wx / mass;
-            cy = wy / mass;
-            cz = wz / mass;
-        } else {
-            const double k = static_cast<double>(count == 0 ? 1 : count);
-            cx = mx / k;
-            cy = my / k;
-            cz = mz / k;
-        }
-        finish_node(node, mass, cx, cy, cz, node_geo[node], theta, cube, false, b, 0,
-                    walk_escape(node_next[node], b + node_count[node], system_end), moment, walk);
-        if (quad64 != nullptr) {
-            double q[6] = {0, 0, 0, 0, 0, 0};
-#pragma unroll
-            for (int k = 0; k < kMaxChildren; ++k) {
-                if (child[k] == kNoChild) continue;
-                const double* cq = quad64 + 6 * static_cast<std::size_t>(child[k]);
-                for (int j = 0; j < 6; ++j) q[j] += cq[j];
-                const double4 cm = cms[k];
-                add_displaced(q, cm.w, cm.x - cx, cm.y - cy, cm.z - cz);
-            }
-            store_quad(node, q, quad64, quadf);
+        std::uint32_t up = children[static_cast<std::size_t>(kMaxChildren) * node];
+        while (up != kNoChild) {
+            std::uint32_t* const link = link_words(moment, up);
+            const std::uint32_t above = __hip_atomic_load(link, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // The child's moments are in memory before the count says so (the
+            // stores above go past the L2; this waits for them), and the
+            // siblings' are read after it.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (__hip_atomic_fetch_sub(link + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 1) break;
+            asm volatile("" ::: "memory");
+            internal_moments(up, node_begin, node_count, node_next, children, node_geo, theta, cube, system_end,
+                             moment, walk, quad64, quadf);
+            up = above;
         }
     }
 }
@@ -1350,11 +1407,8 @@ void tree_enqueue(orr_ctx* ctx, const orr_tree_args& a, const SegmentView& segs,
     const double* cube = ctx->order_bbox.as<double>();
     {
         PhaseTimer t(ctx, kBuild);
-        hipLaunchKernelGGL(clear_counters, dim3(1), dim3(kBlock), 0, ctx->stream, L.c32,
-                           seg_stats != nullptr ? nullptr : L.c64, 4 * segs.count);
-        ORR_LAUNCHED("clear_counters");
         hipLaunchKernelGGL(tree_levels, dim3(blocks), dim3(kBlock), 0, ctx->stream, codes, seg_of, n32,
-                           L.d);
+                           L.d, L.c32, seg_stats != nullptr ? nullptr : L.c64, 4 * segs.count);
         ORR_LAUNCHED("tree_levels");
         hipLaunchKernelGGL(tree_chain, dim3(blocks), dim3(kBlock), 0, ctx->stream, L.d, n32, cap,
                            L.chain, L.leaf_level);
@@ -1364,9 +1418,6 @@ void tree_enqueue(orr_ctx* ctx, const orr_tree_args& a, const SegmentView& segs,
                            L.leaf_level, L.chain, L.first_node, n32, L.block_counts, L.begin,
                            L.level);
         ORR_LAUNCHED("tree_chains");
-        hipLaunchKernelGGL(tree_counts, dim3(1), dim3(kBlock), 0, ctx->stream, L.block_counts,
-                           blocks, L.c32);
-        ORR_LAUNCHED("tree_counts");
         hipLaunchKernelGGL(tree_node_fill, dim3(node_blocks), dim3(kBlock), 0, ctx->stream, codes,
                            L.leaf_level, L.first_node, n32, seg_of, seg_start, cube, L.c32,
                            L.begin, L.level, L.count, L.next, L.geo, L.leaf_of);
@@ -1381,20 +1432,14 @@ void tree_enqueue(orr_ctx* ctx, const orr_tree_args& a, const SegmentView& segs,
     }
     {
         PhaseTimer t(ctx, kMoments);
-        hipLaunchKernelGGL(leaf_moments, dim3(node_blocks), dim3(kBlock), 0, ctx->stream, L.c32,
-                           L.level, L.leaf_level, L.begin, L.count, L.next, L.geo, L.sorted, theta,
-                           cube, seg_of, seg_start, n32, L.moment, L.walk, L.quad64, L.quadf);
-        ORR_LAUNCHED("leaf_moments");
-        hipLaunchKernelGGL(tree_children, dim3(node_blocks), dim3(kBlock), 0, ctx->stream, L.c32,
-                           L.level, L.leaf_level, L.begin, L.next, L.children);
-        ORR_LAUNCHED("tree_children");
-        for (int level = static_cast<int>(kLevels) - 1; level >= 0; --level) {
-            hipLaunchKernelGGL(internal_moments, dim3(node_blocks), dim3(kBlock), 0, ctx->stream,
-                               static_cast<unsigned>(level), L.c32, L.level, L.leaf_level, L.begin,
-                               L.count, L.next, L.children, L.geo, theta, cube, seg_of, seg_start,
-                               n32, L.moment, L.walk, L.quad64, L.quadf);
-            ORR_LAUNCHED("internal_moments");
-        }
+        hipLaunchKernelGGL(tree_links, dim3(node_blocks + 1), dim3(kBlock), 0, ctx->stream, L.c32,
+                           L.level, L.leaf_level, L.begin, L.next, L.block_counts, blocks, L.children,
+                           L.moment);
+        ORR_LAUNCHED("tree_links");
+        hipLaunchKernelGGL(tree_moments, dim3(node_blocks), dim3(kBlock), 0, ctx->stream, L.c32,
+                           L.level, L.leaf_level, L.begin, L.count, L.next, L.children, L.geo, L.sorted,
+                           theta, cube, seg_of, seg_start, n32, L.moment, L.walk, L.quad64, L.quadf);
+        ORR_LAUNCHED("tree_moments");
     }
     {
         PhaseTimer t(ctx, kWalk);

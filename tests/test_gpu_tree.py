@@ -68,6 +68,33 @@ def test_quadrupole_moments_bitwise(ctx, gen, n, cap):
     assert np.array_equal(s.quadrupoles(), t.quad)
 
 
+@pytest.mark.parametrize("n,cap,shape", [
+    (1, 1, "ball"), (2, 1, "ball"), (2, 1, "close"), (9, 1, "close"), (300, 1, "close"), (50, 8, "same"),
+    (4000, 1, "close"), (257, 1, "ball"), (60000, 2, "ball"), (300000, 16, "ball")])
+def test_moments_climb_every_shape(ctx, n, cap, shape):
+    """Root leaves, chains of cells with one child down to the last level, leaves over
+    capacity there, and many leaves: the moments bit for bit, each of three times in a row."""
+    rng = np.random.default_rng(n)
+    pts = rng.normal(size=(n, 3))
+    if shape == "close":
+        pts = 0.7 + 1e-6 * pts
+        pts[0] = 0.0
+    if shape == "same":
+        pts[1:] = pts[1]
+    x, y, z = (np.ascontiguousarray(pts[:, k]) for k in range(3))
+    m = rng.random(n) / n
+    codes, index, origin, size = oracle.morton_order(x, y, z)
+    i = index.astype(np.int64)
+    t = oracle.tree_build(x[i], y[i], z[i], m[i], codes, origin, size, 0.5, cap, quadrupole=True)
+    s = E.HipTreeSolver(E.TreeParameters(0.5, cap, quadrupole=True), E.Softening(0.05), context=ctx)
+    for _ in range(3):
+        s.evaluate((x, y, z), m, [np.zeros(n) for _ in range(3)])
+        got = s.nodes()
+        assert s.tree_summary()["depth"] == t.depth and s.tree_summary()["leaf_count"] == t.leaves
+        assert np.array_equal(got["mass"], t.mass) and np.array_equal(got["com"], t.com)
+        assert np.array_equal(got["acc_r2"], t.acc_r2) and np.array_equal(s.quadrupoles(), t.quad)
+
+
 def test_quadrupole_accuracy_reference_setup(ctx):
     # docs/performance/tree_accuracy.csv setup: Plummer standard units, N = 16384,
     # eps = 0.05, leaf 32; the reference's quadrupole walk: RMS 9.76e-4 at theta 0.5.
