@@ -647,7 +647,8 @@ struct WalkTarget {
     float4 xi, oi;
     std::uint32_t own;
     float sx, sy, sz, kx, ky, kz, px, py, pz;
-    std::uint32_t pc;  // accepted nodes, at most M
+    // Accepted nodes and particle-particle terms: at most M and n.
+    std::uint32_t pc, pp;
 };
 
 // Separation of the target from a node's centre of mass, and its square.
@@ -769,14 +770,23 @@ __device__ __forceinline__ std::uint32_t lane_read(std::uint32_t reg, std::uint3
     return static_cast<std::uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(reg), static_cast<int>(lane)));
 }
 
-// The wave's accepted nodes (idle lanes count none).
-template<int kR> __device__ unsigned long long accepted(const WalkTarget (&t)[kR]) {
-    unsigned long long v = 0;
+// The wave's counts (idle lanes count none): pairs and accepted nodes.
+struct WalkCounts {
+    unsigned long long pp, pc;
+};
+template<int kR> __device__ WalkCounts wave_counts(const WalkTarget (&t)[kR]) {
+    unsigned long long v[2] = {0, 0};
 #pragma unroll
-    for (int r = 0; r < kR; ++r) v += t[r].pc;
+    for (int r = 0; r < kR; ++r) {
+        v[0] += t[r].pp;
+        v[1] += t[r].pc;
+    }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
+    }
+    return {v[0], v[1]};
 }
 
 // One system's counts from a wave that walked several.
@@ -816,8 +826,7 @@ __device__ __forceinline__ float walk_reach(float weight) {
 // reach each of its children, and all that reached the cell go on after it. So
 // opening a cell pushes the mask of its sibling list with the escape index that
 // ends it, and reaching that index pops it. Which lanes accept is one compare
-// and scalar logic, the counts are scalar population counts, and the next node
-// needs no reduction over the lanes.
+// and scalar logic, and the next node needs no reduction over the lanes.
 //
 // kMany: the targets may belong to several systems (a batch); the systems of
 // a wave's targets are then walked one after another.
@@ -894,7 +903,7 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
         todo[r] = __ballot(valid);
         t[r].sx = t[r].sy = t[r].sz = t[r].kx = t[r].ky = t[r].kz = 0.f;
         t[r].px = t[r].py = t[r].pz = 0.f;
-        t[r].pc = 0;
+        t[r].pc = t[r].pp = 0;
     }
     if constexpr (kSplit > 1) {
         if (threadIdx.x < kSplit) s_done[threadIdx.x] = 0;
@@ -908,9 +917,9 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
     std::uint32_t steps = 0;
     std::uint32_t systems = 0;   // systems walked by this wave
     std::uint32_t seg0 = 0;      // the first of them
-    // Particle-particle terms, and the visits that accepted nothing (leaves
-    // and opened cells); accepted nodes are counted per target.
-    unsigned long long pp = 0, stopped = 0;
+    // Visits that accepted nothing (leaves and opened cells), one per target;
+    // the other counts are kept per target.
+    unsigned long long stopped = 0;
     // A split walk: the runs kept for the replay, whether the sums so far are
     // here yet (`direct`), and the targets whose last run ends with the walk.
     std::uint32_t kept = 0;
@@ -968,14 +977,14 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
         }
         if (kMany && systems > 0) {
             // A second system: the counts so far belong to the one before it.
-            const unsigned long long pc = accepted(t);
+            const WalkCounts c = wave_counts(t);
             if (lane == 0) {
-                add_counts(stats, seg0, pp, pc, pc + stopped,
+                add_counts(stats, seg0, c.pp, c.pc, c.pc + stopped,
                            static_cast<unsigned long long>(steps) * (kR * kLanes) / 64);
             }
 #pragma unroll
-            for (int r = 0; r < kR; ++r) t[r].pc = 0;
-            pp = stopped = 0;
+            for (int r = 0; r < kR; ++r) t[r].pc = t[r].pp = 0;
+            stopped = 0;
             steps = 0;
         }
         seg0 = own_seg;
@@ -991,8 +1000,8 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
         // those still walking.
         std::uint64_t open = 0, alive = ~std::uint64_t{0};
         bool tail = false;
-        std::uint32_t main_steps = 0, main_pc = 0;
-        unsigned long long main_pp = 0, main_stopped = 0;
+        std::uint32_t main_steps = 0, main_pc = 0, main_pp = 0;
+        unsigned long long main_stopped = 0;
         auto up = [&] {
             // The end of one or more sibling lists: back to the masks of the
             // lists they lie in (cur > 0, so never past the outermost).
@@ -1108,16 +1117,14 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
                 const std::uint32_t next = max(nb.y, step);
                 std::uint32_t go = next;
                 if (any != 0) {
+#pragma unroll
+                    for (int r = 0; r < kR; ++r) stopped += __popcll(rest[r]);
                     if (nb.w != 0) {
                         const double4 cb = node_geo[cur];
                         const std::uint32_t b = nb.z, e = nb.z + nb.w;
 #pragma unroll
                         for (int r = 0; r < kR; ++r) {
                             if (rest[r] == 0) continue;
-                            const std::uint32_t here = __popcll(rest[r]);
-                            stopped += here;
-                            pp += static_cast<unsigned long long>(here) * nb.w -
-                                  __popcll(__ballot(t[r].own == cur) & rest[r]);
                             if (__builtin_amdgcn_inverse_ballot_w64(rest[r])) {
                                 leaf_pairs<kSafe>(t[r], cb, s_own[r][0][slot], s_own[r][1][slot],
                                                   s_own[r][2][slot], leaf_rel, b, e, eps2, lane0);
@@ -1131,6 +1138,7 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
                                     }
                                 }
                                 t[r].px = t[r].py = t[r].pz = 0.f;
+                                t[r].pp += nb.w - (t[r].own == cur ? 1u : 0u);
                             }
                             if constexpr (kSplit > 1) {
                                 if (tail) {
@@ -1149,8 +1157,6 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
                     } else {
                         // Open: the children for those that did, then everyone here
                         // goes on at `next`.
-#pragma unroll
-                        for (int r = 0; r < kR; ++r) stopped += __popcll(rest[r]);
                         open_cell(next, rest);
                         go = step;
                     }
@@ -1164,9 +1170,9 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
             // its end. The part that owns these nodes counts them.
             tail = true;
             main_steps = steps;
-            main_pp = pp;
             main_stopped = stopped;
             main_pc = t[0].pc;
+            main_pp = t[0].pp;
             alive = open;
             mask[0] &= open;
             stop = M;
@@ -1174,9 +1180,9 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
         if constexpr (kSplit > 1) {
             if (tail) {
                 steps = main_steps;
-                pp = main_pp;
                 stopped = main_stopped;
                 t[0].pc = main_pc;
+                t[0].pp = main_pp;
             }
             last_run |= open;
         }
@@ -1197,12 +1203,12 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
     // Counts: a wave inside one system writes its sums to its own slot, summed
     // per system by walk_counts (atomics on one address would serialise every
     // wave); a wave spanning systems adds them per system.
-    const unsigned long long pc = accepted(t);
-    unsigned long long count[4] = {pp, pc, pc + stopped, steps};
+    const WalkCounts c = wave_counts(t);
+    unsigned long long count[4] = {c.pp, c.pc, c.pc + stopped, steps};
     const bool mixed = kMany && systems > 1;
     if (mixed) {
-        if (lane == 0) add_counts(stats, seg0, pp, pc, pc + stopped, count[3] * (kR * kLanes) / 64);
-        for (int c = 0; c < 4; ++c) count[c] = 0;
+        if (lane == 0) add_counts(stats, seg0, count[0], count[1], count[2], count[3] * (kR * kLanes) / 64);
+        for (int k = 0; k < 4; ++k) count[k] = 0;
     }
     if constexpr (kSplit > 1) {
         if (part + 1 < kSplit) {
@@ -1215,14 +1221,14 @@ __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
                 s_chain[5][lane] = t[0].kz;
             }
             if (lane == 0) {
-                for (int c = 0; c < 4; ++c) s_count[part][c] = count[c];
+                for (int k = 0; k < 4; ++k) s_count[part][k] = count[k];
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             if (lane == 0) *static_cast<volatile std::uint32_t*>(&s_done[part]) = 1;
             return;
         }
         for (int q = 0; q + 1 < kSplit; ++q) {
-            for (int c = 0; c < 4; ++c) count[c] += s_count[q][c];
+            for (int k = 0; k < 4; ++k) count[k] += s_count[q][k];
         }
     }
 #pragma unroll
