@@ -111,6 +111,9 @@ __global__ __launch_bounds__(kBlock) void tree_levels(const std::uint64_t* __res
 }
 
 // Chain length of the nodes that start at particle k; leaf level in `leaf_level`.
+// The searches read kAhead levels at once: one at a time, each waits for the
+// one before (16,384 particles 10.8 -> 5.5 us, 2,097,152 37 -> 22).
+constexpr int kAhead = 8;
 __global__ __launch_bounds__(kBlock) void tree_chain(const std::uint8_t* __restrict__ d,
                                                      std::uint32_t n, std::uint32_t cap,
                                                      std::uint32_t* __restrict__ chain,
@@ -128,20 +131,28 @@ __global__ __launch_bounds__(kBlock) void tree_chain(const std::uint8_t* __restr
             const unsigned P = dk - 1;
             const std::uint32_t lo = k + 1 > cap ? k + 1 - cap : 0;
             std::int64_t p = -1;
-            for (std::int64_t j = static_cast<std::int64_t>(k) - 1; j >= static_cast<std::int64_t>(lo); --j) {
-                if (d[j] <= P) {
-                    p = j;
-                    break;
+            for (std::int64_t j = static_cast<std::int64_t>(k) - 1; j >= static_cast<std::int64_t>(lo) && p < 0;
+                 j -= kAhead) {
+                std::uint8_t level[kAhead];
+                // Past the end of the search, its last element again.
+#pragma unroll
+                for (int u = 0; u < kAhead; ++u) level[u] = d[std::max<std::int64_t>(j - u, lo)];
+#pragma unroll
+                for (int u = kAhead - 1; u >= 0; --u) {
+                    if (level[u] <= P) p = std::max<std::int64_t>(j - u, lo);
                 }
             }
             if (p >= 0) {
                 const std::uint64_t limit = static_cast<std::uint64_t>(p) + cap;  // q must be <= limit
                 std::uint64_t q = n;
                 const std::uint64_t stop = limit < n - 1 ? limit : n - 1;
-                for (std::uint64_t j = k + 1; j <= stop; ++j) {
-                    if (d[j] <= P) {
-                        q = j;
-                        break;
+                for (std::uint64_t j = k + 1; j <= stop && q == n; j += kAhead) {
+                    std::uint8_t level[kAhead];
+#pragma unroll
+                    for (int u = 0; u < kAhead; ++u) level[u] = d[std::min<std::uint64_t>(j + u, stop)];
+#pragma unroll
+                    for (int u = kAhead - 1; u >= 0; --u) {
+                        if (level[u] <= P) q = std::min<std::uint64_t>(j + u, stop);
                     }
                 }
                 head = !(q <= limit);
@@ -152,7 +163,12 @@ __global__ __launch_bounds__(kBlock) void tree_chain(const std::uint8_t* __restr
                 lleaf = dk;
             } else {
                 unsigned w = kNoBoundary;
-                for (std::uint32_t j = k + 1; j <= k + cap; ++j) w = min(w, static_cast<unsigned>(d[j]));
+                for (std::uint32_t j = k + 1; j <= k + cap; j += kAhead) {
+#pragma unroll
+                    for (std::uint32_t u = 0; u < kAhead; ++u) {
+                        w = min(w, static_cast<unsigned>(d[min(j + u, k + cap)]));
+                    }
+                }
                 lleaf = min(kLevels, max(dk, w));
             }
             len = lleaf - dk + 1;
@@ -169,23 +185,46 @@ __device__ std::uint32_t prefix_end(const std::uint64_t* __restrict__ codes, std
     const unsigned s = 3u * (kLevels - level);
     const std::uint64_t want = key >> s;
     if (lo >= n || (codes[lo] >> s) != want) return lo;
-    // Gallop, then bisect: codes[lo] shares the prefix.
-    std::uint32_t good = lo;
-    std::uint32_t step = 1;
-    std::uint32_t bad = n;
-    while (true) {
-        const std::uint64_t probe = static_cast<std::uint64_t>(good) + step;
-        if (probe >= n) break;
-        if ((codes[probe] >> s) != want) {
-            bad = static_cast<std::uint32_t>(probe);
-            break;
+    // Gallop, then narrow down: codes[lo] shares the prefix. Four probes at once:
+    // one at a time, each waits for the one before, 27 in a row for a root of
+    // 16,384 particles (tree_node_fill of 60,000 particles 11.6 -> 9.3 us, of
+    // 262,144 12.4 -> 9.8).
+    constexpr unsigned kProbes = 4;
+    auto matches = [&](std::uint64_t at) { return (codes[at] >> s) == want; };
+    std::uint32_t good = lo, bad = n;
+    bool found = false;
+    for (unsigned power = 0; !found; power += kProbes) {
+        bool match[kProbes];
+#pragma unroll
+        for (unsigned u = 0; u < kProbes; ++u) {
+            match[u] = matches(std::min<std::uint64_t>(lo + (std::uint64_t{1} << (power + u)), n - 1));
         }
-        good = static_cast<std::uint32_t>(probe);
-        step <<= 1;
+#pragma unroll
+        for (unsigned u = 0; u < kProbes; ++u) {
+            const std::uint64_t at = lo + (std::uint64_t{1} << (power + u));
+            if (found) continue;
+            found = at >= n || !match[u];
+            if (at < n) (match[u] ? good : bad) = static_cast<std::uint32_t>(at);
+        }
     }
     while (bad - good > 1) {
-        const std::uint32_t mid = good + (bad - good) / 2;
-        if ((codes[mid] >> s) != want) bad = mid; else good = mid;
+        const std::uint32_t step = (bad - good + kProbes) / (kProbes + 1);
+        const std::uint32_t from = good, to = bad;
+        bool match[kProbes];
+#pragma unroll
+        for (unsigned u = 0; u < kProbes; ++u) {
+            match[u] = matches(std::min<std::uint64_t>(from + std::uint64_t{step} * (u + 1), to - 1));
+        }
+        // The probes that match come first.
+#pragma unroll
+        for (unsigned u = 0; u < kProbes; ++u) {
+            const std::uint64_t at = std::min<std::uint64_t>(from + std::uint64_t{step} * (u + 1), to - 1);
+            if (match[u]) {
+                good = static_cast<std::uint32_t>(at);
+            } else if (at < bad) {
+                bad = static_cast<std::uint32_t>(at);
+            }
+        }
     }
     return bad;
 }
