@@ -208,11 +208,12 @@ ORR_API int orr_tree_eval(orr_ctx* ctx, const orr_tree_args* args, orr_tree_stat
  * traversal): targets_per_lane 1 or 2 -- how many targets each lane of a
  * wave walks together -- or -1 for the engine's choice (1; the default); lanes
  * 64 or 32 -- how many lanes of a wave hold targets -- or -1 to choose by size
- * (16 for a launch of at most 256 full waves, 32 up to 2048, two per SIMD, else
- * 64; the default). Results are
- * bit-identical either way; only the speed differs. sort_mode chooses the
+ * (the default: groups of 16 targets walked by eight or four waves to 8192 and
+ * 24,576 particles, groups of 32 by two to 73,728, 32 a wave to 102,400, else 64).
+ * Results are bit-identical either way; only the speed differs. sort_mode chooses the
  * Morton sort of every path (the tree's, the batch's, the direct ordering of
- * more than 4096 particles): 1 (the default) one launch per radix pass after
+ * more than 20,480 particles): 1 (the default) systems of up to 196,608 particles
+ * in chunks sorted in LDS and merged by rank, larger ones in one launch per radix pass after
  * one launch that counts every pass's digits, 2 histogram, scan and scatter
  * launches per pass; the same permutation either way. Zero keeps the current
  * value; the getter reports -1 while a choice is by size. */

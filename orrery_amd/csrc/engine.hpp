@@ -134,10 +134,10 @@ struct orr_ctx {
     // 1: the pairs path's equal-mass form where the masses allow it, 2: never.
     int direct_equal_masses = 1;
     int direct_small_order = 1;  // 1: ordering by rank up to kRankOrder particles, 2: never
-    int sort_mode = 1;  // Morton sort: 1 one-sweep passes, 2 histogram + scan + scatter per pass
+    int sort_mode = 1;  // Morton sort: 1 chunks merged by rank or one-sweep passes, 2 histogram + scan + scatter per pass
     // Barnes-Hut walk configuration (orr_ctx_set_tree_config); 0 chooses by size.
     int walk_targets_per_lane = 0;
-    int walk_lanes = 0;  // active lanes per walk wave: 32, 64, or 0 = by size (16, 32 or 64)
+    int walk_lanes = 0;  // active lanes per walk wave: 32, 64, or 0 = by size (16, 32 or 64, and several waves a group)
 
     // Host mirror of the last tree summary and the shape of its device layout.
     orr_tree_stats last_tree{};
