@@ -1955,7 +1955,7 @@ void direct_evaluate_static(orr_ctx* ctx, const orr_direct_args& a) {
         ob.index[0] = c.take<std::uint32_t>(oz.index);
         ob.index[1] = c.take<std::uint32_t>(oz.index);
         ob.hist = c.take<std::uint32_t>(oz.hist);
-        // The order direct_evaluate uses: the four upper radix passes.
+        // The order direct_evaluate uses: by the upper half of the codes.
         const int cur = morton_enqueue_into(ctx, a.x, a.y, a.z, n, SegmentView{}, nullptr, 4, ob, false);
         order = ob.index[cur];
     }

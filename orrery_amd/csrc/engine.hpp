@@ -387,7 +387,7 @@ std::uint64_t direct_static_max_count();
 // context.hip: device bytes held by a context's scratch buffers.
 std::size_t ctx_device_bytes(const orr_ctx* ctx);
 
-// morton.hip: bounding cube, codes and stable radix sort from identity order.
+// morton.hip: bounding cube, codes and stable order from identity.
 // Leaves ascending codes and permutation in ctx->order_codes / order_index
 // (uint64 / uint32). Returns nothing on the host; cube lands in ctx->order_bbox.
 // first_digit > 0 skips the sort's low 8-bit digits: the order is then by the

@@ -26,10 +26,11 @@
 // contraction disabled, so masses, centres of mass and acceptance radii
 // (octree.cpp:374-387) are the reference's bit for bit.
 //
-// The walk (tree_walk.cpp:20-83 per target) runs one wave over 64 consecutive
-// sorted targets. The wave visits node min(next node of each lane) -- each lane
-// still follows exactly its own walk, as the reference's coherent CUDA walk
-// does (ADR-0029) -- with the node read through the scalar unit. Accepted cells
+// The walk (tree_walk.cpp:20-83 per target) runs waves over groups of up to 64
+// consecutive sorted targets. A wave goes through the nodes that any of its
+// targets visits -- each target still takes part in exactly its own walk, as in the
+// reference's coherent CUDA walk (ADR-0029) -- with the node read through the
+// scalar unit. Accepted cells
 // use FP32 positions relative to the root centre; leaf particles are stored as
 // FP32 offsets from their leaf's geometric centre and a lane interacting with a
 // leaf re-expresses its own offset against that centre in FP64, so close pairs
