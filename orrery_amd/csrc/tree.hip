@@ -889,10 +889,13 @@ __device__ __forceinline__ float walk_reach(float weight) {
 // for nobody, so every wait ends. A visit is counted by the part that owns the node.
 //
 // The one-wave walk of one system is held to 64 vector registers, eight waves
-// a SIMD (of 67 it would take; 2,097,152 particles: 8.6 -> 8.3 ms).
+// a SIMD (of 67 it would take; 2,097,152 particles: 8.6 -> 8.3 ms), that of
+// several systems to 72, seven waves (of 75; 147 systems of 4096 to 16,384
+// particles, a whole evaluation: 2.12 -> 2.01 ms; eight waves, with registers
+// spilled, 1.99, but 0.77 instead of 0.76 ms for 40 systems).
 template<int kR, bool kSafe, bool kQuad, int kLanes, bool kMany, int kSplit>
 __global__ __launch_bounds__(kSplit == 1 ? kBlock : 64 * kSplit,
-                             kSplit == 1 && kR == 1 && !kMany ? 8 : 1) void tree_walk(
+                             kSplit == 1 && kR == 1 ? (kMany ? 7 : 8) : 1) void tree_walk(
     const WalkNode* __restrict__ nodes, const QuadF* __restrict__ quads,
     const double4* __restrict__ node_geo,
     const float4* __restrict__ root_rel, const float4* __restrict__ leaf_rel,
