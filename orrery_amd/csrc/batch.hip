@@ -303,6 +303,7 @@ void evaluate_direct(orr_batch* b) {
     v.eps2 = b->deps2;
     v.G = b->dG;
     v.safe = b->safe;
+    v.alone = b->n == b->n_direct;
     direct_batch_enqueue(ctx, b->array(0), b->array(1), b->array(2), b->array(9),
                          ctx->order_index.as<std::uint32_t>(), v, b->array(6), b->array(7),
                          b->array(8));

@@ -42,6 +42,7 @@
 #include <cstdint>
 #include <mutex>
 #include <type_traits>
+#include <utility>
 
 #include "close_pair.hpp"
 #include "engine.hpp"
@@ -243,14 +244,16 @@ constexpr int kRun = 16;
 // Terms of a near tile summed plainly in FP32 before each Kahan addition.
 constexpr int kNearRun = 8;
 
-template<int R, bool kSafe, bool kRefine, bool kGivenNear = false, int kUnroll = 16>
-__device__ __forceinline__ void source_tile(
+//
+// source_tile_to hands each far run's sums, or the near tile's pair, to its
+// caller; source_tile adds them.
+template<int R, bool kSafe, bool kRefine, bool kGivenNear, int kUnroll, class Far, class Near>
+__device__ __forceinline__ void source_tile_to(
     const float4* __restrict__ packed, const float4* __restrict__ packed_lo,
     const double4* __restrict__ centres, const float4* __restrict__ extents, std::uint32_t J,
     bool given_near, std::uint32_t sources, const bool (&live)[R], float eps2,
     const float (&ox)[R], const float (&oy)[R], const float (&oz)[R], const float (&lx)[R], const float (&ly)[R], const float (&lz)[R], const double (&cx)[R],
-    const double (&cy)[R], const double (&cz)[R], const float4 (&ce)[R], float (&sx)[R],
-    float (&sy)[R], float (&sz)[R], float (&kx)[R], float (&ky)[R], float (&kz)[R]) {
+    const double (&cy)[R], const double (&cz)[R], const float4 (&ce)[R], Far&& far_run, Near&& near_pair_sums) {
     const double4 C = centres[J];
     const float4 E = extents[J];
     const float4* __restrict__ src = packed + static_cast<std::size_t>(J) * kTile;
@@ -295,11 +298,7 @@ __device__ __forceinline__ void source_tile(
                                          px[r], py[r], pz[r]);
             }
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                kahan(px[r], sx[r], kx[r]);
-                kahan(py[r], sy[r], ky[r]);
-                kahan(pz[r], sz[r], kz[r]);
-            }
+            for (int r = 0; r < R; ++r) far_run(r, run, px[r], py[r], pz[r]);
         }
         return;
     }
@@ -406,11 +405,30 @@ __device__ __forceinline__ void source_tile(
         }
     }
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-        kahan_df(px[r], -pkx[r], sx[r], kx[r]);
-        kahan_df(py[r], -pky[r], sy[r], ky[r]);
-        kahan_df(pz[r], -pkz[r], sz[r], kz[r]);
-    }
+    for (int r = 0; r < R; ++r) near_pair_sums(r, px[r], py[r], pz[r], pkx[r], pky[r], pkz[r]);
+}
+
+template<int R, bool kSafe, bool kRefine, bool kGivenNear = false, int kUnroll = 16>
+__device__ __forceinline__ void source_tile(
+    const float4* __restrict__ packed, const float4* __restrict__ packed_lo,
+    const double4* __restrict__ centres, const float4* __restrict__ extents, std::uint32_t J,
+    bool given_near, std::uint32_t sources, const bool (&live)[R], float eps2,
+    const float (&ox)[R], const float (&oy)[R], const float (&oz)[R], const float (&lx)[R], const float (&ly)[R], const float (&lz)[R], const double (&cx)[R],
+    const double (&cy)[R], const double (&cz)[R], const float4 (&ce)[R], float (&sx)[R],
+    float (&sy)[R], float (&sz)[R], float (&kx)[R], float (&ky)[R], float (&kz)[R]) {
+    source_tile_to<R, kSafe, kRefine, kGivenNear, kUnroll>(
+        packed, packed_lo, centres, extents, J, given_near, sources, live, eps2, ox, oy, oz, lx, ly, lz, cx, cy,
+        cz, ce,
+        [&](int r, int, float x, float y, float z) {
+            kahan(x, sx[r], kx[r]);
+            kahan(y, sy[r], ky[r]);
+            kahan(z, sz[r], kz[r]);
+        },
+        [&](int r, float x, float y, float z, float cx_, float cy_, float cz_) {
+            kahan_df(x, -cx_, sx[r], kx[r]);
+            kahan_df(y, -cy_, sy[r], ky[r]);
+            kahan_df(z, -cz_, sz[r], kz[r]);
+        });
 }
 
 // The near flags of every (target tile, source tile) pair, one bit each, rows
@@ -878,6 +896,85 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
         out[3 * kTile + lane] = kx[0];
         out[4 * kTile + lane] = ky[0];
         out[5 * kTile + lane] = kz[0];
+    }
+}
+
+// The same, kWaves waves an item, for batches of direct systems alone with fewer
+// items than the chip holds waves (beside a tree branch, which is the longer one and
+// then has fewer waves of its own running, a 48-system batch went from 19.7 to 20.2 ms): each wave takes every kWaves-th source tile and leaves the
+// tile's run sums in LDS; after each round of kWaves tiles a wave a component
+// adds them in tile order, so the sums are the same bits. Alone on its
+// SIMD, a wave took some 17 us a source tile, sixteen in a row. Whole
+// evaluations of batches of systems of 256 to 4096 particles with one, four and
+// eight waves an item, us: 197 items 207, 128, 107; 1212 items 244, 157, 147;
+// 1770 items 246, 177, 178; 5023 items 340, 323, 337; 13,720 items 649, 725, 777.
+constexpr std::uint32_t kEightWaveItems = 1536;
+constexpr std::uint32_t kFourWaveItems = 5120;
+
+template<bool kSafe, bool kRefine, int kWaves>
+__global__ __launch_bounds__(64 * kWaves) void direct_items_wide(
+    const float4* __restrict__ packed, const float4* __restrict__ packed_lo,
+    const double4* __restrict__ centres, const float4* __restrict__ extents,
+    const uint4* __restrict__ tile, const uint4* __restrict__ item, std::uint32_t items,
+    const float* __restrict__ eps2_of, float* __restrict__ partial) {
+    constexpr int kRuns = kTile / kRun;
+    static_assert(3 * kRuns >= 6 && kWaves >= 3);
+    __shared__ float s_sums[kWaves][3 * kRuns][kTile];  // far: run by run; near: the pair, sums then compensations
+    __shared__ std::uint32_t s_near[kWaves];
+    const unsigned lane = threadIdx.x & (kTile - 1);
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kTile);
+    for (std::uint32_t next = blockIdx.x; next < items; next += gridDim.x) {
+        const uint4 it = item[next];
+        const uint4 own = tile[it.x];
+        const float eps2 = eps2_of[own.z];
+        const bool live[1] = {lane < own.y};
+        const std::uint32_t k = it.x * kTile + lane;
+        const float4 o = packed[k];
+        const float4 l = packed_lo[k];
+        const double4 c = centres[it.x];
+        const float ox[1] = {o.x}, oy[1] = {o.y}, oz[1] = {o.z};
+        const float lx[1] = {l.x}, ly[1] = {l.y}, lz[1] = {l.z};
+        const double cx[1] = {c.x}, cy[1] = {c.y}, cz[1] = {c.z};
+        const float4 ce[1] = {extents[it.x]};
+        float sum = 0.f, compensation = 0.f;  // component `wave`
+        for (std::uint32_t J0 = it.y; J0 < it.z; J0 += kWaves) {
+            const std::uint32_t J = J0 + wave;
+            if (J < it.z) {
+                if (lane == 0) s_near[wave] = 0;
+                source_tile_to<1, kSafe, kRefine, false, kItemUnroll>(
+                    packed, packed_lo, centres, extents, J, false, tile[J].y, live, eps2, ox, oy, oz, lx, ly, lz,
+                    cx, cy, cz, ce,
+                    [&](int, int run, float x, float y, float z) {
+                        s_sums[wave][3 * run][lane] = x;
+                        s_sums[wave][3 * run + 1][lane] = y;
+                        s_sums[wave][3 * run + 2][lane] = z;
+                    },
+                    [&](int, float x, float y, float z, float kx, float ky, float kz) {
+                        const float v[6] = {x, y, z, kx, ky, kz};
+#pragma unroll
+                        for (int u = 0; u < 6; ++u) s_sums[wave][u][lane] = v[u];
+                        if (lane == 0) s_near[wave] = 1;
+                    });
+            }
+            __syncthreads();
+            if (wave < 3) {
+                const std::uint32_t met = min(it.z - J0, static_cast<std::uint32_t>(kWaves));
+                for (std::uint32_t w = 0; w < met; ++w) {
+                    if (s_near[w] != 0) {
+                        kahan_df(s_sums[w][wave][lane], -s_sums[w][3 + wave][lane], sum, compensation);
+                    } else {
+#pragma unroll
+                        for (int run = 0; run < kRuns; ++run) kahan(s_sums[w][3 * run + wave][lane], sum, compensation);
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (wave < 3) {
+            float* out = partial + static_cast<std::size_t>(it.w) * 6 * kTile;
+            out[wave * kTile + lane] = sum;
+            out[(3 + wave) * kTile + lane] = compensation;
+        }
     }
 }
 
@@ -1831,12 +1928,20 @@ void direct_batch_enqueue(orr_ctx* ctx, const double* x, const double* y, const 
         PhaseTimer t(ctx, kDirectKernel);
         // Eight blocks of four waves per CU; never more waves than items.
         const std::uint32_t cap = static_cast<std::uint32_t>(std::max(1, ctx->compute_units)) * 8;
-        const std::uint32_t blocks = std::max<std::uint32_t>(1, std::min(cap, (b.items + 3) / 4));
         const bool refine = ctx->direct_refine != 0;
-        auto kernel = b.safe ? (refine ? direct_items<true, true> : direct_items<true, false>)
-                             : (refine ? direct_items<false, true> : direct_items<false, false>);
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), 0, ctx->stream, packed, packed_lo,
-                           centres, extents, b.tile, b.item, b.items, b.eps2, partials);
+        auto pick = [&](auto safe, auto refined) {
+            constexpr bool kS = decltype(safe)::value, kF = decltype(refined)::value;
+            if (b.alone && b.items <= kEightWaveItems) return std::make_pair(&direct_items_wide<kS, kF, 8>, 8);
+            if (b.alone && b.items <= kFourWaveItems) return std::make_pair(&direct_items_wide<kS, kF, 4>, 4);
+            return std::make_pair(&direct_items<kS, kF>, 1);
+        };
+        const auto [kernel, waves] =
+            b.safe ? (refine ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{}))
+                   : (refine ? pick(std::false_type{}, std::true_type{}) : pick(std::false_type{}, std::false_type{}));
+        const std::uint32_t blocks = std::max<std::uint32_t>(
+            1, waves == 1 ? std::min(cap, (b.items + 3) / 4) : std::min(cap * 4 / waves, b.items));
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(waves == 1 ? kBlock : 64 * waves), 0, ctx->stream, packed,
+                           packed_lo, centres, extents, b.tile, b.item, b.items, b.eps2, partials);
         ORR_LAUNCHED("direct_items");
     }
     {

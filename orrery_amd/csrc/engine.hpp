@@ -289,6 +289,7 @@ struct DirectBatchView {
     const float* eps2 = nullptr;             // [systems] softening squared
     const double* G = nullptr;               // [systems] gravitational constant
     bool safe = false;                       // some system has zero softening
+    bool alone = false;                      // the batch has no tree branch beside it
 };
 void direct_batch_enqueue(orr_ctx* ctx, const double* x, const double* y, const double* z,
                           const double* m, const std::uint32_t* order, const DirectBatchView& b,

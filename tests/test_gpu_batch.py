@@ -343,3 +343,24 @@ def test_device_bytes_within_bound(ctx, quadrupole, leaf, items):
     parts = sum(E.DeviceBatch.bytes_bound([s], cfg) for s in systems)
     assert bound <= parts
     b.close()
+
+
+@pytest.mark.parametrize("per_item", [1, 3, 4, 7, 8, 9, 16, 64])
+@pytest.mark.parametrize("ns", [[1], [65], [700, 64, 63, 2], [4000, 129, 1500]], ids=len)
+def test_waves_of_an_item_sum_as_one(ctx, ns, per_item):
+    # Direct systems alone are summed by four or eight waves an item, beside a tree system
+    # by one: the same bits, for items of fewer tiles than waves, as many, and ragged rounds.
+    config = E.BatchConfig(tiles_per_item=per_item, leaf_capacity=16, use_graph=False)
+    out = []
+    for extra in ([], [(300, 1)]):
+        systems = [E.BatchSystem(n, EPS, 1e-3, solver=0) for n in ns]
+        systems += [E.BatchSystem(n, EPS, 1e-3, solver=k) for n, k in extra]
+        b = E.DeviceBatch(ctx, systems, config)
+        for k, s in enumerate(systems):
+            b.upload(k, *oracle.plummer(s.count, 70 + k).arrays())
+        b.refresh()
+        out.append([b.download(k) for k in range(len(ns))])
+        b.close()
+    for one, wide in zip(*out):
+        for key in ("ax", "ay", "az"):
+            assert np.array_equal(one[key], wide[key])
