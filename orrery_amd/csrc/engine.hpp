@@ -482,8 +482,8 @@ void diagnostics(orr_ctx* ctx, std::uint64_t n, const double* x, const double* y
 // Enqueued on ctx->stream without waiting; `out` (8 doubles, best pinned host
 // memory) holds {kinetic, potential, p, L} once the stream reaches it. The
 // scratch (ctx->diag_scratch) grows only here: callers that enqueue several
-// reserve diagnostics_scratch_bytes(largest n) first, so no growth frees memory
-// that queued kernels still use.
+// reserve the largest of their diagnostics_scratch_bytes(n) first (not always
+// the largest n's), so no growth frees memory that queued kernels still use.
 std::size_t diagnostics_scratch_bytes(std::uint64_t n);
 void diagnostics_enqueue(orr_ctx* ctx, std::uint64_t n, const double* x, const double* y,
                          const double* z, const double* vx, const double* vy, const double* vz,

@@ -104,24 +104,18 @@ struct Compensated {
 
 constexpr int kTerms = 8;  // ke, px, py, pz, lx, ly, lz, pe
 
-// The potential's rows are summed in column chunks of whole kPotTile columns:
-// at most kColumnChunks of them for a system whose row blocks fill the device,
-// up to kMaxChunks below that (a few thousand particles otherwise give a few
-// dozen workgroups: a diagnostic of 4096 took 182 us with chunks of 2048
-// columns, 58 us with chunks of 256).
-constexpr int kPotTile = 256;  // rows of a block, one a thread
+// Columns of the potential's rows are summed in at most kColumnChunks chunks
+// of at least kColumnMin columns, each with a slot a row in memory. That memory
+// is part of what a server charges a request for, so more chunks are not how a
+// small system is spread over the chip: the waves of a block share a chunk instead.
+constexpr std::uint64_t kColumnMin = 2048;
 constexpr std::uint64_t kColumnChunks = 16;
-constexpr std::uint64_t kMaxChunks = 64;
-// Row blocks times chunks wanted: a few dozen rounds of waves even out the
-// blocks on the diagonal (65,536 particles: 1.43 ms at 4096, 1.38 at 16,384).
-constexpr std::uint64_t kPotBlocks = 16384;
+constexpr std::uint64_t kColumnUnit = 256;  // a chunk's columns are a multiple of it
 
 __host__ __device__ inline std::uint64_t column_width(std::uint64_t n) {
-    const std::uint64_t row_blocks = (n + kPotTile - 1) / kPotTile;
-    std::uint64_t chunks = row_blocks == 0 ? 1 : kPotBlocks / row_blocks;
-    chunks = chunks < kColumnChunks ? kColumnChunks : (chunks > kMaxChunks ? kMaxChunks : chunks);
-    const std::uint64_t w = (n + chunks - 1) / chunks;
-    return (w + kPotTile - 1) / kPotTile * kPotTile;
+    const std::uint64_t even = (n + kColumnChunks - 1) / kColumnChunks;
+    const std::uint64_t w = even > kColumnMin ? even : kColumnMin;
+    return (w + kColumnUnit - 1) / kColumnUnit * kColumnUnit;
 }
 
 // Accumulates m / sqrt(v), v = |d|^2 + e2 for the separation d = (dx, dy, dz),
@@ -150,27 +144,42 @@ __device__ __forceinline__ void add_potential(double m, double dx, double dy, do
 
 // Row i of the potential over column chunk blockIdx.y: an FP64 sum over j > i
 // of m_j / sqrt(r^2 + e^2) in index order (diagnostics.cpp:129-158 sums the
-// whole row plainly; here the chunks' sums are folded in chunk order). A block
-// holds kPotTile rows, one a thread; the columns are wave-uniform and read four
-// at a time through the scalar unit, so no lane waits on LDS or a barrier
-// (staged through LDS, the four broadcast reads a pair took nearly as many
-// cycles a CU as the arithmetic). Blocks wholly below the diagonal write zeros
-// and leave. Bound by FP64 issue (4.5 cycles an instruction, 16 the root):
-// a diagnostic of 65,536 particles 1.82 -> 1.38 ms, of 131,072 6.23 -> 4.70 ms,
-// 1.8e12 pairs a second.
+// whole row plainly; here the waves' sums and then the chunks' are folded in
+// order). A block holds 64 rows, one a lane of each of its kPotWaves waves,
+// which take a sixteenth of the chunk's columns each and meet in LDS. The
+// columns are wave-uniform and read four at a time through the scalar unit, so
+// no lane waits on LDS or a barrier (staged through LDS, the four broadcast
+// reads a pair took nearly as many cycles a CU as the arithmetic). Bound by FP64
+// issue (4.5 cycles an instruction, 16 the root). A diagnostic, us, with LDS
+// staging, with 256 rows a block and up to 64 chunks, and like this: 1000
+// particles 127, 57, 48; 4096 179, 57, 57; 16,384 252, 149, 126; 65,536 1653,
+// 1242, 1171; 262,144 23,080, 17,824, 17,181 (2.0e12 pairs a second). Two or
+// four times the rows a block with as many fewer waves on them: 61 and 113
+// at 4096, 1178 and 1270 at 65,536.
+constexpr int kPotWaves = 16;
+constexpr int kPotRows = 64;
+static_assert(kColumnUnit % kPotWaves == 0);
+// Rows a launch takes: a grid's threads along x fit 32 bits, and a row has sixteen.
+constexpr std::uint64_t kPotLaunch = std::uint64_t{1} << 27;
+
 template<bool kSoft>
-__global__ __launch_bounds__(kPotTile) void potential_rows(std::uint64_t n, std::uint64_t width,
-                                                           const double* __restrict__ x,
-                                                           const double* __restrict__ y,
-                                                           const double* __restrict__ z,
-                                                           const double* __restrict__ m, double e2,
-                                                           double* __restrict__ rows) {
-    const std::uint64_t row0 = static_cast<std::uint64_t>(blockIdx.x) * kPotTile;
-    const std::uint64_t i = row0 + threadIdx.x;
-    const std::uint64_t c0 = static_cast<std::uint64_t>(blockIdx.y) * width;
-    const std::uint64_t c1 = c0 + width < n ? c0 + width : n;
+__global__ __launch_bounds__(kPotRows * kPotWaves) void potential_rows(std::uint64_t first, std::uint64_t n,
+                                                                       std::uint64_t width,
+                                                                       const double* __restrict__ x,
+                                                                       const double* __restrict__ y,
+                                                                       const double* __restrict__ z,
+                                                                       const double* __restrict__ m, double e2,
+                                                                       double* __restrict__ rows) {
+    __shared__ double s_part[kPotWaves][kPotRows];
+    const std::uint32_t lane = threadIdx.x % kPotRows;
+    const std::uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kPotRows);
+    const std::uint64_t row0 = first + static_cast<std::uint64_t>(blockIdx.x) * kPotRows;
+    const std::uint64_t i = row0 + lane;
+    const std::uint64_t share = width / kPotWaves;
+    const std::uint64_t c0 = static_cast<std::uint64_t>(blockIdx.y) * width + wave * share;
+    const std::uint64_t c1 = c0 + share < n ? c0 + share : n;
     // From here on the columns lie above every row of the block.
-    const std::uint64_t beyond = row0 + kPotTile;
+    const std::uint64_t beyond = row0 + kPotRows;
     std::uint64_t j = c0 > row0 + 1 ? c0 : row0 + 1;
     double sum = 0.0, fix = 0.0;
     if (j < c1) {
@@ -202,7 +211,13 @@ __global__ __launch_bounds__(kPotTile) void potential_rows(std::uint64_t n, std:
             if (j > i) add_potential<kSoft>(m[j], x[j] - xi, y[j] - yi, z[j] - zi, e2, sum, fix);
         }
     }
-    if (i < n) rows[static_cast<std::uint64_t>(blockIdx.y) * n + i] = sum + fix;
+    s_part[wave][lane] = sum + fix;
+    __syncthreads();
+    if (wave != 0 || i >= n) return;
+    double total = 0.0;
+#pragma unroll
+    for (int w = 0; w < kPotWaves; ++w) total += s_part[w][lane];
+    rows[static_cast<std::uint64_t>(blockIdx.y) * n + i] = total;
 }
 
 // Per-particle terms, term-major [kTerms][n].
@@ -364,9 +379,12 @@ void diagnostics_enqueue(orr_ctx* ctx, std::uint64_t n, const double* x, const d
     PhaseTimer t(ctx, kEnergy);
     const std::uint32_t row_blocks = static_cast<std::uint32_t>((n + 255) / 256);
     auto rows_kernel = e2 > 0.0 ? potential_rows<true> : potential_rows<false>;
-    hipLaunchKernelGGL(rows_kernel, dim3(static_cast<std::uint32_t>((n + kPotTile - 1) / kPotTile), columns),
-                       dim3(kPotTile), 0, ctx->stream, n, width, x, y, z, m, e2, rows);
-    ORR_LAUNCHED("potential_rows");
+    for (std::uint64_t first = 0; first < n; first += kPotLaunch) {
+        const std::uint64_t count = n - first < kPotLaunch ? n - first : kPotLaunch;
+        hipLaunchKernelGGL(rows_kernel, dim3(static_cast<std::uint32_t>((count + kPotRows - 1) / kPotRows), columns),
+                           dim3(kPotRows * kPotWaves), 0, ctx->stream, first, n, width, x, y, z, m, e2, rows);
+        ORR_LAUNCHED("potential_rows");
+    }
     hipLaunchKernelGGL(diagnostic_terms, dim3(row_blocks), dim3(256), 0, ctx->stream, n, x, y, z,
                        vx, vy, vz, m, rows, columns, G, terms);
     ORR_LAUNCHED("diagnostic_terms");

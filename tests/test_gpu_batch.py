@@ -364,3 +364,15 @@ def test_waves_of_an_item_sum_as_one(ctx, ns, per_item):
     for one, wide in zip(*out):
         for key in ("ax", "ay", "az"):
             assert np.array_equal(one[key], wide[key])
+
+
+@pytest.mark.parametrize("ns", [[16384, 16385], [36864, 36865], [300, 4096, 4097, 20000]], ids=str)
+def test_diagnostics_scratch_is_reserved_up_front(ctx, ns):
+    # Diagnostics are enqueued behind running steps: whichever system they are of,
+    # their scratch is there from the start, since growing it would free memory in use.
+    b, states = make_batch(ctx, ns, E.BatchConfig(use_graph=False), solver=0)
+    held = b.info()["device_bytes"]
+    for k in range(len(ns)):
+        b.diagnostics(k)
+        assert b.info()["device_bytes"] == held
+    b.close()
