@@ -1372,9 +1372,8 @@ std::size_t layout_bytes(std::uint64_t n, std::size_t nodes, bool quadrupole, st
     const std::size_t per_quad = quadrupole ? 6 * sizeof(double) + sizeof(QuadF) : 0;
     const std::size_t per_node = nodes * (4 * 3 + 1 + 4 * kMaxChildren + 32 + 32 + sizeof(WalkNode) + per_quad);
     const std::size_t counters = 16 + 8 * 4 * static_cast<std::size_t>(segments) +
-                                 8 * ((n + kBlock - 1) / kBlock) +
-                                 32 * (kBlock / 64) * (((64 / kMinLanes) * n + kBlock - 1) / kBlock) + 512;
-    return per_particle + per_node + counters + 22 * 256 + 48;
+                                 8 * ((n + kBlock - 1) / kBlock) + 512;
+    return per_particle + per_node + counters + 22 * 256 + 64;
 }
 
 Layout layout(orr_ctx* ctx, std::uint64_t n, std::size_t nodes, bool quadrupole, std::uint32_t segments,
@@ -1407,8 +1406,11 @@ Layout layout(orr_ctx* ctx, std::uint64_t n, std::size_t nodes, bool quadrupole,
     L.c32 = carve<std::uint32_t>(p, 4);
     L.c64 = carve<unsigned long long>(p, 4 * static_cast<std::size_t>(segments));
     L.block_counts = carve<uint2>(p, (n + kBlock - 1) / kBlock);
-    // Walks with fewer lanes a wave launch more waves.
-    L.wave_stats = carve<unsigned long long>(p, 4 * (kBlock / 64) * (((64 / kMinLanes) * n + kBlock - 1) / kBlock));
+    // The walk's counts lie where the chain lengths were, which nothing reads once
+    // the chains are placed: 32 bytes a wave of at least kMinLanes targets, or of a
+    // block of four waves of twice that, in 4 bytes a particle (at least 256).
+    static_assert(32 <= 4 * kMinLanes && 4 * 32 <= 256);
+    L.wave_stats = reinterpret_cast<unsigned long long*>(L.chain);
     return L;
 }
 
