@@ -510,8 +510,14 @@ __device__ __forceinline__ void store_field(std::uint64_t dst, double gx, double
 // four (four waves of one target on different source tiles took 1.6 times as
 // long at N = 20,001). With one block a target (gridDim.y == 1) the field is
 // written here.
+//
+// One target a lane is held to eight waves a SIMD: its 106 scalar registers
+// left seven, and the far loop waits for every scalar load (an evaluation at
+// N = 20,001 277 -> 258 us, at 262,144 23.6 -> 19.8 ms, at 900,000, where the
+// pairs path's slots no longer fit, 269.7 -> 223.7 ms; the kernel before the
+// groups' FP64 sums, of 86 scalar registers, took 375 us, 23.4 and 265.7 ms).
 template<int R, bool kSafe, bool kRefine>
-__global__ __launch_bounds__(kBlock) void direct_fold(
+__global__ __launch_bounds__(kBlock, R == 1 ? 8 : 1) void direct_fold(
     const float4* __restrict__ packed, const float4* __restrict__ packed_lo,
     const double4* __restrict__ centres, const float4* __restrict__ extents, std::uint32_t tiles,
     std::uint32_t per_group, std::uint32_t groups, float eps2, double* __restrict__ partial, FieldOut out) {
