@@ -1629,7 +1629,10 @@ DirectShape direct_shape(const orr_ctx* ctx, std::uint64_t n) {
     DirectShape d;
     d.tiles = static_cast<std::uint32_t>((n + kTile - 1) / kTile);
     d.npad = d.tiles * kTile;
-    d.R = ctx->direct_targets_per_lane;
+    // Up to four tiles a block has a wave for each: more targets a lane would be the
+    // last tile over again (64 particles, evaluation: four a lane 47.6 us, one 23.8;
+    // 256: 72.6 and 43.4).
+    d.R = d.tiles <= kBlock / kTile ? 1 : ctx->direct_targets_per_lane;
     d.blocks_i = (d.npad + kBlock * d.R - 1) / (kBlock * d.R);
     // Source tiles summed together in FP32: `block_target` blocks of four target
     // tiles times groups, each group at least one tile.

@@ -533,3 +533,18 @@ def test_rank_order_is_the_radix_order(ctx, n, layout):
     finally:
         ctx.set_direct_config(small_order=1, pair_mode=1)
     np.testing.assert_array_equal(np.stack(results[0]), np.stack(results[1]))
+
+
+@pytest.mark.parametrize("n", [2, 64, 65, 200, 256])
+def test_targets_a_lane_beyond_the_system(ctx, n):
+    """A system of up to four tiles has no second target for a lane: the same bits whatever is configured."""
+    p = oracle.plummer(n, n)
+    results = []
+    try:
+        for targets in (1, 2, 4):
+            ctx.set_direct_config(targets_per_lane=targets)
+            results.append(np.stack(evaluate(ctx, (p.x, p.y, p.z), p.m, eps=0.01)[0]))
+    finally:
+        ctx.set_direct_config(targets_per_lane=1)
+    np.testing.assert_array_equal(results[0], results[1])
+    np.testing.assert_array_equal(results[0], results[2])
