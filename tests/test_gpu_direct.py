@@ -548,3 +548,22 @@ def test_targets_a_lane_beyond_the_system(ctx, n):
         ctx.set_direct_config(targets_per_lane=1)
     np.testing.assert_array_equal(results[0], results[1])
     np.testing.assert_array_equal(results[0], results[2])
+
+
+@pytest.mark.parametrize("eps", [0.0, 0.01])
+@pytest.mark.parametrize("n", [64, 65, 191, 192, 193, 200, 256, 257])
+def test_unordered_evaluations_either_way(ctx, n, eps):
+    """Small evaluations in the caller's order, in one workgroup or by launches (which
+    small_order 2 asks for): the same bits on both sides of the line between them."""
+    p = oracle.plummer(n, n)
+    results = []
+    try:
+        for small in (1, 2):
+            ctx.set_direct_config(small_order=small)
+            s = E.HipDirectSolver(E.Softening(eps), context=ctx, spatial_order=False)
+            a = [np.zeros(n) for _ in range(3)]
+            s.evaluate((p.x, p.y, p.z), p.m, a)
+            results.append(np.stack(a))
+    finally:
+        ctx.set_direct_config(small_order=1)
+    np.testing.assert_array_equal(results[0], results[1])
