@@ -636,6 +636,15 @@ __device__ __forceinline__ void kahan(float p, float& s, float& c) {
 //   24,576 Dm 0.473 0.493   -   0.358 0.373    106,496 Pq 1.062 1.017 1.151
 // More parts pay while the launch leaves the SIMDs short of waves; past that
 // the nodes walked twice, and the room in LDS, cost more than they hide.
+//
+// A small opening angle visits thousands of leaves a target where a part has
+// room for a few dozen runs, and each part ends up waiting for the one before:
+// from kOnePartFrom particles a system on, angles up to kOnePartAngle take one
+// part. Whole evaluations of Plummer spheres, us, in parts and in one: 10,000
+// at angle 0.1 (leaves of 4) 3423 and 3038; 16,384 at 0.1 (4) 5517 and 4402,
+// at 0.15 (8) 3587 and 3132, at 0.2 (8) 2751 and 2643, at 0.3 (8) 1578 and 1776;
+// 24,576 at 0.1 (4) 7937 and 6161; 60,000 at 0.15 (16) 6961 and 5687, at 0.5
+// (16) 812 and 861.
 struct WalkShape {
     int lanes, parts;
 };
@@ -643,10 +652,14 @@ constexpr std::uint64_t kEightPartWaves = 128;
 constexpr std::uint64_t kFourPartWaves = 384;
 constexpr std::uint64_t kTwoPartWaves = 1152;
 constexpr std::uint64_t kHalfLaneWaves = 1600;
-WalkShape walk_shape(std::uint64_t full_waves) {
-    if (full_waves <= kEightPartWaves) return {16, 8};
-    if (full_waves <= kFourPartWaves) return {16, 4};
-    if (full_waves <= kTwoPartWaves) return {32, 2};
+constexpr double kOnePartAngle = 0.15;
+constexpr std::uint64_t kOnePartFrom = 10240;
+// `longest`: particles of the launch's largest system.
+WalkShape walk_shape(std::uint64_t full_waves, std::uint64_t longest, double theta) {
+    const bool one_part = theta <= kOnePartAngle && longest > kOnePartFrom;
+    if (full_waves <= kEightPartWaves && !one_part) return {16, 8};
+    if (full_waves <= kFourPartWaves && !one_part) return {16, 4};
+    if (full_waves <= kTwoPartWaves && !one_part) return {32, 2};
     return {full_waves <= kHalfLaneWaves ? 32 : 64, 1};
 }
 
@@ -1508,7 +1521,7 @@ void tree_enqueue(orr_ctx* ctx, const orr_tree_args& a, const SegmentView& segs,
         const WalkShape shape = ctx->walk_lanes != 0 || R != 1
                                     ? WalkShape{ctx->walk_lanes != 0 ? ctx->walk_lanes
                                                 : full_waves <= kHalfLaneWaves ? 32 : 64, 1}
-                                    : walk_shape(full_waves);
+                                    : walk_shape(full_waves, segs.count > 1 ? segs.longest : n, theta);
         const int lanes = shape.lanes, split = shape.parts;
         using Walk = decltype(&tree_walk<1, true, true, 64, false, 1>);
         auto many = [&](auto r, auto l, auto p, auto sv, auto q) -> Walk {

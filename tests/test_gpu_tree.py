@@ -431,3 +431,24 @@ def test_waves_chosen_by_size_walk_as_full_waves(ctx, n, quadrupole):
         ctx.set_tree_config(lanes=-1)
     np.testing.assert_array_equal(out[0][0], out[1][0])
     assert out[0][1:] == out[1][1:]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,theta", [(10240, 0.15), (10241, 0.15), (10241, 0.1500001), (24577, 0.1), (40000, 0.15)])
+def test_small_angles_walk_in_one_part(ctx, n, theta):
+    """Either side of the line below which a walk is not split: the same accelerations
+    and counts bit for bit as full waves."""
+    p = oracle.plummer(n, 4)
+    out = []
+    try:
+        for lanes in (-1, 64):
+            ctx.set_tree_config(lanes=lanes)
+            s = E.HipTreeSolver(E.TreeParameters(theta, 8), E.Softening(0.01), context=ctx)
+            a = [np.zeros(n) for _ in range(3)]
+            s.evaluate((p.x, p.y, p.z), p.m, a)
+            c = s.interaction_count()
+            out.append((np.stack(a), c.particle_particle, c.particle_cell, s.node_visits()))
+    finally:
+        ctx.set_tree_config(lanes=-1)
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:]
