@@ -11,7 +11,7 @@
 //   D  = (b_hi + b_lo) - (a_hi + a_lo)   each sum exact in FP64, one rounding,
 //   R  = |D|^2 + eps^2                   by FMA,
 //   y  = 1 / sqrt(R)                     the hardware FP64 reciprocal square
-//                                        root and two Newton steps,
+//                                        root and one third-order step,
 //   G  = y^3 D                           the term per unit mass, about 1e-15
 //                                        relative.
 //
@@ -21,10 +21,13 @@
 // source's (or target's) mass and adds it to its FP32 sums as (hi, lo).
 //
 // Host and device: the host build seeds the reciprocal square root with
-// 1/sqrt(x) (a CPU test checks the term against long-double arithmetic).
+// 1/sqrt(x) off by 2^-22 up or down, the most the hardware's may be (a CPU test
+// checks the term from it against long-double arithmetic).
 #pragma once
 
 #include <cmath>
+#include <cstdint>
+#include <cstring>
 
 #ifndef __HIPCC__
 #define ORR_HD
@@ -38,7 +41,9 @@ ORR_HD inline double seed_rsq64(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
     return __builtin_amdgcn_rsq(x);
 #else
-    return 1.0 / std::sqrt(x);
+    std::uint64_t bits;
+    std::memcpy(&bits, &x, sizeof(bits));
+    return (1.0 + ((bits & 1u) != 0 ? 0x1p-22 : -0x1p-22)) / std::sqrt(x);
 #endif
 }
 

@@ -1,9 +1,9 @@
 """The FP64 close-pair term of the direct kernels, on the CPU.
 
 orrery_amd/csrc/close_pair.hpp is plain FP64 arithmetic (the separation from
-the positions' (hi, lo) float parts, a reciprocal square root seed and two
-Newton steps), so the host compiler runs the same steps as the device from a
-correctly rounded seed; the harness tests/cpp/test_close_pair.cpp checks the
+the positions' (hi, lo) float parts, a reciprocal square root seed and one
+third-order step), so the host compiler runs the same steps as the device from
+a seed as far off as the hardware's may be; the harness tests/cpp/test_close_pair.cpp checks the
 term, split into two floats as the kernels add it, against long-double
 arithmetic on 200,000 pairs whose separations reach down to the positions' own
 rounding.

@@ -567,3 +567,42 @@ def test_unordered_evaluations_either_way(ctx, n, eps):
     finally:
         ctx.set_direct_config(small_order=1)
     np.testing.assert_array_equal(results[0], results[1])
+
+
+@pytest.mark.parametrize("eps", [0.0, 2.0**-10])
+@pytest.mark.parametrize("route", ["one workgroup", "launches", "batch"])
+def test_close_pair_term_on_the_device(ctx, route, eps):
+    """The root of a close pair's term, from the hardware's seed. Two particles far closer
+    than their tile is wide and a third of next to no mass; coordinates are multiples of
+    2^-40, so the (hi, lo) floats hold them exactly. The term is within 2^-49 of itself
+    once split into two floats, a few 2^-53 before, and the FP32 term of the third
+    particle, 2^-60 of the pair's or less, adds nothing that shows."""
+    r = np.random.default_rng(17)
+    systems = []
+    for k in range(200):
+        x = np.zeros((3, 3))
+        x[1] = np.rint(2.0**40 * 2.0 ** -r.uniform(5, 17) * r.uniform(0.2, 1, 3) * r.choice([-1, 1], 3)) * 2.0**-40
+        x[2] = np.rint(2.0**40 * r.uniform(0.6, 0.9, 3)) * 2.0**-40
+        systems.append(x)
+    m = np.array([0.75, 1.0, 2.0**-60])
+    got = []
+    if route == "batch":
+        b = E.DeviceBatch(ctx, [E.BatchSystem(3, eps, 1e-3, solver=0)] * len(systems), E.BatchConfig(use_graph=False))
+        for k, x in enumerate(systems):
+            b.upload(k, *x.T, *np.zeros((3, 3)), m)
+        b.refresh()
+        got = [np.stack([b.download(k)[a] for a in ("ax", "ay", "az")]) for k in range(len(systems))]
+        b.close()
+    else:
+        try:
+            ctx.set_direct_config(small_order=1 if route == "one workgroup" else 2)
+            got = [np.stack(evaluate(ctx, tuple(np.ascontiguousarray(c) for c in x.T), m, eps=eps)[0]) for x in systems]
+        finally:
+            ctx.set_direct_config(small_order=1)
+    worst = 0.0
+    for x, a in zip(systems, got):
+        d = (x[1] - x[0]).astype(np.longdouble)
+        term = d / ((d * d).sum() + np.longdouble(eps) ** 2) ** np.longdouble(1.5)
+        for mine, of in ((a[:, 0], m[1] * term), (a[:, 1], -m[0] * term)):
+            worst = max(worst, float(np.abs(mine - of).max() / np.abs(of).max()))
+    assert worst <= 2.0**-47
