@@ -376,3 +376,54 @@ def test_diagnostics_scratch_is_reserved_up_front(ctx, ns):
         b.diagnostics(k)
         assert b.info()["device_bytes"] == held
     b.close()
+
+
+@pytest.mark.parametrize("eps", [0.0, EPS])
+@pytest.mark.parametrize("per_item", [1, 5, 16])
+def test_waves_of_an_item_without_softening(ctx, per_item, eps):
+    # As test_waves_of_an_item_sum_as_one, with and without softening and with coincident
+    # particles, which attract neither each other nor themselves.
+    ns = [700, 65, 64, 1500, 3]
+    config = E.BatchConfig(tiles_per_item=per_item, leaf_capacity=16, use_graph=False)
+    out = []
+    for extra in ([], [300]):
+        systems = [E.BatchSystem(n, eps, 1e-3, solver=0) for n in ns]
+        systems += [E.BatchSystem(n, eps, 1e-3, solver=1) for n in extra]
+        b = E.DeviceBatch(ctx, systems, config)
+        for k, s in enumerate(systems):
+            arrays = [a.copy() for a in oracle.plummer(s.count, 70 + k).arrays()]
+            for a in arrays[:3]:
+                a[-2:] = a[0]
+            b.upload(k, *arrays)
+        b.refresh()
+        out.append([b.download(k) for k in range(len(ns))])
+        b.close()
+    for one, wide in zip(*out):
+        for key in ("ax", "ay", "az"):
+            assert np.isfinite(one[key]).all() and np.array_equal(one[key], wide[key])
+
+
+@pytest.mark.parametrize("quadrupole", [False, True])
+@pytest.mark.parametrize("systems,lo,hi", [(11, 1, 1300), (23, 300, 1300), (41, 900, 2400), (150, 100, 1100),
+                                           (4, 7000, 11000)])
+def test_shared_walk_groups_walk_as_full_waves(ctx, systems, lo, hi, quadrupole):
+    # Tree systems whose targets share groups, walked by eight, four, two and one waves a
+    # group (by the particles of all together), against full waves: the same accelerations
+    # and each system's own counts, bit for bit.
+    r = np.random.default_rng(systems)
+    ns = [int(n) for n in r.integers(lo, hi, systems)]
+    config = E.BatchConfig(leaf_capacity=4, quadrupole=quadrupole, use_graph=False)
+    out = []
+    try:
+        for lanes in (-1, 64):
+            ctx.set_tree_config(lanes=lanes)
+            b, _ = make_batch(ctx, ns, config, solver=1)
+            b.refresh()
+            out.append([(b.download(k), b.counts(k)) for k in range(systems)])
+            b.close()
+    finally:
+        ctx.set_tree_config(lanes=-1)
+    for (one, count), (full, other) in zip(*out):
+        assert count == other
+        for key in ("ax", "ay", "az"):
+            assert np.array_equal(one[key], full[key])

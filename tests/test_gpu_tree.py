@@ -452,3 +452,26 @@ def test_small_angles_walk_in_one_part(ctx, n, theta):
         ctx.set_tree_config(lanes=-1)
     np.testing.assert_array_equal(out[0][0], out[1][0])
     assert out[0][1:] == out[1][1:]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quadrupole", [False, True])
+@pytest.mark.parametrize("n", [8192, 8193, 24576, 24577, 73728, 73729, 102400, 102401])
+def test_walk_shapes_at_their_edges(ctx, n, quadrupole):
+    """Both sides of each line between the walk's shapes (eight, four, two and one waves
+    a group, 32 and 64 targets a wave) against full waves: the same accelerations and
+    counts bit for bit."""
+    p = oracle.plummer(n, 13)
+    out = []
+    try:
+        for lanes in (-1, 64):
+            ctx.set_tree_config(lanes=lanes)
+            s = E.HipTreeSolver(E.TreeParameters(0.7, 16, quadrupole=quadrupole), E.Softening(0.0), context=ctx)
+            a = [np.zeros(n) for _ in range(3)]
+            s.evaluate((p.x, p.y, p.z), p.m, a)
+            c = s.interaction_count()
+            out.append((np.stack(a), c.particle_particle, c.particle_cell, s.node_visits()))
+    finally:
+        ctx.set_tree_config(lanes=-1)
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][1:] == out[1][1:]
