@@ -511,13 +511,19 @@ __device__ __forceinline__ void store_field(std::uint64_t dst, double gx, double
 // long at N = 20,001). With one block a target (gridDim.y == 1) the field is
 // written here.
 //
-// One target a lane is held to eight waves a SIMD: its 106 scalar registers
-// left seven, and the far loop waits for every scalar load (an evaluation at
-// N = 20,001 277 -> 258 us, at 262,144 23.6 -> 19.8 ms, at 900,000, where the
-// pairs path's slots no longer fit, 269.7 -> 223.7 ms; the kernel before the
-// groups' FP64 sums, of 86 scalar registers, took 375 us, 23.4 and 265.7 ms).
-template<int R, bool kSafe, bool kRefine>
-__global__ __launch_bounds__(kBlock, R == 1 ? 8 : 1) void direct_fold(
+// kPerSimd 8 asks the compiler for eight waves a SIMD, and it then takes one
+// source's term after another where it otherwise interleaves four: faster from
+// kFoldEightTiles tiles on, slower while a launch's own latency counts.
+// Evaluations with kPerSimd 1 and 8: 1000 particles 56.9 and 58.0 us, 4096 66.9 and
+// 67.7, 8192 118.6 and 117.6, 20,001 275 and 259, 131,072 6.44 and 5.55 ms,
+// 262,144 23.6 and 19.9, 900,000, where the pairs path's slots no longer fit,
+// 269.7 and 223.7 (before the groups' FP64 sums 375 us at 20,001, 23.3 and 265.7
+// ms). It is the order that does it: with eight waves by fewer scalar registers
+// alone 23.7 ms at 262,144.
+constexpr std::uint32_t kFoldEightTiles = 128;
+
+template<int R, bool kSafe, bool kRefine, int kPerSimd>
+__global__ __launch_bounds__(kBlock, kPerSimd) void direct_fold(
     const float4* __restrict__ packed, const float4* __restrict__ packed_lo,
     const double4* __restrict__ centres, const float4* __restrict__ extents, std::uint32_t tiles,
     std::uint32_t per_group, std::uint32_t groups, float eps2, double* __restrict__ partial, FieldOut out) {
@@ -1501,13 +1507,13 @@ __global__ __launch_bounds__(256) void pairs_reduce(const float* __restrict__ jp
     store_field(dst, G * a0, G * a1, G * a2, ax, ay, az, kick);
 }
 
-template<int R>
+template<int R, int kPerSimd>
 void launch_fold(orr_ctx* ctx, bool safe, bool refine, dim3 grid, const float4* packed,
                  const float4* packed_lo, const double4* centres, const float4* extents,
                  std::uint32_t tiles, std::uint32_t per_group, std::uint32_t groups, float eps2,
                  double* partial, const FieldOut& out) {
-    auto kernel = safe ? (refine ? direct_fold<R, true, true> : direct_fold<R, true, false>)
-                       : (refine ? direct_fold<R, false, true> : direct_fold<R, false, false>);
+    auto kernel = safe ? (refine ? direct_fold<R, true, true, kPerSimd> : direct_fold<R, true, false, kPerSimd>)
+                       : (refine ? direct_fold<R, false, true, kPerSimd> : direct_fold<R, false, false, kPerSimd>);
     hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, ctx->stream, packed, packed_lo, centres, extents, tiles, per_group, groups, eps2, partial, out);
     ORR_LAUNCHED("direct_fold");
 }
@@ -1735,7 +1741,9 @@ void direct_launch(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* 
     {
         PhaseTimer t(ctx, kDirectKernel, timed);
         const dim3 grid(d.blocks_i, d.blocks_j);
-        auto launch = d.R == 1 ? launch_fold<1> : d.R == 2 ? launch_fold<2> : launch_fold<4>;
+        auto launch = d.R == 4   ? launch_fold<4, 1>
+                      : d.R == 2 ? launch_fold<2, 1>
+                      : d.tiles >= kFoldEightTiles ? launch_fold<1, 8> : launch_fold<1, 1>;
         launch(ctx, safe, refine, grid, packed, packed_lo, centres, extents, tiles, d.per_split, d.splits,
                eps2, partial, out);
     }
