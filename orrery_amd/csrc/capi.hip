@@ -244,6 +244,7 @@ int orr_upload_rows(orr_ctx* ctx, double* const* dst, const double* const* src, 
         use_device(ctx);
         if (rows == 0 || count == 0) return;
         require(dst != nullptr && src != nullptr, "null argument");
+        require(count <= ~uint64_t{0} / (sizeof(double) * orr::kStageRows), "rows longer than any memory");
         for (uint32_t k = 0; k < rows; ++k) require(dst[k] != nullptr && src[k] != nullptr, "null row");
         orr::stage_upload(ctx, dst, src, static_cast<int>(rows), count);
     });
@@ -255,6 +256,7 @@ int orr_download_rows(orr_ctx* ctx, double* const* dst, double* const* src, uint
         use_device(ctx);
         if (rows == 0 || count == 0) return;
         require(dst != nullptr && src != nullptr, "null argument");
+        require(count <= ~uint64_t{0} / (sizeof(double) * orr::kStageRows), "rows longer than any memory");
         for (uint32_t k = 0; k < rows; ++k) require(dst[k] != nullptr && src[k] != nullptr, "null row");
         orr::stage_download(ctx, dst, src, static_cast<int>(rows), count);
     });

@@ -8,6 +8,8 @@ Golden vectors held by the reference (web/tests/fixtures):
 The device field uses FP32 pairwise terms, so trajectories are compared to
 what those terms can hold, and conserved quantities in FP64.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -501,3 +503,18 @@ def test_state_round_trip_at_the_staging_limit(ctx, n):
     for key, a in zip(("x", "y", "z", "vx", "vy", "vz"), sent):
         np.testing.assert_array_equal(back[key], a)
     assert not any(back[k].any() for k in ("ax", "ay", "az"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [2**61, 2**61 + 1, 2**64 - 1, (2**64 - 1) // 80 + 1])
+def test_rows_whose_bytes_wrap_around_are_refused(ctx, count):
+    """Row transfers choose their way by their size in bytes: a count whose size does not
+    fit 64 bits must not pass for a small one."""
+    C = E.solvers.C
+    d, h = E.DeviceArray(ctx, 4), np.zeros(4)
+    device, host = (ctypes.c_void_p * 1)(d.ptr), (ctypes.c_void_p * 1)(h.ctypes.data)
+    for call, args in ((C.load().orr_upload_rows, (device, host)), (C.load().orr_download_rows, (host, device))):
+        with pytest.raises(C.EngineError) as e:
+            C.check(call(ctx.handle, *args, 1, count))
+        assert e.value.status == 1
+    d.release()
