@@ -143,19 +143,19 @@ ORR_API int orr_direct_static_limits(uint64_t* max_count, uint64_t* scratch_byte
  * target tiles times groups, each of at least one tile (the groups' sums are
  * added in FP64). pair_mode 1 (default)
  * evaluates each far pair of 64-particle tiles once and applies it to both
- * tiles where that is faster and fits: from 704 tiles (44,993 particles) up to
+ * tiles where it fits, from 704 tiles (44,993 particles) up to
  * 856,064 particles (3 doubles per particle and later block of 8 tiles within
  * 16 GiB); pair_mode 3 does so wherever it fits (from 4 blocks of 8 tiles,
  * 1,537 particles); pair_mode 2 always runs the one-sided kernel, to which
- * targets_per_lane and block_target apply. equal_masses 1 (default) lets the
+ * targets_per_lane (one up to 256 particles, whatever is set) and block_target apply. equal_masses 1 (default) lets the
  * pairs path take its equal-mass form when every particle has one mass (the
  * mass leaves the pair term and multiplies the folded sums: two multiplies
  * fewer per pair; the same bits when that mass is a power of two), 2 never.
  * small_order 1 (default) orders a system of at most 20,480 particles by
  * counting each key's rank (one launch up to 4096 particles, four above, instead
  * of a launch per radix pass; the same permutation, so the
- * same bits) and takes whole steps of at most 256 particles in one workgroup
- * (the same bits again), 2 neither. targets_per_lane 0, refine -1, block_target 0,
+ * same bits) and takes whole steps and evaluations of at most 256 particles (evaluations
+ * without an order: 192) in one workgroup (the same bits again), 2 neither. targets_per_lane 0, refine -1, block_target 0,
  * pair_mode 0, equal_masses 0 and small_order 0 keep the current value. */
 typedef struct {
     int32_t targets_per_lane;
@@ -209,7 +209,8 @@ ORR_API int orr_tree_eval(orr_ctx* ctx, const orr_tree_args* args, orr_tree_stat
  * wave walks together -- or -1 for the engine's choice (1; the default); lanes
  * 64 or 32 -- how many lanes of a wave hold targets -- or -1 to choose by size
  * (the default: groups of 16 targets walked by eight or four waves to 8192 and
- * 24,576 particles, groups of 32 by two to 73,728, 32 a wave to 102,400, else 64).
+ * 24,576 particles, groups of 32 by two to 73,728, 32 a wave to 102,400, else 64;
+ * systems of more than 10,240 particles at opening angles up to 0.15: 32 a wave from there on).
  * Results are bit-identical either way; only the speed differs. sort_mode chooses the
  * Morton sort of every path (the tree's, the batch's, the direct ordering of
  * more than 20,480 particles): 1 (the default) systems of up to 196,608 particles

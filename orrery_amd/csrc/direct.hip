@@ -19,9 +19,8 @@
 //     the separation), 12 VALU operations and one v_rsq_f32 of (r^2+eps^2)^3
 //     per interaction.
 //   * Near tiles -- boxes whose gap is at most a tenth of their summed
-//     half-widths (the mask: one bit per tile pair, written once per
-//     evaluation) -- use the double-float separation (o_j - t) + (o_lo_j -
-//     t_lo). Pairs among them closer than a quarter of the wider tile's
+//     half-widths (near_tiles) -- use the double-float separation (o_j - t) +
+//     (o_lo_j - t_lo). Pairs among them closer than a quarter of the wider tile's
 //     half-width are marked and evaluated afterwards in FP64 (close_pair.hpp):
 //     their single term can be many times the net force on either particle.
 //   * Far tiles' terms are summed in FP32 in runs of 16, near tiles' in runs
@@ -431,10 +430,10 @@ __device__ __forceinline__ void source_tile(
         });
 }
 
-// The near flags of every (target tile, source tile) pair, one bit each, rows
-// of ceil(tiles / 32) words: computed once per evaluation so that the kernels
-// read one word per 32 source tiles through the scalar unit instead of each
-// wave repeating the (wave-uniform) box test on its vector lanes.
+// For the pairs path: the near flags of every (target tile, source tile) pair,
+// one bit each, rows of ceil(tiles / 32) words, computed once per evaluation so
+// that its kernels read one word per 32 source tiles through the scalar unit
+// instead of each wave repeating the (wave-uniform) box test on its vector lanes.
 constexpr int kMaskRows = 8;  // target tiles per block of the mask pass
 
 __global__ __launch_bounds__(256) void near_mask(const double4* __restrict__ centres,
@@ -912,9 +911,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8, 8))) 
 }
 
 // The same, kWaves waves an item, for batches of direct systems alone with fewer
-// items than the chip holds waves (beside a tree branch, which is the longer one and
-// then has fewer waves of its own running, a 48-system batch went from 19.7 to 20.2 ms): each wave takes every kWaves-th source tile and leaves the
-// tile's run sums in LDS; after each round of kWaves tiles a wave a component
+// items than the chip holds waves (beside a tree branch that is the longer one and
+// then has fewer waves of its own running, a 48-system batch went from 19.7 to
+// 20.2 ms; a batch with any tree system, also a small one, takes one wave an
+// item): each wave takes every kWaves-th source tile and leaves the tile's run sums in LDS; after each round of kWaves tiles a wave a component
 // adds them in tile order, so the sums are the same bits. Alone on its
 // SIMD, a wave took some 17 us a source tile, sixteen in a row. Whole
 // evaluations of batches of systems of 256 to 4096 particles with one, four and
@@ -1544,10 +1544,15 @@ constexpr std::size_t kPairSlotBytes = std::size_t{1} << 34;
 // the last with twice the stationary-side slots).
 constexpr std::uint64_t kPairItems = 65536;
 
-// Below this many tiles the one-sided kernel is faster (measured per
-// evaluation: N = 40,960 0.694 vs 0.702 ms, N = 49,152 0.894 vs 0.881 ms,
-// N = 16,384 0.32 vs 0.36 ms): pair mode 1 takes the pairs path from here,
-// pair mode 3 wherever it applies.
+// From this many tiles on pair mode 1 takes the pairs path, pair mode 3 wherever
+// it applies. Evaluations one-sided and in pairs, us, Plummer spheres of equal
+// masses (and of spread ones in pairs; one-sided they are the same): 16,384 225 and 305
+// (323), 24,576 366 and 372 (418), 32,768 539 and 489 (542), 36,000 544 and 612
+// (607), 40,960 735 and 636 (684), 44,992 788 and 704 (763), 49,152 966 and 809
+// (877), 65,536 1602 and 1223 (1348). Two-disc collisions of 30,000 427 and 617,
+// 40,960 975 and 763, 49,152 1213 and 889. The two cross between 32,768 and 40,960
+// particles, depending on the masses and on how the count falls on whole waves;
+// the line, set for an earlier one-sided kernel, lies somewhat above.
 constexpr std::uint32_t kPairMinTiles = 704;
 
 PairPlan pair_plan(std::uint32_t tiles, bool masked, int mode) {
@@ -1834,8 +1839,8 @@ bool direct_tiny_steps(orr_ctx* ctx, const SystemArrays& s, std::uint64_t n, con
             t.kick[p] = t.drift[p] / 2;
         }
     }
-    // A launch of a few hundred steps lasts some milliseconds: no kernel holds
-    // the device for long.
+    // A launch of so many steps lasts up to some 30 ms (Runge-Kutta, 256 particles; velocity
+    // Verlet 7 ms): no kernel holds the device for long.
     constexpr std::uint64_t kStepsPerLaunch = 256;
     while (steps > 0) {
         t.steps = static_cast<std::uint32_t>(std::min(steps, kStepsPerLaunch));
@@ -1977,14 +1982,14 @@ void direct_batch_enqueue(orr_ctx* ctx, const double* x, const double* y, const 
 // ---- the direct sum on the library's static scratch ----------------------
 //
 // For callers that cannot allocate device memory: every buffer of the
-// evaluation -- packed tiles, centres, near mask, the Morton order's codes,
-// index and histograms, the one-sided kernel's split partials -- is carved out
+// evaluation -- packed tiles, centres, the Morton order's codes, index and
+// histograms, the one-sided kernel's FP64 sums a block -- is carved out
 // of `scratch` below, a fixed array each device holds from the first call
 // until the process ends. Limits: at most kStaticMaxCount particles; the
-// one-sided kernel always (the pairs path's slots do not fit); the split count
-// of direct_shape, lowered where its partials would not fit (the same bits as
-// direct_evaluate with the one-sided kernel whenever it fits, else the same
-// terms grouped into fewer Kahan-summed splits). Nothing in the scratch has to
+// one-sided kernel always (the pairs path's slots do not fit); the groups of
+// direct_shape, fewer where a sum and compensation a target and group would not
+// fit (the same bits as direct_evaluate with the one-sided kernel whenever they
+// do, else the same terms in fewer Kahan-summed groups). Nothing in the scratch has to
 // start at zero: every launch writes what the next reads. Calls on one device
 // share the array, so calls that overlap on one device (two contexts, two
 // host threads) race.
@@ -2051,8 +2056,9 @@ void direct_evaluate_static(orr_ctx* ctx, const orr_direct_args& a) {
     const bool ordered = a.spatial_order != 0 && n > 64;
     const OrderSizes oz = order_sizes(n, 1, 0, false);
     // What the groups of source tiles are sized by: room beside the other
-    // buffers for one FP32 sum and compensation a target and group (and a mask),
-    // more than the FP64 sums of a block need.
+    // buffers for one FP32 sum and compensation a target and group and for a near
+    // mask. Neither is carved (the FP64 sums of a block need less); counting
+    // them keeps the groups, and so the bits.
     const std::size_t fixed = aligned(packed_buffer_bytes(d)) + aligned(centre_buffer_bytes(d)) +
                               aligned(sizeof(std::uint32_t) * static_cast<std::size_t>(d.words) * d.tiles) +
                               (ordered ? aligned(oz.bbox) + 2 * aligned(oz.codes) +

@@ -400,8 +400,11 @@ void morton_enqueue(orr_ctx* ctx, const double* x, const double* y, const double
 // kSmallOrder, four up to kRankOrder; the same permutation. ctx->order_codes
 // holds no 64-bit codes afterwards.
 constexpr std::uint64_t kSmallOrder = 4096;
-// Order and launch gaps, rank counting against radix passes: 33 against 66 us at
-// 8192 particles, 48 / 81 at 16,384, 65 / 79 at 20,001, 95 / 83 at 24,576.
+// Whole evaluations with the order by rank and by chunks (morton_enqueue), us: 300
+// particles 57 and 63, 4096 68 and 81, 6000 87 and 90, 8192 117 and 117, 12,000
+// 146 and 141, 16,384 225 and 214, 20,001 258 and 236. The line was set where the
+// radix passes, which took these sizes before the chunks, were the faster order
+// (20,001 65 us by rank and 79 by passes, 24,576 95 and 83).
 constexpr std::uint64_t kRankOrder = 20480;
 void morton_enqueue_small(orr_ctx* ctx, const double* x, const double* y, const double* z,
                           std::uint64_t n);
