@@ -517,8 +517,10 @@ __device__ __forceinline__ void store_field(std::uint64_t dst, double gx, double
 // 67.7, 8192 118.6 and 117.6, 20,001 275 and 259, 131,072 6.44 and 5.55 ms,
 // 262,144 23.6 and 19.9, 900,000, where the pairs path's slots no longer fit,
 // 269.7 and 223.7 (before the groups' FP64 sums 375 us at 20,001, 23.3 and 265.7
-// ms). It is the order that does it: with eight waves by fewer scalar registers
-// alone 23.7 ms at 262,144.
+// ms). It is that sequence that does it: with eight waves by fewer scalar registers
+// alone 23.7 ms at 262,144. Near tiles lose by it, so particles taken in the
+// caller's order, whose tiles may all be near, keep kPerSimd 1 (unsorted: 16,384
+// 433 and 443 us, 40,000 2.18 and 2.23 ms).
 constexpr std::uint32_t kFoldEightTiles = 128;
 
 template<int R, bool kSafe, bool kRefine, int kPerSimd>
@@ -1748,7 +1750,7 @@ void direct_launch(orr_ctx* ctx, const orr_direct_args& a, const std::uint32_t* 
         const dim3 grid(d.blocks_i, d.blocks_j);
         auto launch = d.R == 4   ? launch_fold<4, 1>
                       : d.R == 2 ? launch_fold<2, 1>
-                      : d.tiles >= kFoldEightTiles ? launch_fold<1, 8> : launch_fold<1, 1>;
+                      : order != nullptr && d.tiles >= kFoldEightTiles ? launch_fold<1, 8> : launch_fold<1, 1>;
         launch(ctx, safe, refine, grid, packed, packed_lo, centres, extents, tiles, d.per_split, d.splits,
                eps2, partial, out);
     }
